@@ -273,3 +273,17 @@ def test_attention_rejects_bad_shapes(tg):
                         ctypes.c_float(1e-6))
     assert "kv_len" in tg.last_error()
     assert (out == 7.0).all()
+
+
+@pytest.mark.parametrize("hd,nkv,ratio,kv_len,window", [
+    (64, 2, 8, 1, 0), (64, 2, 4, 127, 0), (64, 2, 4, 128, 0), (64, 2, 4, 129, 0), (64, 8, 8, 4225, 0),
+    (64, 1, 1, 4096, 0), (64, 4, 2, 900, 333), (128, 2, 2, 63, 0), (128, 2, 2, 64, 0), (128, 4, 8, 4161, 0),
+    (128, 1, 5, 2500, 0), (128, 4, 3, 700, 129)])
+def test_attention_span_edges(tg, orc, hd, nkv, ratio, kv_len, window):
+    """k_attn_span at the edges of its tiles (32 positions of 64 values, 16 of
+    128, four to a workgroup), spans of one tile and of many, head groups
+    that leave MFMA columns empty, windows that start inside a tile."""
+    say("attention span", hd, nkv, ratio, kv_len, window)
+    c = _case(500 + kv_len + hd, 256, nkv * ratio, nkv, hd, (Q80, Q80, Q80, Q80), kv_len + 3, kv_len, norms=ratio != 4,
+              sinks=ratio == 8, x_scale=0.02 if ratio == 4 else 1.0)
+    _check(orc, c, window, _gpu(tg, c, window), _oracle(orc, c, window))

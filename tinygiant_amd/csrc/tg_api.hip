@@ -1292,7 +1292,9 @@ static void attn_run(int fmt_q, int fmt_k, int fmt_v, int fmt_o, const void *wq,
             launch_gemv_multi(fmts[i], jobs, nj, embed_dim, xq, 1, st);
         }
     }
-    float *att = (float *)(scratch + L.att);
+    /* the attention output goes straight to the caller's buffer where the
+     * combine's 16-byte stores can */
+    float *att = att_out && ((uintptr_t)att_out & 15) == 0 ? att_out : (float *)(scratch + L.att);
     Q8Rows aq = q8_view(scratch + L.aq, 1, q_dim, att);
     /* attention; q8 of its output fused into the combine where the block
      * layout allows, and the combine into the partial kernel for short spans
@@ -1303,7 +1305,8 @@ static void attn_run(int fmt_q, int fmt_k, int fmt_v, int fmt_o, const void *wq,
                           fuse_q8 ? &aq : nullptr, st, fused_x ? ctr : nullptr);
     if (fmt_o != TG_FMT_F16 && !fuse_q8) launch_quantize(att, q_dim, 1, q_dim, aq, st);
     launch_gemv(fmt_o, (const uint8_t *)wo, embed_dim, q_dim, bo, aq, 1, output, embed_dim, st);
-    if (att_out) HIPCHECK(hipMemcpyAsync(att_out, att, (size_t)q_dim * 4, hipMemcpyDeviceToDevice, st));
+    if (att_out && att != att_out)
+        HIPCHECK(hipMemcpyAsync(att_out, att, (size_t)q_dim * 4, hipMemcpyDeviceToDevice, st));
 }
 
 TG_API size_t tg_hip_attention_scratch_bytes(int embed_dim, int n_heads, int n_kv_heads, int head_dim, int kv_max) {

@@ -4,19 +4,21 @@
  * projections and the output projection (those are the library's q8 + GEMV
  * kernels).
  *
- *   k_attn_partial  split over the sequence: one workgroup per (KV head,
- *                   32 positions) stages those K and V rows and the GQA query
- *                   heads that share them in LDS, so each cache byte is read
- *                   once; per query head it writes the chunk's max score,
- *                   sum of exponentials and unnormalised V sum.  It also does
- *                   the heads' preparation: the optional QK RMS norm
- *                   (tg_rms_norm, :680-698) and RoPE at pos
- *                   (apply_rope_inplace, :702-719) of its query heads, and, in
- *                   the chunk that ends at kv_len, of the new K row, which it
- *                   stores with the new V row at kv_len of the cache.
- *                   For short spans (attention_fuse_ok) the same kernel also
- *                   combines: the last workgroup of each KV head, by a
+ *   k_attn_span     head_dim 64 and 128, split over the sequence: one
+ *                   workgroup per (KV head, span of positions) runs the GQA
+ *                   query heads that share the K and V rows over them on f32
+ *                   MFMA, so each cache byte is read once; per query head it
+ *                   writes the span's max score, sum of exponentials and
+ *                   unnormalised V sum.  It also does the heads' preparation:
+ *                   the optional QK RMS norm (tg_rms_norm, :680-698) and RoPE
+ *                   at pos (apply_rope_inplace, :702-719) of its query heads,
+ *                   and, in the last span, of the new K row, which it stores
+ *                   with the new V row at kv_len of the cache.
+ *                   For up to ATTN_FUSE_MAX_CHUNKS spans the same kernel can
+ *                   also combine: the last workgroup of each KV head, by a
  *                   ticket counter, merges its query heads (combine_group)
+ *   k_attn_partial  the same per 32 positions, staged in LDS, for the other
+ *                   head sizes
  *   k_attn_combine  one workgroup per query head merges the chunks with the
  *                   optional sink logit (head_task, :862-904);
  *                   k_attn_combine_q8 does the same for the heads of one
@@ -32,6 +34,8 @@
 #include <math.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "tg_attn.h"
 #include "tg_device.hpp"
 #include "tg_xchg.hpp"
@@ -43,6 +47,14 @@ namespace {
 constexpr int CHUNK = ATTN_CHUNK;       /* positions per workgroup */
 constexpr int MAXHD = ATTN_MAX_HEAD_DIM;
 constexpr int MAXR = ATTN_MAX_GQA;
+
+/* k_attn_span: positions of a wave's tile (8 KB of K), and the workgroups a
+ * layer's span is cut into at most: one a CU.  Two a CU read the cache no
+ * faster and write twice the records (whole calls, 4 KV heads of 128: 29.9
+ * against 33.3 us at 12,000 positions; 8 of 64: 34.1 against 37.8 us at
+ * 8,000, 56.1 against 57.7 at 30,001). */
+constexpr int SPAN_TP(int head_dim) { return head_dim == 64 ? 32 : 16; }
+constexpr int SPAN_WGS = 256;
 
 }  // namespace
 
@@ -96,7 +108,7 @@ __device__ inline void head_out(const HeadIn &in, bool norm, int head_dim, float
  *   thread t: head t / (head_dim / 4), values 4 (t % (head_dim / 4)) .. + 3,
  *             so wave w holds values 4 lane .. 4 lane + 3 of block w.
  * Needs nchunks <= ATTN_FUSE_MAX_CHUNKS, ratio <= 8 and ratio * head_dim a
- * multiple of 256 (attention_fuse_ok). */
+ * multiple of 256 (attention_group_ok). */
 __device__ inline void combine_group(const Buf pb, const AttnFuse &fz, int kh, int ratio, int head_dim,
                                      int nchunks) {
     __shared__ float scl[ATTN_MAX_GQA][ATTN_FUSE_MAX_CHUNKS];
@@ -158,6 +170,21 @@ __device__ inline void combine_group(const Buf pb, const AttnFuse &fz, int kh, i
     }
     const int nblk = ratio * head_dim / 256;
     if (wave < nblk) q8_block_store(o0, o1, o2, o3, lane, fz.aq, 0, kh * nblk + wave);
+}
+
+/* The ticket that decides which workgroup of KV head kh combines: every
+ * write of a workgroup has completed before it takes one, so the workgroup
+ * with the last ticket sees all chunks' partials (no waiting anywhere) */
+__device__ inline void fuse_combine(const Buf pb, const AttnFuse &fz, int kh, int ratio, int head_dim, int nchunks) {
+    __shared__ unsigned ticket;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    /* system scope: performed at memory (sc1), not in one XCD's L2 */
+    if (threadIdx.x == 0)
+        ticket = __hip_atomic_fetch_add(fz.ctr + kh, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __syncthreads();
+    if (ticket != (unsigned)(nchunks - 1)) return;
+    combine_group(pb, fz, kh, ratio, head_dim, nchunks);
 }
 
 /* grid (chunks, n_kv): part[(h * nchunks + c) * (head_dim + 2)] =
@@ -309,19 +336,253 @@ __global__ __launch_bounds__(256) void k_attn_partial(const float *__restrict__ 
             }
         }
     }
-    if constexpr (FUSE) {
-        /* every write of this workgroup has completed before it takes a
-         * ticket; the workgroup with the last ticket of its KV head sees all
-         * chunks' partials and combines the head group (no waiting anywhere) */
-        __shared__ unsigned ticket;
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        /* system scope: performed at memory (sc1), not in one XCD's L2 */
-        if (tid == 0) ticket = __hip_atomic_fetch_add(fz.ctr + kh, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        __syncthreads();
-        if (ticket != (unsigned)(nchunks - 1)) return;
-        combine_group(pb, fz, kh, ratio, head_dim, nchunks);
+    if constexpr (FUSE) fuse_combine(pb, fz, kh, ratio, head_dim, nchunks);
+}
+
+/* ---- the span kernel: head_dim 64 and 128 on f32 MFMA ----
+ *
+ * One workgroup of four waves per (contiguous span of cached positions, KV
+ * head).  A wave walks tiles of TP positions (every fourth of the span's)
+ * with K and V straight from the cache into registers, as the operands of
+ * v_mfma_f32_16x16x4_f32 (f32 in, f32 sums, no rounding added):
+ *   scores  S^T[position][head] = K . Q^T: A lane l = position l % 16, K slot
+ *           l / 16 = dims 16 j + 4 (l / 16) + e of MFMA (j, e), so a lane's
+ *           K values are 16-byte pieces and four lanes read 64 contiguous
+ *           bytes of a row; B lane l = head l % 16, the same dims, held in
+ *           registers for the whole kernel.  D lane l: head l % 16, positions
+ *           4 (l / 16) + v.
+ *   values  O^T[dim][head] += V^T . P^T: the scores' D register v is the B
+ *           operand of the MFMA over positions 4 (l / 16) + v, as it lies; A
+ *           lane l = dims 4 (l % 16) + t, so a lane's V values are 16-byte
+ *           pieces too.  D lane l: head l % 16, dims 16 (l / 16) + 4 v + t.
+ * A head's running maximum and its sums then sit in the same lanes as its
+ * outputs: the online softmax needs two shuffles a tile and no LDS.  K of
+ * the next tile loads while the values are summed, V while the scores are.
+ * The row at kv_len never comes from the cache: the last span's workgroup
+ * prepares it in LDS, stores it and takes it as a tile of one position.
+ * The four waves meet in LDS once, at the end, and the workgroup writes one
+ * record {max, sum, o[HD]} per query head, as k_attn_partial does per 32
+ * positions.
+ *
+ * Measured (whole calls, k_attn_partial before): 30,001 positions, 8 KV
+ * heads of 64, 91.3 -> 56.1 us; 4 KV heads of 128: 31,000 positions 70.6 ->
+ * 44.8, 4,000 28.5 -> 25.8, 500 23.6 -> 21.4 us.  k_attn_partial read both
+ * factors of every product from LDS and wrote a record per 32 positions
+ * (16 MB at 30,001).
+ *
+ * Bound: the bytes of the cache.  A 16-position tile of a 64-value head is
+ * 8 KB for 32 MFMAs of 32 cycles, 32 bytes a cycle and CU, four times the
+ * CU's share of HBM, even with half of the 16 columns empty. */
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+template <int HD, bool FUSE>
+__global__ __launch_bounds__(256) void k_attn_span(const float *__restrict__ qkv, const float *__restrict__ q_norm_w,
+                                                   const float *__restrict__ k_norm_w, const float *__restrict__ rc,
+                                                   const float *__restrict__ rs, float *kv_k, float *kv_v, float *part,
+                                                   int n_heads, int n_kv, int kv_len, int kv_max, int start, int per,
+                                                   float inv_sqrt, float eps, AttnFuse fz) {
+    constexpr int J = HD / 16, H = HD / 64;   /* 16-byte pieces a lane of a K row; 64-dim halves of a V row */
+    constexpr int SUB = SPAN_TP(HD) / 16, TP = 16 * SUB;
+    __shared__ __attribute__((aligned(16))) float qs[MAXR][HD];
+    __shared__ __attribute__((aligned(16))) float knew[HD], vnew[HD];
+    __shared__ __attribute__((aligned(16))) float mo[4][MAXR][HD];
+    __shared__ float mm[4][MAXR], ml[4][MAXR];
+    const int kh = blockIdx.y, c = blockIdx.x, nchunks = gridDim.x;
+    const int ratio = n_heads / n_kv;
+    const int lo = start + c * per, hi = min(lo + per, kv_len);   /* cached positions of this workgroup */
+    const bool last = c == nchunks - 1;                           /* it also takes the new row */
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c16 = lane & 15, kq = lane >> 4;
+    const int q_dim = n_heads * HD, kv_dim = n_kv * HD;
+    const bool norm = q_norm_w != nullptr;
+    /* the inputs of this wave's heads first, so their preparation waits only
+     * for them and not for the first tile */
+    HeadIn hin[3];
+    float vn[2] = {0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const int j = w + 4 * k;
+        if (j < ratio) {
+            hin[k] = head_in(qkv + (size_t)(kh * ratio + j) * HD, q_norm_w, rc, rs, HD, lane);
+        } else if (j == ratio && last) {
+            hin[k] = head_in(qkv + q_dim + (size_t)kh * HD, norm ? k_norm_w : nullptr, rc, rs, HD, lane);
+            const float *vsrc = qkv + q_dim + kv_dim + (size_t)kh * HD;
+#pragma unroll
+            for (int u = 0; u < HD / 64; u++) vn[u] = vsrc[lane + 64 * u];
+        }
     }
+    /* rows from kv_len on read as zeros */
+    const Buf kb = make_buf(kv_k + (size_t)kh * kv_max * HD, (uint32_t)kv_len * HD * 4u);
+    const Buf vb = make_buf(kv_v + (size_t)kh * kv_max * HD, (uint32_t)kv_len * HD * 4u);
+    u32x4 kr[SUB][J], vr[SUB][4][H];
+    auto load_k = [&](int t0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < SUB; s++)
+#pragma unroll
+            for (int j = 0; j < J; j++)
+                kr[s][j] = ld16(kb, ((uint32_t)(t0 + 16 * s + c16) * HD + 16u * j + 4u * kq) * 4u);
+    };
+    auto load_v = [&](int t0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < SUB; s++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int h = 0; h < H; h++)
+                    vr[s][i][h] = ld16(vb, ((uint32_t)(t0 + 16 * s + 4 * kq + i) * HD + 64u * h + 4u * c16) * 4u);
+    };
+    int t = lo + TP * w;
+    load_k(t);   /* past the rows: zeros, no memory access */
+    load_v(t);
+    /* query heads, then the new K/V row */
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const int j = w + 4 * k;
+        if (j < ratio) {
+            head_out(hin[k], norm, HD, eps, lane, qs[j]);
+        } else if (j == ratio && last) {
+            head_out(hin[k], norm, HD, eps, lane, knew);
+            float *kd = kv_k + ((size_t)kh * kv_max + kv_len) * HD;
+            float *vd = kv_v + ((size_t)kh * kv_max + kv_len) * HD;
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int u = 0; u < HD / 64; u++) {
+                const int i = lane + 64 * u;
+                vnew[i] = vn[u];
+                vd[i] = vn[u];
+                kd[i] = knew[i];
+            }
+        }
+    }
+    bar_lds();   /* the tile stays in flight */
+    v4f q[J];
+#pragma unroll
+    for (int j = 0; j < J; j++)
+        q[j] = c16 < ratio ? *(const v4f *)&qs[c16 < MAXR ? c16 : 0][16 * j + 4 * kq] : v4f{0.f, 0.f, 0.f, 0.f};
+
+    float m = -INFINITY, l = 0.f;   /* head c16: running maximum, this lane's share of the sum */
+    v4f o[H][4];                    /* head c16, dims 64 h + 16 kq + 4 v + t in o[h][t][v] */
+#pragma unroll
+    for (int h = 0; h < H; h++)
+#pragma unroll
+        for (int x = 0; x < 4; x++) o[h][x] = v4f{0.f, 0.f, 0.f, 0.f};
+    auto scores = [&](v4f (&sc)[SUB]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < SUB; s++) {
+            v4f a = {0.f, 0.f, 0.f, 0.f}, b = {0.f, 0.f, 0.f, 0.f};   /* two chains */
+#pragma unroll
+            for (int j = 0; j < J; j++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const float kv = __uint_as_float(kr[s][j][e]);
+                    if (e & 1) b = __builtin_amdgcn_mfma_f32_16x16x4f32(kv, q[j][e], b, 0, 0, 0);
+                    else a = __builtin_amdgcn_mfma_f32_16x16x4f32(kv, q[j][e], a, 0, 0, 0);
+                }
+            sc[s] = a + b;
+        }
+    };
+    /* online softmax of a tile's scores; position i of the tile is valid below n */
+    auto softmax = [&](v4f (&sc)[SUB], int n) __attribute__((always_inline)) {
+        float mt = -INFINITY;
+#pragma unroll
+        for (int s = 0; s < SUB; s++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                sc[s][v] = 16 * s + 4 * kq + v < n ? sc[s][v] * inv_sqrt : -INFINITY;
+                mt = fmaxf(mt, sc[s][v]);
+            }
+        mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
+        mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+        const float mn = fmaxf(m, mt), base = mn == -INFINITY ? 0.f : mn, alpha = expf(m - base);
+        m = mn;
+        l *= alpha;
+#pragma unroll
+        for (int s = 0; s < SUB; s++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                sc[s][v] = expf(sc[s][v] - base);
+                l += sc[s][v];
+            }
+#pragma unroll
+        for (int h = 0; h < H; h++)
+#pragma unroll
+            for (int x = 0; x < 4; x++) o[h][x] *= alpha;
+    };
+    auto values = [&](const v4f (&p)[SUB]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < SUB; s++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int h = 0; h < H; h++)
+#pragma unroll
+                    for (int x = 0; x < 4; x++)
+                        o[h][x] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(vr[s][i][h][x]), p[s][i],
+                                                                       o[h][x], 0, 0, 0);
+    };
+    for (; t < hi; t += 4 * TP) {
+        v4f sc[SUB];
+        scores(sc);
+        load_k(t + 4 * TP);
+        softmax(sc, hi - t);
+        values(sc);
+        load_v(t + 4 * TP);
+    }
+    if (last && w == 0) {   /* the new row as position 0 of a tile of its own */
+#pragma unroll
+        for (int s = 0; s < SUB; s++) {
+#pragma unroll
+            for (int j = 0; j < J; j++)
+                kr[s][j] = s == 0 && c16 == 0 ? *(const u32x4 *)&knew[16 * j + 4 * kq] : u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int h = 0; h < H; h++)
+                    vr[s][i][h] = s == 0 && i == 0 && kq == 0 ? *(const u32x4 *)&vnew[64 * h + 4 * c16] : u32x4{0u, 0u, 0u, 0u};
+        }
+        v4f sc[SUB];
+        scores(sc);
+        softmax(sc, 1);
+        values(sc);
+    }
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    if (c16 < ratio) {
+#pragma unroll
+        for (int h = 0; h < H; h++)
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                *(v4f *)&mo[w][c16][64 * h + 16 * kq + 4 * v] = v4f{o[h][0][v], o[h][1][v], o[h][2][v], o[h][3][v]};
+        if (kq == 0) {
+            mm[w][c16] = m;
+            ml[w][c16] = l;
+        }
+    }
+    __syncthreads();
+    /* the four waves' records merged, in wave order */
+    const Buf pb = make_buf(part, (uint32_t)((size_t)n_heads * nchunks * (HD + 2) * 4));
+    for (int i = tid; i < ratio * HD; i += 256) {
+        const int j = i / HD, d = i - j * HD;
+        const float M = fmaxf(fmaxf(mm[0][j], mm[1][j]), fmaxf(mm[2][j], mm[3][j])), base = M == -INFINITY ? 0.f : M;
+        float r = 0.f, L = 0.f;
+#pragma unroll
+        for (int x = 0; x < 4; x++) {
+            const float e = expf(mm[x][j] - base);
+            r = fmaf(mo[x][j][d], e, r);
+            L = fmaf(ml[x][j], e, L);
+        }
+        const uint32_t off = (((uint32_t)(kh * ratio + j) * (uint32_t)nchunks + (uint32_t)c) * (HD + 2)) * 4u;
+        /* fused: written through to memory, the combining workgroup may sit
+         * on another XCD */
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(r), pb.r, (int)(off + 4u * (2 + d)), 0,
+                                              FUSE ? CPOL_SC1 : CPOL_PLAIN);
+        if (d == 0) {
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(M), pb.r, (int)off, 0, FUSE ? CPOL_SC1 : CPOL_PLAIN);
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(L), pb.r, (int)(off + 4u), 0,
+                                                  FUSE ? CPOL_SC1 : CPOL_PLAIN);
+        }
+    }
+    if constexpr (FUSE) fuse_combine(pb, fz, kh, ratio, HD, nchunks);
 }
 
 /* max / sum over the 256 threads of a workgroup (4 waves) */
@@ -472,25 +733,59 @@ __global__ __launch_bounds__(CQ_WAVES * 64) void k_attn_combine_q8(const float *
     }
 }
 
+/* the shapes whose combine can run in the last workgroup of a KV head:
+ * whole 256-value q8 blocks per head group, one wave each */
+static bool attention_group_ok(int n_heads, int n_kv, int head_dim) {
+    const int ratio = n_heads / n_kv;
+    return attention_combine_q8_ok(n_heads, head_dim) && ratio <= 8 && (ratio * head_dim) % 256 == 0;
+}
+
 void launch_attention_core(const float *qkv, const float *q_norm_w, const float *k_norm_w, const float *sinks,
                            float *kv_k, float *kv_v, int kv_len, int kv_max, int window, const float *rope_cos_row,
                            const float *rope_sin_row, int n_heads, int n_kv, int head_dim, float eps, float *part,
                            float *att, const Q8Rows *aq, hipStream_t st, unsigned *ctr) {
     const int seq_len = kv_len + 1;
     const int start = (window > 0 && seq_len > window) ? seq_len - window : 0;
-    const int nchunks = (seq_len - start + CHUNK - 1) / CHUNK;
     const float inv_sqrt = 1.f / sqrtf((float)head_dim);
-    if (aq && ctr && attention_fuse_ok(n_heads, n_kv, head_dim, kv_len, window)) {
-        const AttnFuse fz = {ctr, sinks, att, *aq};
-        hipLaunchKernelGGL(k_attn_partial<true>, dim3(nchunks, n_kv), dim3(256), 0, st, qkv, q_norm_w, k_norm_w,
+    const bool fuse_ok = aq && ctr && attention_group_ok(n_heads, n_kv, head_dim);
+    const AttnFuse none = {};
+    int nchunks;
+    if (head_dim == 64 || head_dim == 128) {
+        /* contiguous spans of whole tiles, four tiles (one a wave) and more */
+        const int tp = SPAN_TP(head_dim), nc = kv_len - start;   /* rows read from the cache */
+        const int tiles = (nc + tp - 1) / tp, most = std::max(1, SPAN_WGS / n_kv);
+        const int want = std::max(1, std::min((tiles + 3) / 4, most));
+        const int per = tp * std::max(4, (tiles + want - 1) / want);
+        nchunks = std::max(1, (nc + per - 1) / per);
+        const bool fuse = fuse_ok && nchunks <= ATTN_FUSE_MAX_CHUNKS;
+        const AttnFuse fz = fuse ? AttnFuse{ctr, sinks, att, *aq} : none;
+        const dim3 grid(nchunks, n_kv);
+#define SPAN(HD, F)                                                                                                    \
+    hipLaunchKernelGGL((k_attn_span<HD, F>), grid, dim3(256), 0, st, qkv, q_norm_w, k_norm_w, rope_cos_row,            \
+                       rope_sin_row, kv_k, kv_v, part, n_heads, n_kv, kv_len, kv_max, start, per, inv_sqrt, eps, fz)
+        if (head_dim == 64) {
+            if (fuse) SPAN(64, true);
+            else SPAN(64, false);
+        } else {
+            if (fuse) SPAN(128, true);
+            else SPAN(128, false);
+        }
+#undef SPAN
+        if (fuse) return;
+    } else {
+        nchunks = (seq_len - start + CHUNK - 1) / CHUNK;
+        const bool fuse = fuse_ok && nchunks <= ATTN_FUSE_MAX_CHUNKS;
+        const AttnFuse fz = fuse ? AttnFuse{ctr, sinks, att, *aq} : none;
+        if (fuse) {
+            hipLaunchKernelGGL(k_attn_partial<true>, dim3(nchunks, n_kv), dim3(256), 0, st, qkv, q_norm_w, k_norm_w,
+                               rope_cos_row, rope_sin_row, kv_k, kv_v, part, n_heads, n_kv, head_dim, kv_len, kv_max,
+                               start, seq_len, inv_sqrt, eps, fz);
+            return;
+        }
+        hipLaunchKernelGGL(k_attn_partial<false>, dim3(nchunks, n_kv), dim3(256), 0, st, qkv, q_norm_w, k_norm_w,
                            rope_cos_row, rope_sin_row, kv_k, kv_v, part, n_heads, n_kv, head_dim, kv_len, kv_max,
                            start, seq_len, inv_sqrt, eps, fz);
-        return;
     }
-    const AttnFuse none = {};
-    hipLaunchKernelGGL(k_attn_partial<false>, dim3(nchunks, n_kv), dim3(256), 0, st, qkv, q_norm_w, k_norm_w,
-                       rope_cos_row, rope_sin_row, kv_k, kv_v, part, n_heads, n_kv, head_dim, kv_len, kv_max, start,
-                       seq_len, inv_sqrt, eps, none);
     if (aq) {
         hipLaunchKernelGGL(k_attn_combine_q8, dim3(n_heads * head_dim / 256), dim3(CQ_WAVES * 64), 0, st, part, sinks,
                            att, n_heads, head_dim, nchunks, *aq);
@@ -503,15 +798,6 @@ void launch_attention_core(const float *qkv, const float *q_norm_w, const float 
 bool attention_combine_q8_ok(int n_heads, int head_dim) {
     /* k_attn_combine_q8 holds at most 4 heads per block */
     return head_dim >= 64 && 256 % head_dim == 0 && (n_heads * head_dim) % 256 == 0;
-}
-
-bool attention_fuse_ok(int n_heads, int n_kv, int head_dim, int kv_len, int window) {
-    const int seq_len = kv_len + 1;
-    const int span = (window > 0 && seq_len > window) ? window : seq_len;
-    const int nchunks = (span + CHUNK - 1) / CHUNK;
-    const int ratio = n_heads / n_kv;
-    return attention_combine_q8_ok(n_heads, head_dim) && nchunks <= ATTN_FUSE_MAX_CHUNKS && ratio <= 8 &&
-           (ratio * head_dim) % 256 == 0;
 }
 
 }  // namespace tg
