@@ -1,0 +1,61 @@
+"""tg_hip_matmul_dev over its dispatch: every format at row lengths that give a
+lane one to four items (16 for F16), partial q8 blocks and rows past what the
+staged kernel holds, row counts around a wave's groups and past one grid, and
+input row counts that quantize in the kernel, in a launch of their own, and in
+several staged chunks.  Bar: max|d| <= 1e-5 max|ref| against the oracle, whose
+sums run in another order."""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+Q4K, F16, Q6K, MXFP4, Q80 = 0, 1, 2, 3, 4
+
+
+def _matrix(tg, rng, fmt, nrows, ncols):
+    import tinygiant_amd.synth as S
+    if fmt == F16:
+        return (rng.standard_normal(nrows * ncols) * 0.05).astype(np.float16).view(np.uint8)
+    return S.matrix_host(fmt, int(rng.integers(1 << 40)), nrows, ncols)
+
+
+@pytest.mark.parametrize("fmt,nrows,ncols,k,bias", [
+    (Q4K, 1, 256, 1, True), (Q4K, 33, 512, 2, False), (Q6K, 63, 768, 5, True), (Q6K, 7, 2048, 3, False),
+    (Q4K, 130, 4096, 16, True), (Q6K, 41, 12288, 1, True), (Q4K, 9, 16384, 4, False), (Q4K, 9, 16640, 2, True),
+    (Q4K, 40001, 256, 1, False), (Q6K, 40001, 256, 3, True),
+    (Q80, 5, 32, 1, True), (Q80, 65, 288, 3, True), (Q80, 100, 2880, 1, True), (Q80, 31, 2880, 9, False),
+    (Q80, 17, 4096, 1, False), (Q80, 13, 8192, 9, True), (Q80, 13, 8224, 2, True),
+    (MXFP4, 77, 2880, 16, True), (MXFP4, 8, 96, 1, False), (MXFP4, 19, 5888, 2, True),
+    (F16, 3, 32, 1, True), (F16, 70, 1056, 5, False), (F16, 33, 2880, 4, True), (F16, 21, 8192, 3, True),
+    (F16, 9, 8224, 2, False), (F16, 1025, 512, 1, True)])
+def test_matmul_dev_forms(tg, orc, fmt, nrows, ncols, k, bias):
+    print(f"matmul fmt {fmt} {nrows} x {ncols}, {k} rows, bias {bias}", flush=True)
+    lib = tg.lib()
+    rng = np.random.default_rng(fmt * 1000 + nrows + ncols + k)
+    w = _matrix(tg, rng, fmt, nrows, ncols)
+    x = rng.standard_normal((k, ncols)).astype(np.float32)
+    b = (rng.standard_normal(nrows) * 0.1).astype(np.float32) if bias else None
+    bufs = []
+
+    def dev(a):
+        d = tg.DeviceArray(a.nbytes)
+        d.upload(a)
+        bufs.append(d)
+        return d
+
+    guard = np.full((k, nrows + 8), 7.0, np.float32)   # the rows lie densely: what follows must stay
+    y, wd, xd, bd = dev(guard), dev(w), dev(x), dev(b) if bias else None
+    sc = dev(np.zeros(lib.tg_hip_matmul_scratch_bytes(k, ncols), np.uint8))
+    lib.tg_hip_clear_error()
+    lib.tg_hip_matmul_dev(fmt, wd.ptr, bd.ptr if bias else None, xd.ptr, y.ptr, nrows, ncols, k, sc.ptr, None)
+    lib.tg_hip_synchronize()
+    assert tg.last_error() == ""
+    flat = y.download(np.float32, guard.size)
+    for d in bufs:
+        d.free()
+    got = flat[:k * nrows].reshape(k, nrows)
+    assert (flat[k * nrows:] == 7.0).all()
+    for j in range(k):
+        ref = orc.matmul(fmt, w, b, x[j], nrows, ncols)
+        assert np.abs(got[j] - ref).max() <= 1e-5 * np.abs(ref).max(), j

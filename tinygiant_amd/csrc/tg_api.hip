@@ -744,8 +744,8 @@ void matmul_host(int fmt, const void *mat, const float *bias, const float *input
     HIPCHECK(hipMemcpyAsync(dev + o_in, input, (size_t)ncols * 4, hipMemcpyHostToDevice, g.st));
     for (auto &it : sg.items) HIPCHECK(hipMemcpyAsync(dev + it.off, it.host, it.n, hipMemcpyHostToDevice, g.st));
     Q8Rows q = q8_view(dev + o_q, 1, ncols, (const float *)(dev + o_in));
-    if (fmt != TG_FMT_F16) launch_quantize((const float *)(dev + o_in), ncols, 1, ncols, q, g.st);
-    launch_gemv(fmt, (const uint8_t *)m, nrows, ncols, (const float *)bi, q, 1, (float *)(dev + o_out), nrows, g.st);
+    launch_matmul(fmt, (const uint8_t *)m, nrows, ncols, (const float *)bi, (const float *)(dev + o_in), q, 1,
+                  (float *)(dev + o_out), nrows, g.st);
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipMemcpyAsync(output, dev + o_out, (size_t)nrows * 4, hipMemcpyDeviceToHost, g.st));
     HIPCHECK(hipStreamSynchronize(g.st));
@@ -1137,8 +1137,7 @@ TG_API void tg_hip_matmul_dev(int fmt, const void *mat_dev, const float *bias_de
     ensure_init();
     hipStream_t st = stream ? (hipStream_t)stream : g.st;
     Q8Rows q = q8_view((uint8_t *)scratch_dev, k, ncols, inputs_dev);
-    if (fmt != TG_FMT_F16) launch_quantize(inputs_dev, ncols, k, ncols, q, st);
-    launch_gemv(fmt, (const uint8_t *)mat_dev, nrows, ncols, bias_dev, q, k, outputs_dev, nrows, st);
+    launch_matmul(fmt, (const uint8_t *)mat_dev, nrows, ncols, bias_dev, inputs_dev, q, k, outputs_dev, nrows, st);
     HIPCHECK(hipGetLastError());
 }
 
@@ -1200,8 +1199,7 @@ TG_API void tg_hip_matmul_dev_noalloc(int fmt, const void *mat_dev, const float 
     }
     hipStream_t st = stream ? (hipStream_t)stream : g.st;
     Q8Rows q = q8_view(g.scratch, k, ncols, inputs_dev);
-    if (fmt != TG_FMT_F16) launch_quantize(inputs_dev, ncols, k, ncols, q, st);
-    launch_gemv(fmt, (const uint8_t *)mat_dev, nrows, ncols, bias_dev, q, k, outputs_dev, nrows, st);
+    launch_matmul(fmt, (const uint8_t *)mat_dev, nrows, ncols, bias_dev, inputs_dev, q, k, outputs_dev, nrows, st);
     HIPCHECK(hipGetLastError());
 }
 
@@ -1270,10 +1268,10 @@ static void attn_run(int fmt_q, int fmt_k, int fmt_v, int fmt_o, const void *wq,
     const GemvJob all[3] = {{(const uint8_t *)wq, bq, qkv, q_dim, q_dim},
                             {(const uint8_t *)wk, bk, qkv + q_dim, kv_dim, kv_dim},
                             {(const uint8_t *)wv, bv, qkv + q_dim + kv_dim, kv_dim, kv_dim}};
-    const bool fused_x = gemv_q8x_ok(fmts, 3, embed_dim);
+    const bool fused_x = gemv_staged_ok(fmts, 3, embed_dim);
     if (fused_x) {
-        /* Q4_K / Q6_K: q8 of the input inside the one projection launch,
-         * which also clears the ticket counters of the partial kernel */
+        /* formats of one family: q8 of the input inside the one projection
+         * launch, which also clears the ticket counters of the span kernel */
         const GemvJobs jobs = {{all[0], all[1], all[2]}};
         launch_gemv_q8x(fmts, jobs, 3, embed_dim, input, ctr, n_kv, st);
     } else {
@@ -1302,7 +1300,7 @@ static void attn_run(int fmt_q, int fmt_k, int fmt_v, int fmt_o, const void *wq,
     const bool fuse_q8 = fmt_o != TG_FMT_F16 && attention_combine_q8_ok(n_heads, head_dim);
     launch_attention_core(qkv, q_norm_w, k_norm_w, sinks, kv_k, kv_v, kv_len, kv_max, window, rope_cos_row,
                           rope_sin_row, n_heads, n_kv, head_dim, eps, (float *)(scratch + L.part), att,
-                          fuse_q8 ? &aq : nullptr, st, fused_x ? ctr : nullptr);
+                          fuse_q8 ? &aq : nullptr, st, fused_x && n_kv <= 256 ? ctr : nullptr);
     if (fmt_o != TG_FMT_F16 && !fuse_q8) launch_quantize(att, q_dim, 1, q_dim, aq, st);
     launch_gemv(fmt_o, (const uint8_t *)wo, embed_dim, q_dim, bo, aq, 1, output, embed_dim, st);
     if (att_out && att != att_out)

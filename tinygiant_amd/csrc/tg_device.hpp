@@ -206,6 +206,11 @@ struct Q8Lds {
     const uint8_t *qs, *d, *s32, *s16;
 };
 
+/* One f32 row staged in LDS */
+struct F32Lds {
+    const uint8_t *f;
+};
+
 /* q8 of one 256-value block held by a wave, lane l owning values 4l..4l+3
  * (quantize_q8, csrc/libtinygiant.c:169-208): scale amax/127, quants
  * rint(v * 127/amax) packed four to a word, the lane's 16- and 32-element
@@ -590,7 +595,8 @@ struct FQ80 {
         r.q1 = ld16(w, p + 18);
         return r;
     }
-    __device__ static inline X load_x(const Q8Row &x, int item) {
+    template <class R>   /* Q8Row (global) or Q8Lds */
+    __device__ static inline X load_x(const R &x, int item) {
         FMXFP4::X t = FMXFP4::load_x(x, item);
         X r;
         r.a = t.a;
@@ -630,7 +636,8 @@ struct FF16 {
         r.h = ld16(w, row_off + (uint32_t)item * 16u);
         return r;
     }
-    __device__ static inline X load_x(const Q8Row &x, int item) {
+    template <class R>   /* Q8Row (global) or F32Lds */
+    __device__ static inline X load_x(const R &x, int item) {
         X r;
         r.a = ld16(x.f, (uint32_t)item * 32u);
         r.b = ld16(x.f, (uint32_t)item * 32u + 16u);

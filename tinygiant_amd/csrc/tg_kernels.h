@@ -73,10 +73,8 @@ uint32_t row_bytes(int fmt, int ncols);
  * for a consumer launched next (the fused head's argmax keys) */
 void launch_quantize(const float *x, int ncols, int nrows, long xstride, const Q8Rows &out, hipStream_t st,
                      unsigned long long *clear = nullptr, int nclear = 0);
-void launch_gemv(int fmt, const uint8_t *W, int nrows, int ncols, const float *bias, const Q8Rows &x, int k,
-                 float *y, long ystride, hipStream_t st);
-/* up to three matrices of one format and width (ncols) against the same q8
- * rows, one launch: y_j[r] = dot(W_j row r, x) + bias_j[r] */
+/* up to three matrices of one width (ncols) against the same k rows:
+ * y_j[i * ystride + r] = dot(W_j row r, x_i) + bias_j[r] */
 struct GemvJob {
     const uint8_t *W;
     const float *bias;
@@ -87,18 +85,23 @@ struct GemvJob {
 struct GemvJobs {
     GemvJob j[3];
 };
-void launch_gemv_multi(int fmt, const GemvJobs &jobs, int njobs, int ncols, const Q8Rows &x, int k, hipStream_t st);
-/* q8 of one f32 row (ncols % 256 == 0, at most Q8X_MAX_BLOCKS blocks) and
- * up to three Q4_K / Q6_K GEMVs of it in one launch (fmts[j] per job); the
- * same bits as launch_quantize + launch_gemv_multi.  Also clears n_zero
- * (<= 256) words at `zero` with device-scope stores. */
-#define Q8X_MAX_BLOCKS 32
-struct GemvQ8xMap {
+struct GemvMap {
     int wg0[4];     /* first workgroup of each job, then the total */
     int fmt[3];
     uint32_t rb[3];
 };
-bool gemv_q8x_ok(const int *fmts, int njobs, int ncols);
+/* one matrix, or several of one format, against rows already in q8 */
+void launch_gemv(int fmt, const uint8_t *W, int nrows, int ncols, const float *bias, const Q8Rows &x, int k,
+                 float *y, long ystride, hipStream_t st);
+void launch_gemv_multi(int fmt, const GemvJobs &jobs, int njobs, int ncols, const Q8Rows &x, int k, hipStream_t st);
+/* one matrix against k f32 rows of ncols values; x is the room for their q8,
+ * used where the matrix's launch does not quantize the rows itself */
+void launch_matmul(int fmt, const uint8_t *W, int nrows, int ncols, const float *bias, const float *xf,
+                   const Q8Rows &x, int k, float *y, long ystride, hipStream_t st);
+/* q8 of one f32 row and up to three matrices of one format family (Q4_K and
+ * Q6_K, or Q8_0 and MXFP4; gemv_staged_ok) in one launch, fmts[j] per job.
+ * Also clears n_zero (<= 256) words at `zero` with device-scope stores. */
+bool gemv_staged_ok(const int *fmts, int njobs, int ncols);
 void launch_gemv_q8x(const int *fmts, const GemvJobs &jobs, int njobs, int ncols, const float *x, unsigned *zero,
                      int n_zero, hipStream_t st);
 void launch_isums(int fmt, const uint8_t *W, int nrows, int ncols, const Q8Rows &x, int nsums_row, int32_t *out,

@@ -25,6 +25,7 @@
 #include "tg_device.hpp"
 #include "tg_kernels.h"
 #include "tg_synth.h"
+#include "tg_xchg.hpp"
 
 namespace tg {
 
@@ -35,7 +36,9 @@ __global__ __launch_bounds__(256) void k_quantize_q8(const float *__restrict__ x
                                                      long xstride, Q8Rows out, unsigned long long *clear, int nclear) {
     const int lane = threadIdx.x & 63;
     if (blockIdx.x == 0 && (int)threadIdx.x < nclear) clear[threadIdx.x] = 0;
-    const int wave = (int)((blockIdx.x * (size_t)blockDim.x + threadIdx.x) >> 6);
+    /* readfirstlane: the block's descriptor stays in scalar registers (in
+     * vector ones every load would be wrapped in a loop over its values) */
+    const int wave = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * (size_t)blockDim.x + threadIdx.x) >> 6));
     const int nb = out.nb;
     if (wave >= nrows * nb) return;   /* uniform per wave */
     const int r = wave / nb, b = wave % nb;
@@ -133,20 +136,22 @@ __device__ inline void row_dots(const Buf (&w)[NM], uint32_t roff, bool rv, cons
     }
 }
 
-/* W: nrows rows of rb bytes.  For each activation row j < k:
+/* The general form, for rows of more items than k_gemv_staged holds.  W: nrows rows of rb bytes.  For each activation row j < k:
  *   y[j*ystride + r] = dot(W[r], x_j) + bias[r]
- * Each wave takes `rows_per_wave` consecutive rows in steps of 64/S. */
+ * Each wave takes `rows_per_wave` consecutive rows in steps of 64/S;
+ * blockIdx.y picks the matrix. */
 template <class F, int S, int TB>
-__device__ inline void gemv_rows(const uint8_t *__restrict__ W, uint32_t rb, int nrows,
-                                 const float *__restrict__ bias, const Q8Rows &x, int k, float *y, long ystride,
-                                 int nitems, int T, int rows_per_wave) {
+__global__ __launch_bounds__(256) void k_gemv(GemvJobs jobs, uint32_t rb, Q8Rows x, int k, int nitems, int T,
+                                              int rows_per_wave) {
     constexpr int G = 64 / S;
+    const GemvJob &jb = jobs.j[blockIdx.y];
+    const int nrows = jb.nrows;
     const int lane = threadIdx.x & 63;
     const int seg = lane / S, sl = lane % S;
-    const int wave = (int)((blockIdx.x * (size_t)blockDim.x + threadIdx.x) >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * (size_t)blockDim.x + threadIdx.x) >> 6));
     const int row0 = wave * rows_per_wave;
     if (row0 >= nrows) return;
-    Buf wb = make_buf(W + (size_t)row0 * rb, (uint32_t)((size_t)min(rows_per_wave, nrows - row0) * rb));
+    Buf wb = make_buf(jb.W + (size_t)row0 * rb, (uint32_t)((size_t)min(rows_per_wave, nrows - row0) * rb));
     for (int j = 0; j < k; j++) {
         Q8Row xr = q8_row(x, j);
         for (int rs = 0; rs < rows_per_wave; rs += G) {
@@ -156,127 +161,244 @@ __device__ inline void gemv_rows(const uint8_t *__restrict__ W, uint32_t rb, int
             const Buf ws[1] = {wb};
             row_dots<F, S, TB, 1>(ws, (uint32_t)rl * rb, rv, xr, sl, nitems, T, acc);
             const float v = seg_sum<S>(acc[0]);
-            if (rv && sl == 0) y[(size_t)j * ystride + r] = v + (bias ? bias[r] : 0.f);
+            if (rv && sl == 0) jb.y[(size_t)j * jb.ystride + r] = v + (jb.bias ? jb.bias[r] : 0.f);
         }
     }
 }
 
-template <class F, int S, int TB>
-__global__ __launch_bounds__(256) void k_gemv(const uint8_t *__restrict__ W, uint32_t rb, int nrows,
-                                              const float *__restrict__ bias, Q8Rows x, int k, float *y,
-                                              long ystride, int nitems, int T, int rows_per_wave) {
-    gemv_rows<F, S, TB>(W, rb, nrows, bias, x, k, y, ystride, nitems, T, rows_per_wave);
-}
+/* rows first, first + 1, ... where a row list is asked for */
+struct RowsFrom {
+    int first;
+    __device__ inline int operator[](int i) const { return first + i; }
+};
 
-/* Several matrices of one format and width against the same rows in one
- * launch: blockIdx.y picks the matrix. */
-template <class F, int S, int TB>
-__global__ __launch_bounds__(256) void k_gemv_multi(GemvJobs jobs, uint32_t rb, Q8Rows x, int k, int nitems, int T,
-                                                    int rows_per_wave) {
-    const GemvJob &jb = jobs.j[blockIdx.y];
-    gemv_rows<F, S, TB>(jb.W, rb, jb.nrows, jb.bias, x, k, jb.y, jb.ystride, nitems, T, rows_per_wave);
-}
+/* Staging of k rows in LDS by the whole workgroup, in two halves, so a
+ * caller can issue loads of its own in between: a compute unit returns its
+ * loads in issue order, so rows requested behind a workgroup's weights would
+ * arrive behind them.  load() requests the first units of every thread (or
+ * blocks of every wave), finish() stores those and stages the rest. */
 
-/* q8 of one f32 row of ncols (a multiple of 256) values into LDS by the
- * workgroup's 4 waves, block b by wave b % 4: the arithmetic of
- * k_quantize_q8 */
-__device__ inline void q8_row_lds(const float *__restrict__ x, int ncols, uint8_t *xq, float *xd, int32_t *xs32,
-                                  int32_t *xs16) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int nb = ncols / 256;
-    for (int b = wave; b < nb; b += 4) {
-        Buf xb = make_buf(x + (size_t)b * 256, 1024u);
-        const u32x4 raw = ld16(xb, (uint32_t)lane * 16u);
-        const Q8Quant q = q8_block_quant(__uint_as_float(raw.x), __uint_as_float(raw.y), __uint_as_float(raw.z),
-                                         __uint_as_float(raw.w));
-        reinterpret_cast<uint32_t *>(xq + b * 256)[lane] = q.packed;
-        if ((lane & 3) == 0) xs16[b * 16 + (lane >> 2)] = q.s16;
-        if ((lane & 7) == 0) xs32[b * 8 + (lane >> 3)] = q.s32;
-        if (lane == 0) xd[b] = q.sc;
+/* q8 rows rows[0..n) of q into LDS slots 0..n-1 */
+template <int U>
+struct Q8Copy {
+    u32x4 v[U > 0 ? U : 1];
+    template <class R>
+    __device__ static inline const u32x4 *src(const Q8Rows &q, const R &rows, int u, uint32_t &dst) {
+        const int nb = q.nb, per = nb * 22;   /* 16-byte units of qs, s32 and s16 */
+        const int s = u / per, w = u % per;
+        const size_t r = (size_t)rows[s];
+        dst = (uint32_t)s * q8_lds_stride(nb) + (uint32_t)w * 16u;
+        return w < nb * 16   ? reinterpret_cast<const u32x4 *>(q.qs + r * nb * 256) + w
+               : w < nb * 18 ? reinterpret_cast<const u32x4 *>(q.s32 + r * nb * 8) + (w - nb * 16)
+                             : reinterpret_cast<const u32x4 *>(q.s16 + r * nb * 16) + (w - nb * 18);
     }
+    template <class R>
+    __device__ inline void load(const Q8Rows &q, const R &rows, int n) {
+        const int total = n * q.nb * 22;
+#pragma unroll
+        for (int i = 0; i < U; i++) {
+            const int u = threadIdx.x + i * blockDim.x;
+            uint32_t dst;
+            if (u < total) v[i] = *src(q, rows, u, dst);
+        }
+    }
+    template <class R>
+    __device__ inline void finish(const Q8Rows &q, const R &rows, int n, uint8_t *lds) {
+        const int nb = q.nb, total = n * nb * 22;
+#pragma unroll
+        for (int i = 0; i < U; i++) {
+            const int u = threadIdx.x + i * blockDim.x;
+            uint32_t dst;
+            if (u < total) {
+                src(q, rows, u, dst);
+                *reinterpret_cast<u32x4 *>(lds + dst) = v[i];
+            }
+        }
+        for (int u = threadIdx.x + U * blockDim.x; u < total; u += blockDim.x) {
+            uint32_t dst;
+            const u32x4 x = *src(q, rows, u, dst);
+            *reinterpret_cast<u32x4 *>(lds + dst) = x;
+        }
+        for (int u = threadIdx.x; u < n * nb; u += blockDim.x) {
+            const int s = u / nb, b = u % nb;
+            reinterpret_cast<float *>(lds + (size_t)s * q8_lds_stride(nb) + nb * 352)[b] = q.d[(size_t)rows[s] * nb + b];
+        }
+    }
+};
+
+/* q8 of f32 rows src[rows[s] * ld ..] (nb 256-value blocks each) into LDS
+ * slots 0..n-1, block per wave, with the arithmetic of k_quantize_q8 (the
+ * same bits), B blocks per wave in flight together.  GW: row s is also
+ * written to q8 row grows[s] of gout if gw. */
+template <int B>
+struct Q8Quantize {
+    u32x4 raw[B];
+    template <class R>
+    __device__ inline void batch(const float *__restrict__ src, int ld, const R &rows, int n, int nb, int u0) {
+        const int nw = blockDim.x >> 6;
+#pragma unroll
+        for (int i = 0; i < B; i++) {
+            const int u = u0 + i * nw;
+            const bool uv = u < n * nb;
+            const int s = uv ? u / nb : 0, b = uv ? u % nb : 0;
+            /* a row's last block may be partial: zeros past its end, as k_quantize_q8 reads */
+            const Buf xb = make_buf_uniform(src + (size_t)rows[s] * ld + (size_t)b * 256,
+                                            uv ? (uint32_t)min(256, ld - b * 256) * 4u : 0u);
+            raw[i] = ld16(xb, (uint32_t)(threadIdx.x & 63) * 16u);
+        }
+    }
+    template <class R>
+    __device__ inline void load(const float *__restrict__ src, int ld, const R &rows, int n, int nb) {
+        batch(src, ld, rows, n, nb, __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)));
+    }
+    template <bool GW = false, class R>
+    __device__ inline void finish(const float *__restrict__ src, int ld, const R &rows, int n, int nb, uint8_t *lds,
+                                  bool gw = false, Q8Rows gout = {}, const int *grows = nullptr) {
+        const int lane = threadIdx.x & 63, nw = blockDim.x >> 6;
+        const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+        for (int u0 = wave; u0 < n * nb; u0 += nw * B) {
+            if (u0 != wave) batch(src, ld, rows, n, nb, u0);
+#pragma unroll
+            for (int i = 0; i < B; i++) {
+                const int u = u0 + i * nw;
+                if (u >= n * nb) continue;   /* uniform per wave */
+                const int s = u / nb, b = u % nb;
+                const float v0 = __uint_as_float(raw[i].x), v1 = __uint_as_float(raw[i].y);
+                const float v2 = __uint_as_float(raw[i].z), v3 = __uint_as_float(raw[i].w);
+                const Q8Quant q = q8_block_quant_dpp(v0, v1, v2, v3);
+                uint8_t *slot = lds + (size_t)s * q8_lds_stride(nb);
+                reinterpret_cast<uint32_t *>(slot + b * 256)[lane] = q.packed;
+                if ((lane & 3) == 0) reinterpret_cast<int32_t *>(slot + nb * 288)[b * 16 + (lane >> 2)] = q.s16;
+                if ((lane & 7) == 0) reinterpret_cast<int32_t *>(slot + nb * 256)[b * 8 + (lane >> 3)] = q.s32;
+                if (lane == 0) reinterpret_cast<float *>(slot + nb * 352)[b] = q.sc;
+                if (GW && gw) q8_block_store(v0, v1, v2, v3, lane, gout, grows[s], b);
+            }
+        }
+    }
+};
+
+/* f32 rows first .. first + n - 1 of ncols values into LDS, one after the other */
+__device__ inline void f32_rows_to_lds(const float *__restrict__ x, int ncols, int first, int n, uint8_t *lds) {
+    const Buf b = make_buf(x + (size_t)first * ncols, (uint32_t)n * (uint32_t)ncols * 4u);
+    for (int u = threadIdx.x; u < n * ncols / 4; u += blockDim.x)
+        *reinterpret_cast<u32x4 *>(lds + 16u * u) = ld16(b, 16u * (uint32_t)u);
+}
+/* row s of the rows staged in LDS: q8, or f32 for F16 weights */
+template <class F>
+__device__ inline auto staged_row(const uint8_t *xl, int ncols, int nb, int s) {
+    if constexpr (F::FMT == TG_FMT_F16) return F32Lds{xl + (size_t)s * ncols * 4};
+    else return q8_lds_slot(xl, nb, s);
 }
 
-constexpr int Q8X_MAXP = 4;   /* row passes per wave whose weights are loaded before the q8 */
+constexpr int GEMV_Q8_BATCH = 2;   /* blocks per wave whose loads are in flight together (4 cost registers) */
 
-/* One job's share of k_gemv_q8x: the rows of gemv_rows for wave `wave` of
- * the job, against the q8 row the workgroup builds in LDS.  When each lane
- * holds one item of a row (T == 1), the wave's weights are requested before
- * the q8 is built, so the two latencies overlap; the dots are the same
- * operations in the same order as gemv_rows. */
-template <class F, int S, int TB>
-__device__ inline void q8x_job(const GemvJob &jb, uint32_t rb, const float *__restrict__ x, int ncols, int nitems,
-                               int T, int rows_per_wave, int wave, uint8_t *xq, float *xd, int32_t *xs32,
-                               int32_t *xs16) {
+/* how k_gemv_staged gets its rows: as q8 rows, from f32 rows (q8 made in the
+ * kernel), or from a single f32 row */
+enum { GEMV_Q8 = 0, GEMV_QX = 1, GEMV_ONE = 2 };
+
+/* One job's share of k_gemv_staged for wave `wave` of the job's `nwaves`:
+ * rows in groups of 64/S, a lane's T <= TB items of the next two groups
+ * loading while the current one is dotted with the staged rows. */
+template <class F, int S, int TB, int QX>
+__device__ inline void gemv_staged_job(const GemvJob &jb, uint32_t rb, const float *__restrict__ xf, const Q8Rows &xq,
+                                       int ncols, int nb, int k, int kc, int nitems, int T, int wave, int nwaves,
+                                       uint8_t *xl) {
     constexpr int G = 64 / S;
-    const int lane = threadIdx.x & 63;
-    const int seg = lane / S, sl = lane % S;
-    const int row0 = wave * rows_per_wave;
-    const int nrw = max(0, min(rows_per_wave, jb.nrows - row0));   /* this wave's rows (0 past the job) */
-    const Buf wb = make_buf(jb.W + (size_t)min(row0, jb.nrows) * rb, (uint32_t)((size_t)nrw * rb));
-    const int P = (rows_per_wave + G - 1) / G;
-    const bool pre = T == 1 && P <= Q8X_MAXP;
-    typename F::W wp[Q8X_MAXP];
-    if (pre) {
+    const int lane = threadIdx.x & 63, seg = lane / S, sl = lane % S;
+    const int nrows = jb.nrows, step = nwaves * G;
+    struct Group {
+        typename F::W w[TB];
+        float bias;
+    };
+    /* past the last row: reads zeros, touches no memory */
+    auto load = [&](Group &g, int row0) __attribute__((always_inline)) {
+        const int n = max(0, min(G, nrows - row0)), at = min(row0, nrows);
+        const Buf b = make_buf(jb.W + (size_t)at * rb, (uint32_t)n * rb);
 #pragma unroll
-        for (int p = 0; p < Q8X_MAXP; p++) {
-            const int rl = p * G + seg;
-            const bool iv = p < P && rl < nrw && sl < nitems;
-            wp[p] = F::load_w(wb, iv ? (uint32_t)rl * rb : ROW_OOB, iv ? sl : 0);
+        for (int u = 0; u < TB; u++) {
+            const int item = sl + u * S;
+            const bool iv = seg < n && u < T && item < nitems;
+            g.w[u] = F::load_w(b, iv ? (uint32_t)seg * rb : ROW_OOB, iv ? item : 0);
         }
-    }
-    q8_row_lds(x, ncols, xq, xd, xs32, xs16);
-    __syncthreads();
-    if (nrw == 0) return;
-    const Q8Lds xr = {xq, reinterpret_cast<const uint8_t *>(xd), reinterpret_cast<const uint8_t *>(xs32),
-                      reinterpret_cast<const uint8_t *>(xs16)};
-    if (pre) {
-#pragma unroll
-        for (int p = 0; p < Q8X_MAXP; p++) {
-            const int rl = p * G + seg, r = row0 + rl;
-            if (p >= P) break;
-            const bool rv = rl < nrw;
+        const Buf bb = make_buf(jb.bias ? jb.bias + at : nullptr, jb.bias ? (uint32_t)n * 4u : 0u);
+        g.bias = __uint_as_float(ld4(bb, (uint32_t)seg * 4u));
+    };
+    auto dots = [&](const Group &g, int row0, int c0, int nc) __attribute__((always_inline)) {
+        const int r = row0 + seg;
+        const bool rv = r < nrows;
+        for (int s = 0; s < nc; s++) {
+            const auto xr = staged_row<F>(xl, ncols, nb, s);
             float acc = 0.f;
-            if (rv && sl < nitems) acc += F::value(wp[p], F::load_x(xr, sl), sl);
+#pragma unroll
+            for (int u = 0; u < TB; u++) {
+                const int item = sl + u * S;
+                if (rv && u < T && item < nitems) acc += F::value(g.w[u], F::load_x(xr, item), item);
+            }
             const float v = seg_sum<S>(acc);
-            if (rv && sl == 0) jb.y[r] = v + (jb.bias ? jb.bias[r] : 0.f);
+            if (rv && sl == 0) jb.y[(size_t)(c0 + s) * jb.ystride + r] = v + g.bias;
         }
-    } else {
-        for (int rs = 0; rs < rows_per_wave; rs += G) {
-            const int rl = rs + seg, r = row0 + rl;
-            const bool rv = rl < nrw;
-            float acc[1] = {0.f};
-            const Buf ws[1] = {wb};
-            row_dots<F, S, TB, 1>(ws, (uint32_t)rl * rb, rv, xr, sl, nitems, T, acc);
-            const float v = seg_sum<S>(acc[0]);
-            if (rv && sl == 0) jb.y[r] = v + (jb.bias ? jb.bias[r] : 0.f);
+    };
+    if (QX == GEMV_ONE) k = kc = 1;
+    for (int c0 = 0; c0 < k; c0 += kc) {
+        const int nc = QX == GEMV_ONE ? 1 : min(kc, k - c0);
+        int row = wave * G;
+        Group ga, gb;
+        Q8Quantize<GEMV_Q8_BATCH> qx;
+        Q8Copy<4> qc;
+        if (F::FMT != TG_FMT_F16) {
+            if (QX) qx.load(xf, ncols, RowsFrom{c0}, nc, nb);
+            else qc.load(xq, RowsFrom{c0}, nc);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        load(ga, row);
+        load(gb, row + step);
+        if (c0) bar_lds();   /* the previous rows are no longer read */
+        if (F::FMT == TG_FMT_F16) f32_rows_to_lds(xf, ncols, c0, nc, xl);
+        else if (QX) qx.finish(xf, ncols, RowsFrom{c0}, nc, nb, xl);
+        else qc.finish(xq, RowsFrom{c0}, nc, xl);
+        bar_lds();           /* the weights stay in flight */
+        for (; row < nrows; row += 2 * step) {
+            dots(ga, row, c0, nc);
+            load(ga, row + 2 * step);
+            if (row + step >= nrows) break;   /* uniform per wave */
+            dots(gb, row + step, c0, nc);
+            load(gb, row + 3 * step);
         }
     }
 }
 
-/* q8 of one f32 row and the GEMVs of up to three Q4_K / Q6_K matrices of
- * its width in one launch (decode attention's Q, K and V projections).
- * Every workgroup quantizes the row into LDS itself, with the arithmetic of
- * k_quantize_q8, then runs its rows as k_gemv_multi does, so the results are
- * the same bits.  The grid is flat: job j owns workgroups
- * [map.wg0[j], map.wg0[j + 1]).  Workgroup 0 also clears n_zero words at
- * `zero` (the counters of a kernel that follows). */
-template <int S, int TB>
-__global__ __launch_bounds__(256) void k_gemv_q8x(GemvJobs jobs, GemvQ8xMap map, const float *__restrict__ x,
-                                                  int ncols, int nitems, int T, int rows_per_wave, unsigned *zero,
-                                                  int n_zero) {
-    __shared__ __attribute__((aligned(16))) uint8_t xq[Q8X_MAX_BLOCKS * 256];
-    __shared__ __attribute__((aligned(16))) float xd[Q8X_MAX_BLOCKS];
-    __shared__ __attribute__((aligned(16))) int32_t xs32[Q8X_MAX_BLOCKS * 8];
-    __shared__ __attribute__((aligned(16))) int32_t xs16[Q8X_MAX_BLOCKS * 16];
+/* Bound: latency for one row of a small matrix (its launch, the rows' q8, one
+ * round trip for the weights); the v_dot4 and LDS reads per row beyond a few
+ * rows.  Before, k_gemv walked the rows one after another, re-reading the
+ * weights for each, and waited for a row's weights before it asked for the
+ * next: one q4_K row of 4096 x 2048 7.8 -> 5.0 us, nine 21.3 -> 12.0; q8_0
+ * 4096 x 2880, five rows 21.1 -> 11.6; mxfp4 2880 x 2880, 16 rows 52.4 ->
+ * 19.8; float16 1000 x 8000, one row 52.2 -> 8.3.
+ *
+ * Up to three matrices of one width and one format family (A and B: Q4_K
+ * and Q6_K, or Q8_0 and MXFP4, which cut a row into as many items; F16)
+ * against the same k rows.  A workgroup of four waves stages the q8 of kc
+ * rows in LDS (QX: quantizes them itself, with the arithmetic of
+ * k_quantize_q8; F16: the f32 rows) and reads its weights once for all of
+ * them, two row groups of each wave ahead.
+ * The grid is flat: job j owns workgroups [map.wg0[j], map.wg0[j + 1]).
+ * Workgroup 0 also clears n_zero words at `zero` (the counters of a kernel
+ * that follows). */
+template <class A, class B, int S, int TB, int QX>
+__global__ __launch_bounds__(256) void k_gemv_staged(GemvJobs jobs, GemvMap map, const float *__restrict__ xf,
+                                                     Q8Rows xq, int ncols, int k, int kc, int nitems, int T,
+                                                     unsigned *zero, int n_zero) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t xl[];
     if (blockIdx.x == 0 && (int)threadIdx.x < n_zero)
         __hip_atomic_store(zero + threadIdx.x, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     int j = 0;
     while (j < 2 && (int)blockIdx.x >= map.wg0[j + 1]) j++;
-    const int jw = ((int)blockIdx.x - map.wg0[j]) * 4 + (int)(threadIdx.x >> 6);
-    if (map.fmt[j] == TG_FMT_Q6K)
-        q8x_job<FQ6K, S, TB>(jobs.j[j], map.rb[j], x, ncols, nitems, T, rows_per_wave, jw, xq, xd, xs32, xs16);
+    const int wave = ((int)blockIdx.x - map.wg0[j]) * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int nwaves = (map.wg0[j + 1] - map.wg0[j]) * 4, nb = (ncols + 255) / 256;
+    if (map.fmt[j] == A::FMT)
+        gemv_staged_job<A, S, TB, QX>(jobs.j[j], map.rb[j], xf, xq, ncols, nb, k, kc, nitems, T, wave, nwaves, xl);
     else
-        q8x_job<FQ4K, S, TB>(jobs.j[j], map.rb[j], x, ncols, nitems, T, rows_per_wave, jw, xq, xd, xs32, xs16);
+        gemv_staged_job<B, S, TB, QX>(jobs.j[j], map.rb[j], xf, xq, ncols, nb, k, kc, nitems, T, wave, nwaves, xl);
 }
 
 /* ======================= MoE phases ======================= */
@@ -357,71 +479,8 @@ __global__ __launch_bounds__(256) void k_moe_b(MoeArgs a, int fmt, uint32_t rb, 
  * over the same items in the same order as k_moe_a / k_moe_b, so the
  * results are the same bits. */
 constexpr int MOE_X_MAXP = 8;
+constexpr int MOE_Q8_BATCH = 8;   /* blocks per wave whose loads are in flight together */
 static_assert(MOE_X_MAXP == EXP_ROWS, "the first chunk's rows come from the expert descriptor");
-
-/* q8 rows rows[0..n) of q into LDS slots 0..n-1 by the whole workgroup */
-__device__ inline void q8_rows_to_lds(const Q8Rows &q, const int *rows, int n, uint8_t *lds) {
-    const int nb = q.nb, per = nb * 22;   /* 16-byte units of qs, s32 and s16 */
-    for (int u = threadIdx.x; u < n * per; u += blockDim.x) {
-        const int s = u / per, v = u % per;
-        const size_t r = (size_t)rows[s];
-        const u32x4 *src;
-        uint32_t dst;
-        if (v < nb * 16) {
-            src = reinterpret_cast<const u32x4 *>(q.qs + r * nb * 256) + v;
-            dst = (uint32_t)v * 16;
-        } else if (v < nb * 18) {
-            src = reinterpret_cast<const u32x4 *>(q.s32 + r * nb * 8) + (v - nb * 16);
-            dst = nb * 256 + (uint32_t)(v - nb * 16) * 16;
-        } else {
-            src = reinterpret_cast<const u32x4 *>(q.s16 + r * nb * 16) + (v - nb * 18);
-            dst = nb * 288 + (uint32_t)(v - nb * 18) * 16;
-        }
-        *reinterpret_cast<u32x4 *>(lds + (size_t)s * q8_lds_stride(nb) + dst) = *src;
-    }
-    for (int u = threadIdx.x; u < n * nb; u += blockDim.x) {
-        const int s = u / nb, b = u % nb;
-        reinterpret_cast<float *>(lds + (size_t)s * q8_lds_stride(nb) + nb * 352)[b] = q.d[(size_t)rows[s] * nb + b];
-    }
-}
-
-/* q8 of f32 rows src[rows[s] * ld ..] (nb 256-value blocks each) into LDS
- * slots 0..n-1, block per wave, with the arithmetic of k_quantize_q8 (the
- * same bits).  With gw set, row s is also written to q8 row grows[s] of
- * gout. */
-constexpr int Q8Q_BATCH = 8;   /* blocks per wave whose loads are in flight together */
-__device__ inline void q8_quant_rows_lds(const float *__restrict__ src, int ld, const int *rows, int n, int nb,
-                                         uint8_t *lds, bool gw, Q8Rows gout, const int *grows) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    for (int u0 = wave; u0 < n * nb; u0 += nw * Q8Q_BATCH) {
-        u32x4 raw[Q8Q_BATCH];
-#pragma unroll
-        for (int i = 0; i < Q8Q_BATCH; i++) {
-            const int u = u0 + i * nw;
-            const bool uv = u < n * nb;
-            const int s = uv ? u / nb : 0, b = uv ? u % nb : 0;
-            /* a row's last block may be partial: zeros past its end, as k_quantize_q8 reads */
-            const Buf xb = make_buf(src + (size_t)rows[s] * ld + (size_t)b * 256,
-                                    uv ? (uint32_t)min(256, ld - b * 256) * 4u : 0u);
-            raw[i] = ld16(xb, (uint32_t)lane * 16u);
-        }
-#pragma unroll
-        for (int i = 0; i < Q8Q_BATCH; i++) {
-            const int u = u0 + i * nw;
-            if (u >= n * nb) continue;   /* uniform per wave */
-            const int s = u / nb, b = u % nb;
-            const float v0 = __uint_as_float(raw[i].x), v1 = __uint_as_float(raw[i].y);
-            const float v2 = __uint_as_float(raw[i].z), v3 = __uint_as_float(raw[i].w);
-            const Q8Quant q = q8_block_quant(v0, v1, v2, v3);
-            uint8_t *slot = lds + (size_t)s * q8_lds_stride(nb);
-            reinterpret_cast<uint32_t *>(slot + b * 256)[lane] = q.packed;
-            if ((lane & 3) == 0) reinterpret_cast<int32_t *>(slot + nb * 288)[b * 16 + (lane >> 2)] = q.s16;
-            if ((lane & 7) == 0) reinterpret_cast<int32_t *>(slot + nb * 256)[b * 8 + (lane >> 3)] = q.s32;
-            if (lane == 0) reinterpret_cast<float *>(slot + nb * 352)[b] = q.sc;
-            if (gw) q8_block_store(v0, v1, v2, v3, lane, gout, grows[s], b);
-        }
-    }
-}
 
 /* Phase A, expert-major: grid (x: wave groups over the I rows, y: active
  * expert a.mx_act[y]).  Each wave owns NP passes of 64/S rows, with all
@@ -463,10 +522,15 @@ __global__ __launch_bounds__(256) void k_moe_ax(MoeArgs a, int nitems, int T) {
         __syncthreads();   /* the previous chunk's rows are no longer read */
         if ((int)threadIdx.x < nc) srow[threadIdx.x] = c0 == 0 ? d.row[threadIdx.x] : a.p_row[p0 + c0 + threadIdx.x];
         __syncthreads();
-        if (QX)
-            q8_quant_rows_lds(a.xin, a.D, srow, nc, a.xq.nb, xl, false, a.xq, srow);
-        else
-            q8_rows_to_lds(a.xq, srow, nc, xl);
+        if (QX) {
+            Q8Quantize<MOE_Q8_BATCH> q;
+            q.load(a.xin, a.D, srow, nc, a.xq.nb);
+            q.finish(a.xin, a.D, srow, nc, a.xq.nb, xl);
+        } else {
+            Q8Copy<0> q;
+            q.load(a.xq, srow, nc);
+            q.finish(a.xq, srow, nc, xl);
+        }
         __syncthreads();
         for (int s = 0; s < nc; s++) {
             const Q8Lds xr = q8_lds_slot(xl, a.xq.nb, s);
@@ -538,10 +602,15 @@ __global__ __launch_bounds__(256) void k_moe_bx(MoeArgs a, int fmt, uint32_t rb,
         __syncthreads();
         if ((int)threadIdx.x < nc) srow[threadIdx.x] = p0 + c0 + threadIdx.x;
         __syncthreads();
-        if (QH)
-            q8_quant_rows_lds(a.hidden, a.I, srow, nc, a.hq.nb, xl, blockIdx.x == 0, a.hq, srow);
-        else
-            q8_rows_to_lds(a.hq, srow, nc, xl);
+        if (QH) {
+            Q8Quantize<MOE_Q8_BATCH> q;
+            q.load(a.hidden, a.I, srow, nc, a.hq.nb);
+            q.template finish<true>(a.hidden, a.I, srow, nc, a.hq.nb, xl, blockIdx.x == 0, a.hq, srow);
+        } else {
+            Q8Copy<0> q;
+            q.load(a.hq, srow, nc);
+            q.finish(a.hq, srow, nc, xl);
+        }
         __syncthreads();
         for (int s = 0; s < nc; s++) {
             const Q8Lds xr = q8_lds_slot(xl, a.hq.nb, s);
@@ -735,6 +804,30 @@ uint32_t row_bytes(int fmt, int ncols) {
         default: TG_DISPATCH_TB(TB_, 64, CALL) break;  \
     }
 static int pick_TB(int T) { return T >= 3 ? 4 : T; }
+/* the same for k_gemv_staged, which also has a form of three items */
+#define TG_DISPATCH_T4(TB_, S_, CALL)   \
+    switch (TB_) {                      \
+        case 1: CALL(S_, 1); break;     \
+        case 2: CALL(S_, 2); break;     \
+        case 3: CALL(S_, 3); break;     \
+        default: CALL(S_, 4); break;    \
+    }
+#define TG_DISPATCH_S4(S_, TB_, CALL)                  \
+    switch (S_) {                                      \
+        case 8: TG_DISPATCH_T4(TB_, 8, CALL) break;    \
+        case 16: TG_DISPATCH_T4(TB_, 16, CALL) break;  \
+        case 32: TG_DISPATCH_T4(TB_, 32, CALL) break;  \
+        default: TG_DISPATCH_T4(TB_, 64, CALL) break;  \
+    }
+
+/* k_gemv_staged's F16 forms of 8 and 16 items a lane */
+#define TG_DISPATCH_S16(S_, TB_)          \
+    switch (S_) {                         \
+        case 8: CALL16(8, TB_); break;    \
+        case 16: CALL16(16, TB_); break;  \
+        case 32: CALL16(32, TB_); break;  \
+        default: CALL16(64, TB_); break;  \
+    }
 
 #define TG_DISPATCH_F(fmt, BODY)                    \
     switch (fmt) {                                  \
@@ -753,24 +846,32 @@ void launch_quantize(const float *x, int ncols, int nrows, long xstride, const Q
                        clear ? nclear : 0);
 }
 
-void launch_gemv(int fmt, const uint8_t *W, int nrows, int ncols, const float *bias, const Q8Rows &x, int k,
-                 float *y, long ystride, hipStream_t st) {
-    int T;
-    const int nitems = items_per_row(fmt, ncols);
-    const int S = pick_S(nitems, &T);
-    const uint32_t rb = row_bytes(fmt, ncols);
-    const int G = 64 / S;
-    const int rpw = G * 2;
-    const int waves = (nrows + rpw - 1) / rpw;
-    dim3 grid((waves + 3) / 4);
-    const int TB = pick_TB(T);
-#define CALL(S_, TB_) \
-    hipLaunchKernelGGL((k_gemv<F, S_, TB_>), grid, dim3(256), 0, st, W, rb, nrows, bias, x, k, y, ystride, nitems, T, rpw)
-    TG_DISPATCH_F(fmt, TG_DISPATCH_ST(S, TB, CALL))
-#undef CALL
+static size_t device_max_lds() {
+    static int max_lds = -1;
+    if (max_lds < 0) {
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
+            max_lds = 0;
+    }
+    return (size_t)max_lds;
 }
 
-void launch_gemv_multi(int fmt, const GemvJobs &jobs, int njobs, int ncols, const Q8Rows &x, int k, hipStream_t st) {
+/* k_gemv_staged's grid: one row group a wave up to GEMV_ALL workgroups (all
+ * resident at once), else GEMV_WGS workgroups that walk several, so the rows
+ * are staged once for all of them (12,000 x 8192 q6_K, one row: 19.3 us
+ * against 25.0 with 1024 workgroups and 28.1 with 2048; q8_0 projections of
+ * 5,120 x 2880: two groups a wave are 2 us slower than 640 workgroups).
+ * GEMV_LDS bounds the staged rows: two workgroups a CU (12,000 x 8192, 16
+ * rows: 114 us; half of it 150, half as much again 167).  The kernel
+ * quantizes its rows itself up to GEMV_QX blocks, or one row of any width: a
+ * launch saved against every workgroup repeating the q8 (768 x 2048 q4_K,
+ * one row 7.6 -> 4.4 us; five rows of 768 8.7 -> 6.3; four rows of 2048
+ * 8.6 us with a q8 launch, 10.1 without). */
+constexpr int GEMV_ALL = 1024, GEMV_WGS = 512, GEMV_LDS = 80 << 10, GEMV_QX_BLOCKS = 16;
+
+static void launch_gemv_general(int fmt, const GemvJobs &jobs, int njobs, int ncols, const Q8Rows &x, int k,
+                                hipStream_t st) {
     int T;
     const int nitems = items_per_row(fmt, ncols);
     const int S = pick_S(nitems, &T);
@@ -780,46 +881,114 @@ void launch_gemv_multi(int fmt, const GemvJobs &jobs, int njobs, int ncols, cons
     for (int i = 0; i < njobs; i++) most = std::max(most, jobs.j[i].nrows);
     const int waves = (most + rpw - 1) / rpw;
     dim3 grid((waves + 3) / 4, njobs);
-    const int TB = pick_TB(T);
-#define CALL(S_, TB_) \
-    hipLaunchKernelGGL((k_gemv_multi<F, S_, TB_>), grid, dim3(256), 0, st, jobs, rb, x, k, nitems, T, rpw)
-    TG_DISPATCH_F(fmt, TG_DISPATCH_ST(S, TB, CALL))
+#define CALL(S_) hipLaunchKernelGGL((k_gemv<F, S_, 4>), grid, dim3(256), 0, st, jobs, rb, x, k, nitems, T, rpw)
+    TG_DISPATCH_F(fmt, TG_DISPATCH_S(S, CALL))
 #undef CALL
 }
 
-bool gemv_q8x_ok(const int *fmts, int njobs, int ncols) {
-    if (njobs < 1 || njobs > 3 || ncols <= 0 || ncols % 256 || ncols > Q8X_MAX_BLOCKS * 256) return false;
+/* formats that cut a row into as many items: one launch takes any of them */
+static int gemv_family(int fmt) { return fmt == TG_FMT_Q4K || fmt == TG_FMT_Q6K ? 0 : fmt == TG_FMT_F16 ? 2 : 1; }
+/* items a lane holds of a row, at most */
+static int gemv_max_t(int fmt) { return fmt == TG_FMT_F16 ? 16 : 4; }
+static uint32_t gemv_stride(int fmt, int ncols) {
+    return fmt == TG_FMT_F16 ? (uint32_t)ncols * 4u : q8_lds_stride((ncols + 255) / 256);
+}
+
+bool gemv_staged_ok(const int *fmts, int njobs, int ncols) {
+    if (njobs < 1 || njobs > 3 || ncols <= 0) return false;
     for (int i = 0; i < njobs; i++)
-        if (fmts[i] != TG_FMT_Q4K && fmts[i] != TG_FMT_Q6K) return false;
-    return true;
+        if (gemv_family(fmts[i]) != gemv_family(fmts[0])) return false;
+    const int nitems = items_per_row(fmts[0], ncols);
+    return nitems > 0 && nitems <= 64 * gemv_max_t(fmts[0]) && gemv_stride(fmts[0], ncols) <= device_max_lds();
+}
+
+static void launch_gemv_staged(const int *fmts, const GemvJobs &jobs, int njobs, int ncols, const float *xf,
+                               const Q8Rows &xq, int k, unsigned *zero, int n_zero, hipStream_t st) {
+    const int nitems = items_per_row(fmts[0], ncols);
+    int T, S = pick_S(nitems, &T);
+    while (T > gemv_max_t(fmts[0])) {
+        S *= 2;
+        T = (nitems + S - 1) / S;
+    }
+    const int G = 64 / S;
+    const uint32_t stride = gemv_stride(fmts[0], ncols);
+    const int kc = std::min(k, std::max(1, (int)(GEMV_LDS / stride)));
+    /* a workgroup's row groups: one a wave while the grid stays within
+     * GEMV_WGS workgroups, more above, so the staging is paid once */
+    int wgs[3] = {0, 0, 0}, total = 0;
+    for (int i = 0; i < njobs; i++) total += wgs[i] = (jobs.j[i].nrows + 4 * G - 1) / (4 * G);
+    const int iters = total <= GEMV_ALL ? 1 : (total + GEMV_WGS - 1) / GEMV_WGS;
+    GemvMap m;
+    int wg = 0;
+    for (int i = 0; i < 3; i++) {
+        m.wg0[i] = wg;
+        m.fmt[i] = i < njobs ? fmts[i] : fmts[0];
+        m.rb[i] = i < njobs ? row_bytes(fmts[i], ncols) : 0;
+        wg += (wgs[i] + iters - 1) / iters;
+    }
+    m.wg0[3] = wg;
+    const size_t lds = (size_t)kc * stride;
+#define CALL(S_, TB_)                                                                                                 \
+    do {                                                                                                              \
+        if (xf && k == 1)                                                                                             \
+            hipLaunchKernelGGL((k_gemv_staged<A, B, S_, TB_, GEMV_ONE>), dim3(wg), dim3(256), lds, st, jobs, m, xf,   \
+                               xq, ncols, k, kc, nitems, T, zero, n_zero);                                            \
+        else if (xf)                                                                                                  \
+            hipLaunchKernelGGL((k_gemv_staged<A, B, S_, TB_, GEMV_QX>), dim3(wg), dim3(256), lds, st, jobs, m, xf,    \
+                               xq, ncols, k, kc, nitems, T, zero, n_zero);                                            \
+        else                                                                                                          \
+            hipLaunchKernelGGL((k_gemv_staged<A, B, S_, TB_, GEMV_Q8>), dim3(wg), dim3(256), lds, st, jobs, m, xf,    \
+                               xq, ncols, k, kc, nitems, T, zero, n_zero);                                            \
+    } while (0)
+    if (gemv_family(fmts[0]) == 0) {
+        typedef FQ4K A;
+        typedef FQ6K B;
+        TG_DISPATCH_S4(S, T, CALL)
+    } else if (gemv_family(fmts[0]) == 1) {
+        typedef FQ80 A;
+        typedef FMXFP4 B;
+        TG_DISPATCH_S4(S, T, CALL)
+    } else {
+        typedef FF16 A;
+        typedef FF16 B;
+#define CALL16(S_, TB_)                                                                                               \
+    hipLaunchKernelGGL((k_gemv_staged<A, B, S_, TB_, GEMV_QX>), dim3(wg), dim3(256), lds, st, jobs, m, xf, xq, ncols, k, \
+                       kc, nitems, T, zero, n_zero)
+        if (T > 8) TG_DISPATCH_S16(S, 16)
+        else if (T > 4) TG_DISPATCH_S16(S, 8)
+        else TG_DISPATCH_S4(S, T, CALL16)
+#undef CALL16
+    }
+#undef CALL
 }
 
 void launch_gemv_q8x(const int *fmts, const GemvJobs &jobs, int njobs, int ncols, const float *x, unsigned *zero,
                      int n_zero, hipStream_t st) {
-    int T;
-    const int nitems = items_per_row(TG_FMT_Q4K, ncols);   /* Q6_K rows have as many items */
-    const int S = pick_S(nitems, &T);
-    const int rpw = (64 / S) * 2;
-    GemvQ8xMap m;
-    int wg = 0;
-    for (int i = 0; i < 3; i++) {
-        m.wg0[i] = wg;
-        if (i < njobs) {
-            m.fmt[i] = fmts[i];
-            m.rb[i] = row_bytes(fmts[i], ncols);
-            const int waves = (jobs.j[i].nrows + rpw - 1) / rpw;
-            wg += (waves + 3) / 4;
-        } else {
-            m.fmt[i] = TG_FMT_Q4K;
-            m.rb[i] = 0;
-        }
+    launch_gemv_staged(fmts, jobs, njobs, ncols, x, Q8Rows{}, 1, zero, n_zero, st);
+}
+
+void launch_gemv_multi(int fmt, const GemvJobs &jobs, int njobs, int ncols, const Q8Rows &x, int k, hipStream_t st) {
+    const int fmts[3] = {fmt, fmt, fmt};
+    if (gemv_staged_ok(fmts, njobs, ncols))
+        launch_gemv_staged(fmts, jobs, njobs, ncols, fmt == TG_FMT_F16 ? x.f : nullptr, x, k, nullptr, 0, st);
+    else launch_gemv_general(fmt, jobs, njobs, ncols, x, k, st);
+}
+
+void launch_gemv(int fmt, const uint8_t *W, int nrows, int ncols, const float *bias, const Q8Rows &x, int k,
+                 float *y, long ystride, hipStream_t st) {
+    const GemvJobs jobs = {{{W, bias, y, ystride, nrows}}};
+    launch_gemv_multi(fmt, jobs, 1, ncols, x, k, st);
+}
+
+void launch_matmul(int fmt, const uint8_t *W, int nrows, int ncols, const float *bias, const float *xf,
+                   const Q8Rows &x, int k, float *y, long ystride, hipStream_t st) {
+    if (gemv_staged_ok(&fmt, 1, ncols) && (k == 1 || k * ((ncols + 255) / 256) <= GEMV_QX_BLOCKS)) {
+        const GemvJobs jobs = {{{W, bias, y, ystride, nrows}}};
+        launch_gemv_staged(&fmt, jobs, 1, ncols, xf, x, k, nullptr, 0, st);
+        return;
     }
-    m.wg0[3] = wg;
-    const int TB = pick_TB(T);
-#define CALL(S_, TB_) \
-    hipLaunchKernelGGL((k_gemv_q8x<S_, TB_>), dim3(wg), dim3(256), 0, st, jobs, m, x, ncols, nitems, T, rpw, zero, n_zero)
-    TG_DISPATCH_ST(S, TB, CALL)
-#undef CALL
+    if (fmt != TG_FMT_F16) launch_quantize(xf, ncols, k, ncols, x, st);
+    launch_gemv(fmt, W, nrows, ncols, bias, x, k, y, ystride, st);
 }
 
 void launch_isums(int fmt, const uint8_t *W, int nrows, int ncols, const Q8Rows &x, int nsums_row, int32_t *out,
@@ -861,16 +1030,6 @@ int expert_major() { return g_expert_major; }
 /* the expert-major phases stage up to MOE_X_MAXP q8 rows of nb blocks in
  * dynamic LDS; wider rows than the device allows fall back to the per-pair
  * kernels */
-static size_t device_max_lds() {
-    static int max_lds = -1;
-    if (max_lds < 0) {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
-            max_lds = 0;
-    }
-    return (size_t)max_lds;
-}
 static bool expert_major_ok(const MoeArgs &a, int fmt, int T, int nb) {
     const size_t lds = (size_t)std::min(a.max_rows, MOE_X_MAXP) * q8_lds_stride(nb);
     return (g_expert_major & EM_ON) && a.n_act_a > 0 && T <= 4 && lds <= device_max_lds() &&
