@@ -127,3 +127,23 @@ def test_qk_equals_dot4_phases(tg, orc):
     ok, rel = close(outs["mfma"], ref_b)
     assert ok, ("down+combine", rel)
     say(f"  mfma vs dot4 end-to-end rel {np.abs(outs['mfma'] - outs['dot4']).max() / np.abs(outs['dot4']).max():.2e}")
+
+
+@pytest.mark.parametrize("counts,bias", [
+    ((1, 16, 17, 32, 33), False), ((31, 15, 2), True), ((64, 65, 1, 48, 47), False), ((97,), True)])
+def test_qk_ring_pair_counts(tg, orc, counts, bias):
+    """Experts of one to four passes of up to 32 pairs on the persistent rings'
+    shape (D 2048, I 768), at the edges of their tiles of 16: one tile, a
+    second of one pair, two full ones; gate/up biases with the gpt-oss
+    activation (a down bias, which _check_moe adds too, takes the grid form
+    of the down phase)."""
+    k = max(counts)
+    rng = np.random.default_rng(sum(counts))
+    rw = np.zeros((len(counts), k), np.float32)
+    for e, c in enumerate(counts):
+        rw[e, rng.choice(k, c, replace=False)] = rng.uniform(0.1, 1.0, c)
+    x = rng.standard_normal((k, 2048)).astype(np.float32)
+    say("qk ring pairs", counts, bias)
+    with _qk_rows(tg, 1):
+        _check_moe(tg, orc, len(counts), k, 2048, 768, O.FMT_Q4K, [O.FMT_Q6K] * len(counts),
+                   O.ACT_GPTOSS if bias else O.ACT_SILU, bias, rw, x)

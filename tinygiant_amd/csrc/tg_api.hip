@@ -558,9 +558,9 @@ MoeArgs plan_args(const HostPlan &h, const Layout &L, uint8_t *dev, uint8_t *img
      * first instead of trailing the launch */
     std::stable_sort(ed.begin(), ed.end(), [](const ExpDesc &x, const ExpDesc &y) { return x.np > y.np; });
     a.ed = (const ExpDesc *)put(ed.data(), ed.size() * sizeof(ExpDesc));
-    if (qa_ring_shape(h.gate_fmt, h.D, h.I) && a.n_act_a > 0) {
+    if (qa_ring_shape(h.gate_fmt, h.D, h.I) && a.n_act_a > 0 && a.max_rows <= RING_MAX_ROWS) {
         RingLists r;
-        ring_items(ed.data(), a.n_act_a, h.I / 16, cu_count(), h.p_row.data(), P, r);
+        ring_items(ed.data(), a.n_act_a, h.I / 16, cu_count(), h.p_row.data(), P, QA_RING_COST, r);
         a.rg_items = (const int *)put(r.items.data(), r.items.size() * 4);
         a.rg_rend = (const int *)put(r.rend.data(), r.rend.size() * 4);
         a.rg_runs = (const int *)put(r.runs.data(), r.runs.size() * 4);
@@ -568,9 +568,9 @@ MoeArgs plan_args(const HostPlan &h, const Layout &L, uint8_t *dev, uint8_t *img
         a.rg_off = (const int *)put(r.off.data(), r.off.size() * 4);
         a.rg_n = (int)r.off.size() - 1;
     }
-    if (qb_ring_shape(h.I, h.D) && a.n_act_a > 0) {
+    if (qb_ring_shape(h.I, h.D) && a.n_act_a > 0 && a.max_rows <= RING_MAX_ROWS) {
         RingLists r;
-        ring_items(ed.data(), a.n_act_a, h.D / 32, cu_count(), h.p_row.data(), P, r);
+        ring_items(ed.data(), a.n_act_a, h.D / 32, cu_count(), h.p_row.data(), P, QB_RING_COST, r);
         a.rb_items = (const int *)put(r.items.data(), r.items.size() * 4);
         a.rb_rend = (const int *)put(r.rend.data(), r.rend.size() * 4);
         a.rb_runs = (const int *)put(r.runs.data(), r.runs.size() * 4);

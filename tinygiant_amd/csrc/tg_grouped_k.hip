@@ -43,6 +43,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "tg_device.hpp"
 #include "tg_kernels.h"
@@ -112,6 +113,13 @@ __device__ inline Q4Hdr q4_hdr(u32x4 h) {
     r.mnh = ((h.w >> 4) & m4) | ((h.z >> 2) & 0x30303030u);
     return r;
 }
+/* a word's four bytes (each product below 256) times a factor held in both
+ * halves of f */
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+__device__ inline int mul_bytes(uint32_t q, uint32_t f) {
+    return __builtin_bit_cast(int, (u16x2)(__builtin_bit_cast(u16x2, q) * __builtin_bit_cast(u16x2, f)));
+}
+
 __device__ inline int byte_of(uint32_t w, int i) { return (int)((w >> (8 * i)) & 0xFFu); }
 
 /* copy_lanes with the nontemporal hint: each slab byte is read once per
@@ -289,54 +297,71 @@ __global__ __launch_bounds__(NT) void k_moe_qa(MoeArgs a) {
 
 /* Phase A, persistent, for Q4_K gate/up rows of D = 2048 (8 blocks): one
  * workgroup a compute unit walks its list of items (active expert, 16-row
- * slab, pass of 16 pairs), the slabs streaming through a ring of four LDS
- * slots three items ahead of the item computed, so a compute unit always
- * has weight bytes in flight.
+ * slab, pass of up to RING_P = 32 pairs), the slabs streaming through a ring
+ * of three LDS slots two items ahead of the item computed, so a compute unit
+ * always has weight bytes in flight.
  *
  * Eight compute waves: wave c takes matrix c / 4 (gate, up) and blocks
  * c % 4 and c % 4 + 4 of it, so the partial sums of a block pair meet in
  * LDS in the order of the expert-major kernel (wave order).  They hold the
- * q8 operands of a run of items with the same expert and pass, loaded once
- * a run (a compute unit returns its loads in issue order, so operands loaded
- * per item would wait behind the slabs in flight each time); a workgroup's
- * list is a contiguous stretch of the layer's items ordered expert, pass,
- * slab, so it holds a few runs.  Two copy waves issue the slab copies
+ * q8 operands of a run of items with the same expert and pass, one or two
+ * tiles of 16 pairs, loaded once a run (a compute unit returns its loads in
+ * issue order, so operands loaded per item would wait behind the slabs in
+ * flight each time; for the same reason the loop must hold no spilled
+ * register: a scratch reload waits there too); a workgroup's list is a
+ * contiguous stretch of the layer's items ordered expert, pass, slab, so it
+ * holds a few runs.  They also finish the previous item (its partial sums,
+ * double-buffered in LDS, the activation, the hidden values), one result a
+ * lane, one barrier an item.  Two copy waves issue the slab copies
  * (direct-to-LDS, one matrix each) and nothing else, so each waits for its
- * own with exact counts; two finishing waves finish the previous item (its
- * partial sums, double-buffered in LDS, the activation, the hidden values)
- * while the compute waves work on the current one, one barrier an item.
+ * own with exact counts.
  *
  * A slab's LDS image swizzles each row's 16-byte units within aligned
  * groups of eight (unit u of row r at 72 r + (u ^ ((r >> 1) & 7))): the 16
- * rows a lane group reads at one column then fall on distinct banks. */
+ * rows a lane group reads at one column then fall on distinct banks.
+ *
+ * Bound: an item of one tile takes 1.6 us, the slab's 36 KiB at a compute
+ * unit's share of HBM (1.5 us); of two tiles 2.3 us, VALU and MFMA issue of
+ * the two compute waves of a SIMD.  With one tile a pass every further 16
+ * pairs of an expert streamed its slabs again: 509 tokens (313 passes of 16
+ * pairs, 204 of 32) 107 -> 91 us, the layer with both rings 245 -> 194; 33
+ * tokens 33 -> 32 us and 80 -> 72. */
 constexpr int RG_NB = 8;                              /* Q4_K blocks of a row */
 constexpr int RG_UNITS = RG_NB * 9;                   /* 16-byte units of a 1152-byte row */
 constexpr int RG_SLAB = 16 * RG_UNITS * 16;           /* 18,432 bytes: one matrix's 16 rows */
 constexpr int RG_COPIES = RG_SLAB / 1024;             /* 18 copies of 1 KiB */
-constexpr int RG_SLOTS = 4;
-constexpr int RG_CW = 8, RG_YW = 2, RG_FW = 2;        /* compute, copy and finishing waves */
+constexpr int RG_SLOTS = 3;
+constexpr int RG_CW = 8, RG_YW = 2;                   /* compute and copy waves */
 constexpr int RG_LC = RG_COPIES;                      /* copies a copy wave issues per item (its matrix's slab) */
-constexpr int RG_NT = 64 * (RG_CW + RG_YW + RG_FW);
-constexpr int RG_FO = 16 * 16 / (64 * RG_FW);         /* (pair, row) results a finishing thread writes */
-static_assert(2 * RG_LC <= 63, "a vmcnt count");
+constexpr int RG_NT = 64 * (RG_CW + RG_YW);
+static_assert((RG_SLOTS - 2) * RG_LC <= 63, "a vmcnt count");
 static_assert(RG_SLAB % 1024 == 0, "whole copies");
 static_assert(RG_UNITS % 8 == 0, "the swizzle stays inside a row");
 
+/* Workgroup g runs on XCD g % 8: neighbouring stretches of the item list go
+ * to one XCD, so the passes of an expert read its slabs from that XCD's L2 */
+__device__ inline int ring_wg() {
+    const int g = (int)blockIdx.x, G = (int)gridDim.x;
+    return G % 8 ? g : (g % 8) * (G / 8) + g / 8;
+}
+
 __device__ inline uint32_t rg_unit(int r, int u) { return (uint32_t)(RG_UNITS * r + (u ^ ((r >> 1) & 7))); }
 
-struct RgX {   /* a compute lane's q8 operands of one run, blocks c % 4 and c % 4 + 4 */
-    long xb[2][8];
-    uint32_t bs0[2], bs1[2], xd[2];
-    float xdv[2][4];   /* the scales of pairs 4 g .. 4 g + 3, set once the run starts */
+struct RgX {   /* a compute lane's q8 operands of one run, blocks c % 4 and c % 4 + 4 of its pair in each tile */
+    v4i xb[RING_T][2][2][2];  /* [tile][block][half of the block][low, high nibbles]: 16 values */
+    uint32_t bs[RING_T][2];   /* 32-value sums (below 2^13) of sub-blocks g and 4 + g, 16 bits each */
+    int nt;   /* tiles that hold pairs */
 };
 
 __global__ __launch_bounds__(RG_NT) void k_moe_qa_ring(MoeArgs a) {
     __shared__ __attribute__((aligned(16))) uint8_t ring[RG_SLOTS][2][RG_SLAB];
-    __shared__ __attribute__((aligned(16))) float red[2][RG_CW][4][64];   /* by item parity */
+    __shared__ __attribute__((aligned(16))) float red[2][RING_T][RG_CW][4][64];   /* by item parity */
+    __shared__ __attribute__((aligned(16))) float xdl[RG_CW][RING_T][2][16];      /* the run's q8 scales */
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4,
               c16 = lane & 15;
-    const bool loader = w >= RG_CW, copier = loader && w < RG_CW + RG_YW;
-    const int i0 = ldc(a.rg_off, blockIdx.x), n = ldc(a.rg_off, blockIdx.x + 1) - i0;
+    const bool copier = w >= RG_CW;
+    const int wg = ring_wg();
+    const int i0 = ldc(a.rg_off, wg), n = ldc(a.rg_off, wg + 1) - i0;
     if (n <= 0) return;   /* uniform */
     const uint32_t mbytes = (uint32_t)a.I * (RG_NB * Q4B);
     const Q8Rows &q = a.xq;
@@ -362,23 +387,6 @@ __global__ __launch_bounds__(RG_NT) void k_moe_qa_ring(MoeArgs a) {
         f.s = (it >> 8) & 255;
         return f;
     };
-    struct Fin {   /* a finishing wave's: slab, pairs, biases */
-        int s, tp, p0, np, e;
-        const float *gb, *ub;
-    };
-    auto fin_head = [&](int it) __attribute__((always_inline)) {
-        Fin f;
-        f.s = (it >> 8) & 255;
-        f.tp = 16 * (it & 255);
-        f.p0 = ldc(&a.ed[it >> 16].p0, 0);
-        f.np = ldc(&a.ed[it >> 16].np, 0);
-        f.e = ldc(&a.ed[it >> 16].e, 0);
-        return f;
-    };
-    auto fin_bias = [&](Fin &f) __attribute__((always_inline)) {
-        f.gb = a.gbias ? (const float *)(uintptr_t)ldc(a.gbias, f.e) : nullptr;
-        f.ub = a.ubias ? (const float *)(uintptr_t)ldc(a.ubias, f.e) : nullptr;
-    };
     /* the copy wave's matrix slab of item j, 18 KiB */
     auto issue_copies = [&](int j, const Info &f) __attribute__((always_inline)) {
         const int s = f.s, m = w - RG_CW;
@@ -392,105 +400,184 @@ __global__ __launch_bounds__(RG_NT) void k_moe_qa_ring(MoeArgs a) {
     };
     /* the loader wave waits for item j's copies, k items' copies issued after them */
     auto wait_copies_behind = [&](int k) __attribute__((always_inline)) {
-        if (k >= 2) wait_copies_but<2 * RG_LC>();
-        else if (k == 1) wait_copies_but<RG_LC>();
+        if (k >= 1) wait_copies_but<RG_LC>();
         else wait_copies_but<0>();
     };
-    static_assert(RG_SLOTS - 2 == 2, "wait_copies_behind covers the items in flight");
-    /* the compute lane's operands of run r: its pair c16, whose input row the
-     * run's record holds (one round trip of scalar loads) */
+    static_assert(RG_SLOTS - 2 == 1, "wait_copies_behind covers the items in flight");
+    /* the compute lane's operands of run r: its pair c16 of each tile, whose
+     * input row the run's record holds (one round trip of scalar loads) */
     auto load_x = [&](int r, RgX &x) __attribute__((always_inline)) {
         const int *rc = a.rg_runs + (size_t)RING_REC * r;
         const int nv = ldc(rc, 1);
-        uint32_t rj[16];
+        x.nt = nv > 16 ? 2 : 1;
+        uint32_t bs0[RING_T][2], bs1[RING_T][2], xd[RING_T][2];
 #pragma unroll
-        for (int jj = 0; jj < 16; jj++) rj[jj] = (uint32_t)ldc(rc, 2 + jj);
-        uint32_t prow = 0u;
+        for (int t = 0; t < RING_T; t++) {
+            if (t >= x.nt) break;   /* uniform */
+            uint32_t rj[16];
 #pragma unroll
-        for (int jj = 0; jj < 16; jj++) prow = c16 == jj ? rj[jj] : prow;
-        const bool pv = c16 < nv;
+            for (int jj = 0; jj < 16; jj++) rj[jj] = (uint32_t)ldc(rc, 2 + 16 * t + jj);
+            uint32_t prow = 0u;
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const uint32_t qb = prow * RG_NB + (uint32_t)(bw + 4 * h);
+            for (int jj = 0; jj < 16; jj++) prow = c16 == jj ? rj[jj] : prow;
+            const bool pv = 16 * t + c16 < nv;
 #pragma unroll
-            for (int s = 0; s < 8; s++)
-                x.xb[h][s] = as_long(ld8(qs_b, pv ? qb * 256u + 64u * (s >> 1) + 32u * (s & 1) + 8u * g : OOB));
-            x.bs0[h] = ld4(s32_b, pv ? qb * 32u + 4u * g : OOB);
-            x.bs1[h] = ld4(s32_b, pv ? qb * 32u + 16u + 4u * g : OOB);
-            x.xd[h] = ld4(d_b, pv ? qb * 4u : OOB);
+            for (int h = 0; h < 2; h++) {
+                /* one offset a lane and buffer, the rest in the instructions */
+                const uint32_t qb = prow * RG_NB + (uint32_t)(bw + 4 * h);
+                const uint32_t oq = pv ? qb * 256u + 64u * (g >> 1) + 16u * (g & 1) : OOB, os = pv ? qb * 32u + 4u * g : OOB;
+#pragma unroll
+                for (int s = 0; s < 4; s++)
+                    x.xb[t][h][s >> 1][s & 1] = __builtin_bit_cast(v4i, ld16(qs_b, oq + 128u * (s >> 1) + 32u * (s & 1)));
+                bs0[t][h] = ld4(s32_b, os);
+                bs1[t][h] = ld4(s32_b, os + 16u);
+                xd[t][h] = ld4(d_b, pv ? qb * 4u : OOB);
+            }
+        }
+        /* taken as the values of an empty asm statement: the compiler waits
+         * for the loads there and not at their uses */
+#pragma unroll
+        for (int t = 0; t < RING_T; t++) {
+            if (t >= x.nt) break;
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                v4i(&xb)[2][2] = x.xb[t][h];
+                asm volatile(""
+                             : "+v"(xb[0][0]), "+v"(xb[0][1]), "+v"(xb[1][0]), "+v"(xb[1][1]), "+v"(bs0[t][h]), "+v"(bs1[t][h]), "+v"(xd[t][h]));
+                x.bs[t][h] = (bs0[t][h] & 0xFFFFu) | (bs1[t][h] << 16);
+                /* the pairs' scales, where a lane finds those of its four result
+                 * pairs side by side (the wave's own words, in order) */
+                xdl[w][t][h][c16] = __uint_as_float(xd[t][h]);
+            }
         }
     };
     /* compute item j from its slot with operands x: the wave's two blocks of
-     * its matrix, their sums to red */
-    auto compute = [&](int j, const RgX &x) __attribute__((always_inline)) {
+     * its matrix against NT tiles of pairs, their sums to red.  The codes and
+     * scales are unpacked once for all tiles. */
+    auto compute = [&](int j, const RgX &x, auto tiles) __attribute__((always_inline)) {
+        constexpr int NT_ = decltype(tiles)::value;
         const uint8_t *sb = &ring[j % RG_SLOTS][mw][0];
-        float acc[4] = {0.f, 0.f, 0.f, 0.f};
+        /* byte 2 (g / 2) (or the next) of a word of scales in both its halves */
+        const uint32_t sel0 = 0x0C000C00u + 0x00020002u * (uint32_t)(g >> 1), sel1 = sel0 + 0x00010001u;
+        /* every LDS read of the item first: read where they are used, each
+         * would add its latency to the item (12 reads, 2 waves a SIMD) */
+        u32x4 hd[2];
+        u32x4 qc[2][2];   /* 16 bytes of codes of each half block */
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             const int b = bw + 4 * h;
-            const float *xdv = x.xdv[h];
-            const Q4Hdr hr = q4_hdr(*(const u32x4 *)(sb + 16 * rg_unit(c16, 9 * b)));
-            v4f im = {0.f, 0.f, 0.f, 0.f};
-            im = __builtin_amdgcn_mfma_f32_16x16x4f32((float)(int)x.bs0[h], (float)byte_of(hr.mnl, g), im, 0, 0, 0);
-            im = __builtin_amdgcn_mfma_f32_16x16x4f32((float)(int)x.bs1[h], (float)byte_of(hr.mnh, g), im, 0, 0, 0);
-            int isc[4] = {0, 0, 0, 0};
+            hd[h] = *(const u32x4 *)(sb + 16 * rg_unit(c16, 9 * b));
 #pragma unroll
-            for (int jg = 0; jg < 4; jg++) {
-                const u32x2 qq = *(const u32x2 *)(sb + 16 * rg_unit(c16, 9 * b + 1 + 2 * jg + (g >> 1)) + 8 * (g & 1));
-                u32x2 lo, hi;
-                lo.x = qq.x & 0x0F0F0F0Fu;
-                lo.y = qq.y & 0x0F0F0F0Fu;
-                hi.x = (qq.x >> 4) & 0x0F0F0F0Fu;
-                hi.y = (qq.y >> 4) & 0x0F0F0F0Fu;
-                const v4i dl = mma(x.xb[h][2 * jg], as_long(lo));
-                const v4i dh = mma(x.xb[h][2 * jg + 1], as_long(hi));
-                const uint32_t scw = jg < 2 ? hr.scl : hr.sch;
-                const int s0 = byte_of(scw, 2 * (jg & 1)), s1 = byte_of(scw, 2 * (jg & 1) + 1);
+            for (int p = 0; p < 2; p++) qc[h][p] = *(const u32x4 *)(sb + 16 * rg_unit(c16, 9 * b + 1 + 4 * p + g));
+        }
+        v4f xdv[NT_][2];
 #pragma unroll
-                for (int v = 0; v < 4; v++) isc[v] += __mul24(s0, dl[v]) + __mul24(s1, dh[v]);
+        for (int t = 0; t < NT_; t++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) xdv[t][h] = *(const v4f *)&xdl[w][t][h][4 * g];
+        __builtin_amdgcn_sched_barrier(0);
+        float acc[NT_][4];
+#pragma unroll
+        for (int t = 0; t < NT_; t++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) acc[t][v] = 0.f;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const Q4Hdr hr = q4_hdr(hd[h]);
+            /* sum_s sc[row][s] idot[pair][row][s], exact in int32, without a
+             * multiply per (pair, row, sub-block): the weight codes are scaled
+             * before the product.  A 6-bit scale is 8 h + l, and a code times
+             * h or l stays below 128, so x . (q l) and x . (q h) accumulate
+             * over the whole block inside the MFMAs and meet at the end as
+             * l + 8 h.  The scaling is shared by all pairs.  With the scales
+             * inside, one MFMA may mix sub-blocks: a lane takes 16 bytes of
+             * codes as they lie (bytes 16 g of half p: 16 values of sub-block
+             * 4 p + 2 (g / 2) in the low nibbles, of the next in the high
+             * ones), so its q8 values are 16-byte pieces too. */
+            v4i il[NT_], ih[NT_];
+#pragma unroll
+            for (int t = 0; t < NT_; t++) il[t] = ih[t] = v4i{0, 0, 0, 0};
+#pragma unroll
+            for (int p = 0; p < 2; p++) {
+                const uint32_t sc = p ? hr.sch : hr.scl, s3 = sc & 0x07070707u, s8 = (sc >> 3) & 0x07070707u;
+#pragma unroll
+                for (int n = 0; n < 2; n++) {
+                    u32x4 q4 = qc[h][p];
+                    if (n) q4 >>= 4;
+                    q4 &= 0x0F0F0F0Fu;
+                    const uint32_t fl = __builtin_amdgcn_perm(0u, s3, n ? sel1 : sel0);
+                    const uint32_t fh = __builtin_amdgcn_perm(0u, s8, n ? sel1 : sel0);
+                    const v4i cl = {mul_bytes(q4.x, fl), mul_bytes(q4.y, fl), mul_bytes(q4.z, fl), mul_bytes(q4.w, fl)};
+                    const v4i ch = {mul_bytes(q4.x, fh), mul_bytes(q4.y, fh), mul_bytes(q4.z, fh), mul_bytes(q4.w, fh)};
+#pragma unroll
+                    for (int t = 0; t < NT_; t++) {
+                        il[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x.xb[t][h][p][n], cl, il[t], 0, 0, 0);
+                        ih[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x.xb[t][h][p][n], ch, ih[t], 0, 0, 0);
+                    }
+                }
+            }
+            const float m0 = (float)byte_of(hr.mnl, g), m1 = (float)byte_of(hr.mnh, g);
+            v4f im[NT_];
+#pragma unroll
+            for (int t = 0; t < NT_; t++) {
+                im[t] = v4f{0.f, 0.f, 0.f, 0.f};
+                im[t] = __builtin_amdgcn_mfma_f32_16x16x4f32((float)(int)(int16_t)x.bs[t][h], m0, im[t], 0, 0, 0);
+                im[t] = __builtin_amdgcn_mfma_f32_16x16x4f32((float)((int)x.bs[t][h] >> 16), m1, im[t], 0, 0, 0);
             }
 #pragma unroll
-            for (int v = 0; v < 4; v++) acc[v] += xdv[v] * (hr.d * (float)isc[v] - hr.dmin * im[v]);
+            for (int t = 0; t < NT_; t++)
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    acc[t][v] += xdv[t][h][v] * (hr.d * (float)(il[t][v] + 8 * ih[t][v]) - hr.dmin * im[t][v]);
         }
 #pragma unroll
-        for (int v = 0; v < 4; v++) red[j & 1][w][v][lane] = acc[v];
+        for (int t = 0; t < NT_; t++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) red[j & 1][t][w][v][lane] = acc[t][v];
     };
-    /* the finishing threads, RG_FO (pair, row) results each: the gate and
-     * up waves' sums in wave order, the activation, the hidden values of item
-     * j; the sums of pair 4 g + v and row c16 sit in lane 16 g + c16,
-     * register v */
-    auto finish = [&](int j, const Fin &fi) __attribute__((always_inline)) {
-        const int s = fi.s, tp = fi.tp, p0 = fi.p0, np = fi.np;
-        const float *gb = fi.gb, *ub = fi.ub;
+    /* finishing item j: a compute wave's lane takes one (pair, row) result,
+     * the gate and up waves' sums in wave order, the activation, the hidden
+     * value; wave w has tile w / 4, pairs 4 (w % 4) + g and row c16 of the
+     * slab, whose sums sit in lane 16 (w % 4) + c16, register g.  (Two
+     * finishing waves of their own set the pace: 1.4 us an item of one tile,
+     * 2.3 of two, behind compute waves that took 1.4 and 2.0.) */
+    struct Done {   /* the item to finish: its first pair, pairs from there, first row, biases */
+        int pf, nv, r;
+        float gb, ub;
+    };
+    auto finish = [&](int j, const Done &f) __attribute__((always_inline)) {
+        const int t = w >> 2;
+        if (16 * t >= f.nv) return;   /* uniform */
+        int ln = lane;
+        asm volatile("" : "+v"(ln));   /* what follows of it is computed here, not kept in registers */
+        const int g = ln >> 4, c16 = ln & 15, jj = 16 * t + 4 * (w & 3) + g;
+        const float *p = &red[j & 1][t][0][g][16 * (w & 3) + c16];
+        float gv = 0.f, uv = 0.f;
 #pragma unroll
-        for (int o = tid - 64 * (RG_CW + RG_YW), u = 0; u < RG_FO; u++, o += 64 * RG_FW) {
-            const int jj = o >> 4, rr = o & 15, ln = 16 * (jj >> 2) + rr, v = jj & 3;
-            float gv = 0.f, uv = 0.f;
-#pragma unroll
-            for (int ww = 0; ww < 4; ww++) {
-                gv += red[j & 1][ww][v][ln];
-                uv += red[j & 1][4 + ww][v][ln];
-            }
-            const int r = 16 * s + rr;
-            if (gb) gv += gb[r];
-            if (ub) uv += ub[r];
-            if (tp + jj < np) a.hidden[(size_t)(p0 + tp + jj) * a.I + r] = act_fn(a.act, gv, uv);
+        for (int ww = 0; ww < 4; ww++) {
+            gv += p[ww * 256];
+            uv += p[(4 + ww) * 256];
         }
+        if (a.gbias) {
+            gv += f.gb;
+            uv += f.ub;
+        }
+        if (jj < f.nv) a.hidden[(size_t)(f.pf + jj) * a.I + f.r + c16] = act_fn(a.act, gv, uv);
     };
     /* a run: items of one expert and pass */
     auto run_end = [&](int s) { return min(ldc(a.rg_rend, (size_t)(i0 + s)), i0 + n) - i0; };
 
-    /* The three roles run loops of their own (so the compiler's waits for
-     * the compute waves' operand loads never land in the others' code),
+    /* The two roles run loops of their own (so the compiler's waits for the
+     * compute waves' operand loads never land in the copy waves' code),
      * meeting at one barrier an item.  Between the barriers of items i and
-     * i + 1 the compute waves compute item i (reading slot i % 4, writing
-     * red[i % 2]) while the copy waves copy item i + 3 into item i - 1's slot
-     * and the finishing waves finish item i - 1 (reading red[(i - 1) % 2]):
-     * each wave reaches the next barrier only after its part. */
+     * i + 1 the compute waves finish item i - 1 (reading red[(i - 1) % 2]) and
+     * compute item i (reading slot i % RG_SLOTS, writing red[i % 2]) while
+     * the copy waves copy item i + 2 into item i - 1's slot: each wave
+     * reaches the next barrier only after its part. */
     if (copier) {
         for (int j = 0; j < RG_SLOTS - 1 && j < n; j++) issue_copies(j, info_code(item(j)));
-        Info fc = info_code(item(min(RG_SLOTS - 1, n - 1)));   /* item i + 3 */
-        int code = item(min(RG_SLOTS, n - 1));                  /* item i + 4 */
+        Info fc = info_code(item(min(RG_SLOTS - 1, n - 1)));   /* item i + RG_SLOTS - 1 */
+        int code = item(min(RG_SLOTS, n - 1));                  /* item i + RG_SLOTS */
         for (int i = 0; i < n; i++) {
             wait_copies_behind(min(RG_SLOTS - 2, n - 1 - i));
             /* a copy wave writes no LDS itself: its barrier leaves the scalar
@@ -504,68 +591,40 @@ __global__ __launch_bounds__(RG_NT) void k_moe_qa_ring(MoeArgs a) {
         wait_copies();   /* no copy outlives the workgroup */
         return;
     }
-    if (loader) {
-        Fin ff = fin_head(item(0));                /* item i - 1, biases too */
-        fin_bias(ff);
-        Fin fh = fin_head(item(min(1, n - 1)));    /* item i */
-        int code = item(min(2, n - 1));            /* item i + 1 */
-        for (int i = 0; i < n; i++) {
-            asm volatile("s_barrier" ::: "memory");   /* a finishing wave writes no LDS */
-            if (i > 0) {
-                finish(i - 1, ff);
-                ff = fh;
-                fin_bias(ff);
-                fh = fin_head(code);
-                code = item(min(i + 2, n - 1));
+    /* A run's operands are loaded when it starts, behind the slabs in flight.
+     * (Loading them three items earlier into registers of their own did not
+     * shorten the wait: their bytes only delay the slabs; two tiles leave no
+     * registers for it.) */
+    RgX cur;
+    Done done = {0, 0, 0, 0.f, 0.f};
+    int run = ldc(a.rg_run0, wg);   /* the run of item 0; the runs follow in order */
+    int slab = (item(0) >> 8) & 255;
+    for (int i = 0; i < n; run++, slab = 0) {
+        load_x(run, cur);
+        const int re = run_end(i);
+        const int *rc = a.rg_runs + (size_t)RING_REC * run;
+        const int pf = ldc(rc, 0), nv = ldc(rc, 1), e = ldc(rc, 2 + RING_P);
+        const Buf gb = make_buf(a.gbias ? (const void *)(uintptr_t)ldc(a.gbias, e) : nullptr, a.gbias ? (uint32_t)a.I * 4u : 0u);
+        const Buf ub = make_buf(a.ubias ? (const void *)(uintptr_t)ldc(a.ubias, e) : nullptr, a.ubias ? (uint32_t)a.I * 4u : 0u);
+        auto step = [&](auto tiles) __attribute__((always_inline)) {
+            for (; i < re; i++, slab++) {
+                bar_lds();   /* item i's slab has landed, item i - 1's sums are in LDS */
+                finish(i - 1, done);   /* nothing before the first item: no pairs */
+                done.pf = pf;
+                done.nv = nv;
+                done.r = 16 * slab;
+                if (a.gbias) {   /* both or neither */
+                    done.gb = __uint_as_float(ld4(gb, (uint32_t)(16 * slab + c16) * 4u));
+                    done.ub = __uint_as_float(ld4(ub, (uint32_t)(16 * slab + c16) * 4u));
+                }
+                compute(i, cur, tiles);
             }
-        }
-        asm volatile("s_barrier" ::: "memory");   /* item n - 1's sums are in LDS */
-        finish(n - 1, ff);
-        return;
-    }
-    /* A run's operands are loaded into a staging set while the run before is
-     * computed, three items before its end (ahead of the copies of the next
-     * run's first items, which they would otherwise wait behind), and taken
-     * as the values of an empty asm statement when the run starts: the
-     * compiler waits for the loads there and not at their uses, and the set
-     * in use never has loads in flight. */
-    auto settle = [&](RgX &x) __attribute__((always_inline)) {
-#pragma unroll
-        for (int h = 0; h < 2; h++)
-            asm volatile(""
-                         : "+v"(x.xb[h][0]), "+v"(x.xb[h][1]), "+v"(x.xb[h][2]), "+v"(x.xb[h][3]), "+v"(x.xb[h][4]),
-                           "+v"(x.xb[h][5]), "+v"(x.xb[h][6]), "+v"(x.xb[h][7]), "+v"(x.bs0[h]), "+v"(x.bs1[h]),
-                           "+v"(x.xd[h]));
-    };
-    /* the scale of each of the lane's four result pairs, shuffled once a run */
-    auto prep = [&](RgX &x) __attribute__((always_inline)) {
-#pragma unroll
-        for (int h = 0; h < 2; h++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) x.xdv[h][v] = __uint_as_float(__shfl(x.xd[h], 4 * g + v, 64));
-    };
-    RgX cur, stage;
-    int run = ldc(a.rg_run0, blockIdx.x);   /* the run of item 0; the runs follow in order */
-    load_x(run, cur);
-    settle(cur);
-    prep(cur);
-    int re = run_end(0);
-    for (int i = 0; i < n;) {
-        const int pf = max(i, re - 3);
-        for (; i < re; i++) {
-            if (i == pf && re < n) load_x(run + 1, stage);
-            bar_lds();   /* item i's slab has landed, item i - 1's sums are read */
-            compute(i, cur);
-        }
-        if (i < n) {
-            re = run_end(i);
-            settle(stage);
-            cur = stage;
-            prep(cur);
-            run++;
-        }
+        };
+        if (cur.nt == 1) step(std::integral_constant<int, 1>());
+        else step(std::integral_constant<int, 2>());
     }
     bar_lds();   /* item n - 1's sums are in LDS */
+    finish(n - 1, done);
 }
 
 /* Phase B: part[p][r] = w_p * (down_r . hq_p + bd[r]) for the 64 rows r of
@@ -747,17 +806,19 @@ __global__ __launch_bounds__(NT) void k_moe_qb(MoeArgs a) {
 
 /* Phase B, persistent, for Q6_K down rows of I = 768 (3 blocks, 630 bytes
  * a row) without a down bias: one workgroup a compute unit walks its list
- * of items (active expert, 32-row slab, pass of 16 pairs), the slabs
- * (20,160 contiguous bytes) streaming through a ring of six LDS slots five
+ * of items (active expert, 32-row slab, pass of up to 32 pairs), the slabs
+ * (20,160 contiguous bytes) streaming through a ring of five LDS slots four
  * items ahead, as the gate/up ring does.  Twelve compute waves take one
  * 128-value half-block of one 16-row tile each (wave c: half-block c % 6,
  * block c % 6 / 2, tile c / 6; three a SIMD), with k_moe_qb's arithmetic,
  * and leave each
  * half-block's term d x d_x x (sum - 32 x offsets) in LDS.  Two copy waves
  * issue the slab copies and wait for them with exact counts (they issue no
- * other memory operation, which would enter the counts); two finishing
- * waves finish the previous item: the six terms added in half-block order
- * (k_moe_qb's order), times the pair's weight.  The slab
+ * other memory operation, which would enter the counts).  The compute waves
+ * also finish the previous item: the six terms added in half-block order
+ * (k_moe_qb's order), times the pair's weight (two finishing waves took as
+ * long as an item's copies and products: 103 -> 86 us at 509 tokens with
+ * their work left out).  The slab
  * keeps the matrix's layout in LDS (the copies read 16-byte-aligned sources
  * only), so fields of odd rows and odd blocks lie at 2 mod 4 and are read
  * as covering dwords, shifted. */
@@ -767,44 +828,50 @@ constexpr int DR_ROWS = 32;
 constexpr int DR_SLAB = DR_ROWS * DR_RB;                  /* 20,160 bytes */
 constexpr int DR_COPIES = (DR_SLAB + 1023) / 1024;        /* 20 copies, the last of DR_LAST lanes */
 constexpr int DR_LAST = (DR_SLAB - 1024 * (DR_COPIES - 1)) / 16;
-constexpr int DR_SLOTS = 6;
+constexpr int DR_SLOTS = 5;
 constexpr int DR_HB = 2 * DR_NB;                        /* half-blocks of a row */
-constexpr int DR_CW = 2 * DR_HB, DR_YW = 2, DR_FW = 2;  /* compute, copy and finishing waves */
+constexpr int DR_CW = 2 * DR_HB, DR_YW = 2;             /* compute and copy waves */
 constexpr int DR_LC = DR_COPIES / DR_YW;                  /* copies a copy wave issues per item */
-constexpr int DR_NT = 64 * (DR_CW + DR_YW + DR_FW);
-constexpr int DR_FO = 2 * 16 * 16 / (64 * DR_FW);         /* (pair, row) results a finishing thread writes */
+constexpr int DR_NT = 64 * (DR_CW + DR_YW);
 static_assert(DR_SLAB % 16 == 0 && DR_LAST > 0 && DR_LAST <= 64, "whole 16-byte pieces");
 static_assert(DR_COPIES % DR_YW == 0, "equal copy counts per copy wave");
 static_assert((DR_SLOTS - 2) * DR_LC <= 63, "a vmcnt count");
 
-/* 8 bytes at LDS offset o (o even) of base: the covering dwords, shifted */
-__device__ inline u32x2 dr_ld8(const uint8_t *base, uint32_t o) {
+/* 8 bytes at LDS offset o (o even) of base: the covering dwords, then the
+ * bytes shifted out of them (o and `at` alike mod 4) */
+struct Dr8 {
+    uint32_t d0, d1, d2;
+};
+__device__ inline Dr8 dr_read8(const uint8_t *base, uint32_t o) {
     const uint32_t *p = (const uint32_t *)(base + (o & ~3u));
-    const uint32_t sh = o & 3u;
-    const uint32_t d0 = p[0], d1 = p[1], d2 = p[2];
-    return u32x2{__builtin_amdgcn_alignbyte(d1, d0, sh), __builtin_amdgcn_alignbyte(d2, d1, sh)};
+    return Dr8{p[0], p[1], p[2]};
+}
+__device__ inline u32x2 dr_shift8(const Dr8 &d, uint32_t at) {
+    return u32x2{__builtin_amdgcn_alignbyte(d.d1, d.d0, at & 3u), __builtin_amdgcn_alignbyte(d.d2, d.d1, at & 3u)};
 }
 
-struct DrX {   /* a compute lane's q8 operands of one run: pair c16, its wave's half-block */
-    long x0[4], x1[4];   /* K slice 8 g of chunk m, zero in the half of K the other sub-block takes */
-    float s16a, s16b, xd;
-    float xdv[4];        /* the scales of pairs 4 g .. 4 g + 3, set once the run starts */
+struct DrX {   /* a compute lane's q8 operands of one run: pair c16 of each tile, its wave's half-block */
+    long xb[RING_T][4];   /* K slice 8 g of chunk m */
+    float s16a[RING_T], s16b[RING_T], xd[RING_T];
+    int nt;                              /* tiles that hold pairs */
 };
 
 __global__ __launch_bounds__(DR_NT) void k_moe_qb_ring(MoeArgs a) {
     __shared__ __attribute__((aligned(16))) uint8_t ring[DR_SLOTS][DR_SLAB];
-    __shared__ __attribute__((aligned(16))) float red[2][DR_HB][2][4][64];   /* by item parity */
-    __shared__ float pwl[DR_FW][16];                                          /* a finishing wave's pair weights */
+    __shared__ __attribute__((aligned(16))) float red[2][RING_T][DR_HB][2][4][64];   /* by item parity */
+    __shared__ __attribute__((aligned(16))) float xdl[DR_CW][RING_T][16];            /* the run's q8 scales */
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4,
               c16 = lane & 15;
-    const bool loader = w >= DR_CW, copier = loader && w < DR_CW + DR_YW;
-    const int i0 = ldc(a.rb_off, blockIdx.x), n = ldc(a.rb_off, blockIdx.x + 1) - i0;
+    const bool copier = w >= DR_CW;
+    const int wg = ring_wg();
+    const int i0 = ldc(a.rb_off, wg), n = ldc(a.rb_off, wg + 1) - i0;
     if (n <= 0) return;   /* uniform */
     const uint32_t mbytes = (uint32_t)a.D * DR_RB;
     const Q8Rows &q = a.hq;
     const Buf qs_b = make_buf(q.qs, (uint32_t)((size_t)a.P * DR_NB * 256));
     const Buf s16_b = make_buf(q.s16, (uint32_t)((size_t)a.P * DR_NB * 64));
     const Buf d_b = make_buf(q.d, (uint32_t)((size_t)a.P * DR_NB * 4));
+    const Buf pw_b = make_buf(a.p_w, (uint32_t)a.P * 4u);
     const int hbw = w % DR_HB, bi = hbw >> 1, h = hbw & 1, tw = w / DR_HB;   /* a compute wave's half-block, tile */
 
     auto item = [&](int j) { return ldc(a.rb_items, (size_t)(i0 + j)); };
@@ -824,22 +891,6 @@ __global__ __launch_bounds__(DR_NT) void k_moe_qb_ring(MoeArgs a) {
         f.s = (it >> 8) & 255;
         return f;
     };
-    struct Fin {   /* a finishing wave's: slab, pairs and their weights */
-        int s, tp, p0, np;
-        float pw[16];
-    };
-    auto fin_head = [&](int it) __attribute__((always_inline)) {
-        Fin f;
-        f.s = (it >> 8) & 255;
-        f.tp = 16 * (it & 255);
-        f.p0 = ldc(&a.ed[it >> 16].p0, 0);
-        f.np = ldc(&a.ed[it >> 16].np, 0);
-        return f;
-    };
-    auto fin_pw = [&](Fin &f) __attribute__((always_inline)) {
-#pragma unroll
-        for (int v = 0; v < 16; v++) f.pw[v] = ldc(a.p_w, (size_t)min(f.p0 + f.tp + v, a.P - 1));
-    };
     /* the copy wave's share of item j's copies */
     auto issue_copies = [&](int j, const Info &f) __attribute__((always_inline)) {
         const u32x4 desc = buf_desc((const void *)(uintptr_t)f.base, mbytes);
@@ -852,95 +903,115 @@ __global__ __launch_bounds__(DR_NT) void k_moe_qb_ring(MoeArgs a) {
         }
     };
     auto wait_copies_behind = [&](int k) __attribute__((always_inline)) {
-        if (k >= 4) wait_copies_but<4 * DR_LC>();
-        else if (k == 3) wait_copies_but<3 * DR_LC>();
+        if (k >= 3) wait_copies_but<3 * DR_LC>();
         else if (k == 2) wait_copies_but<2 * DR_LC>();
         else if (k == 1) wait_copies_but<DR_LC>();
         else wait_copies_but<0>();
     };
-    static_assert(DR_SLOTS - 2 == 4, "wait_copies_behind covers the items in flight");
-    /* the compute lane's operands of run r: its pair c16 (the run's first
-     * pair and count from its record, one round trip of scalar loads) */
+    static_assert(DR_SLOTS - 2 == 3, "wait_copies_behind covers the items in flight");
+    /* the compute lane's operands of run r: its pair c16 of each tile (the
+     * run's first pair and count from its record) */
     auto load_x = [&](int r, DrX &x) __attribute__((always_inline)) {
         const int *rc = a.rb_runs + (size_t)RING_REC * r;
         const int pf = ldc(rc, 0), nv = ldc(rc, 1);
-        const bool pv = c16 < nv;
-        const uint32_t qb = (uint32_t)(pf + c16) * DR_NB + (uint32_t)bi;
+        x.nt = nv > 16 ? 2 : 1;
+#pragma unroll
+        for (int t = 0; t < RING_T; t++) {
+            if (t >= x.nt) break;   /* uniform */
+            const bool pv = 16 * t + c16 < nv;
+            const uint32_t qb = (uint32_t)(pf + 16 * t + c16) * DR_NB + (uint32_t)bi;
+            const uint32_t oq = pv ? qb * 256u + 128u * h + 8u * g : OOB, os = pv ? qb * 64u + 32u * h + 4u * g : OOB;
+#pragma unroll
+            for (int m = 0; m < 4; m++) x.xb[t][m] = as_long(ld8(qs_b, oq + 32u * m));
+            x.s16a[t] = (float)(int)ld4(s16_b, os);
+            x.s16b[t] = (float)(int)ld4(s16_b, os + 16u);
+            x.xd[t] = __uint_as_float(ld4(d_b, pv ? qb * 4u : OOB));
+        }
+    };
+    /* compute item j from its slot: the wave's half-block of its row tile
+     * against NT tiles of pairs, the codes unpacked once for all of them */
+    auto compute = [&](int j, const DrX &x, auto tiles) __attribute__((always_inline)) {
+        constexpr int NT_ = decltype(tiles)::value;
+        const uint8_t *sb = &ring[j % DR_SLOTS][0];
+        const uint32_t lo = g < 2 ? ~0u : 0u;
+        const uint32_t rb = (uint32_t)(16 * tw + c16) * DR_RB + (uint32_t)bi * Q6B;   /* row c16's block */
+        /* every LDS read of the item first */
+        const Dr8 r0 = dr_read8(sb, rb + 64u * h + 8u * g), r1 = dr_read8(sb, rb + 64u * h + 32u + 8u * g);
+        const Dr8 r2 = dr_read8(sb, rb + 128u + 32u * h + 8u * g), r3 = dr_read8(sb, rb + 192u + 8u * h);
+        const uint32_t dw = *(const uint32_t *)(sb + ((rb + 208u) & ~3u));
+        __builtin_amdgcn_sched_barrier(0);
+        const u32x2 ql0 = dr_shift8(r0, rb), ql1 = dr_shift8(r1, rb), qh = dr_shift8(r2, rb), scr = dr_shift8(r3, rb);
+        const float dv = ref_f16((rb & 2u) ? (dw >> 16) : (dw & 0xFFFFu));
+        const float sa = (float)(int8_t)(scr.x >> (8 * g)), sb4 = (float)(int8_t)(scr.y >> (8 * g));
+        v4f cf[NT_];
+        int ai[NT_][4];
+#pragma unroll
+        for (int t = 0; t < NT_; t++) {
+            cf[t] = v4f{0.f, 0.f, 0.f, 0.f};
+            cf[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.s16a[t], sa, cf[t], 0, 0, 0);
+            cf[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.s16b[t], sb4, cf[t], 0, 0, 0);
+#pragma unroll
+            for (int v = 0; v < 4; v++) ai[t][v] = 0;
+        }
 #pragma unroll
         for (int m = 0; m < 4; m++) {
-            const long xb = as_long(ld8(qs_b, pv ? qb * 256u + 128u * h + 32u * m + 8u * g : OOB));
-            x.x0[m] = g < 2 ? xb : 0l;
-            x.x1[m] = g < 2 ? 0l : xb;
-        }
-        x.s16a = (float)(int)ld4(s16_b, pv ? qb * 64u + 32u * h + 4u * g : OOB);
-        x.s16b = (float)(int)ld4(s16_b, pv ? qb * 64u + 32u * h + 16u + 4u * g : OOB);
-        x.xd = __uint_as_float(ld4(d_b, pv ? qb * 4u : OOB));
-    };
-    /* compute item j from its slot: the wave's half-block of its tile */
-    auto compute = [&](int j, const DrX &x) __attribute__((always_inline)) {
-        const uint8_t *sb = &ring[j % DR_SLOTS][0];
-        const float *xdv = x.xdv;
-        {
-            const int tq = tw;
-            const uint32_t rb = (uint32_t)(16 * tq + c16) * DR_RB + (uint32_t)bi * Q6B;   /* row c16's block */
-            const u32x2 ql0 = dr_ld8(sb, rb + 64u * h + 8u * g);
-            const u32x2 ql1 = dr_ld8(sb, rb + 64u * h + 32u + 8u * g);
-            const u32x2 qh = dr_ld8(sb, rb + 128u + 32u * h + 8u * g);
-            const u32x2 scr = dr_ld8(sb, rb + 192u + 8u * h);
-            const uint32_t dw = *(const uint32_t *)(sb + ((rb + 208u) & ~3u));
-            const float dv = ref_f16((rb & 2u) ? (dw >> 16) : (dw & 0xFFFFu));
-            v4f cf = {0.f, 0.f, 0.f, 0.f};
-            cf = __builtin_amdgcn_mfma_f32_16x16x4f32(x.s16a, (float)(int8_t)(scr.x >> (8 * g)), cf, 0, 0, 0);
-            cf = __builtin_amdgcn_mfma_f32_16x16x4f32(x.s16b, (float)(int8_t)(scr.y >> (8 * g)), cf, 0, 0, 0);
-            int ai[4] = {0, 0, 0, 0};
+            const u32x2 ql = (m & 1) ? ql1 : ql0;
+            const int sl = 4 * (m >> 1), sh = 2 * m;
+            u32x2 c;
+            c.x = ((ql.x >> sl) & 0x0F0F0F0Fu) | (((qh.x >> sh) & 0x03030303u) << 4);
+            c.y = ((ql.y >> sl) & 0x0F0F0F0Fu) | (((qh.y >> sh) & 0x03030303u) << 4);
+            /* K slots 0-15 (lane groups 0, 1) are sub-block 2 m, 16-31
+             * sub-block 2 m + 1: the codes are zeroed in one half of K */
+            const u32x2 c0 = {c.x & lo, c.y & lo}, c1 = {c.x & ~lo, c.y & ~lo};
+            const uint32_t sw = m < 2 ? scr.x : scr.y;
+            const int sc0 = (int)(int8_t)(sw >> (16 * (m & 1))), sc1 = (int)(int8_t)(sw >> (16 * (m & 1) + 8));
+            if (NT_ > 1) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int m = 0; m < 4; m++) {
-                const u32x2 ql = (m & 1) ? ql1 : ql0;
-                const int sl = 4 * (m >> 1), sh = 2 * m;
-                u32x2 c;
-                c.x = ((ql.x >> sl) & 0x0F0F0F0Fu) | (((qh.x >> sh) & 0x03030303u) << 4);
-                c.y = ((ql.y >> sl) & 0x0F0F0F0Fu) | (((qh.y >> sh) & 0x03030303u) << 4);
-                const v4i d0 = mma(x.x0[m], as_long(c)), d1 = mma(x.x1[m], as_long(c));
-                const uint32_t sw = m < 2 ? scr.x : scr.y;
-                const int sc0 = (int)(int8_t)(sw >> (16 * (m & 1))), sc1 = (int)(int8_t)(sw >> (16 * (m & 1) + 8));
+            for (int t = 0; t < NT_; t++) {
+                const v4i d0 = mma(x.xb[t][m], as_long(c0)), d1 = mma(x.xb[t][m], as_long(c1));
 #pragma unroll
-                for (int v = 0; v < 4; v++) ai[v] += __mul24(sc0, d0[v]) + __mul24(sc1, d1[v]);   /* |.| < 2^24 */
+                for (int v = 0; v < 4; v++) ai[t][v] += __mul24(sc0, d0[v]) + __mul24(sc1, d1[v]);   /* |.| < 2^24 */
             }
+        }
 #pragma unroll
-            for (int v = 0; v < 4; v++) red[j & 1][hbw][tq][v][lane] = dv * xdv[v] * (float)(ai[v] - 32 * (int)cf[v]);
+        for (int t = 0; t < NT_; t++) {
+            const v4f xdv = *(const v4f *)&xdl[w][t][4 * g];   /* of pairs 4 g .. 4 g + 3 */
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                red[j & 1][t][hbw][tw][v][lane] = dv * xdv[v] * (float)(ai[t][v] - 32 * (int)cf[t][v]);
         }
     };
-    /* the finishing threads, DR_FO (pair, row) results each: the six
-     * half-block terms in order, times the pair's weight; the term of pair
-     * 4 g + v and row c16 of tile tq sits in lane 16 g + c16, register v */
-    auto finish = [&](int j, const Fin &fi) __attribute__((always_inline)) {
-        /* the weights (scalars) through the wave's own LDS words: a per-lane
-         * select among them became a lookup through scratch memory */
-        float *pl = pwl[w - DR_CW - DR_YW];
-        if (lane == 0) {
+    /* finishing item j: a compute lane takes one or two (pair, row) results
+     * o = tid and tid + 64 DR_CW of the slab (tile of pairs o / 512, row tile
+     * o / 256 % 2, pair o / 16 % 16, row o % 16): the six half-block terms in
+     * order, times the pair's weight; the term of pair 4 g + v and row c16
+     * sits in lane 16 g + c16, register v */
+    struct Done {   /* the item to finish: its first pair, pairs from there, first row, the lane's pair weights */
+        int pf, nv, r;
+        float pw[2];
+    };
+    auto out_pair = [&](int u) { return 16 * ((tid + 64 * DR_CW * u) >> 9) + (((tid + 64 * DR_CW * u) >> 4) & 15); };
+    auto finish = [&](int j, const Done &f) __attribute__((always_inline)) {
 #pragma unroll
-            for (int v = 0; v < 16; v++) pl[v] = fi.pw[v];
-        }
-        const int f = tid - 64 * (DR_CW + DR_YW);
+        for (int u = 0; u < 2; u++) {
+            const int ow = w + DR_CW * u;   /* o / 64, uniform */
+            if (ow >= 8 * RING_T || 16 * (ow >> 3) >= f.nv) break;
+            int lx = lane;
+            asm volatile("" : "+v"(lx));   /* what follows of it is computed here, not kept in registers */
+            const int t = ow >> 3, tq = (ow >> 2) & 1, v = lx >> 4, c16 = lx & 15, jj = 4 * (ow & 3) + v;
+            const int ln = 16 * (ow & 3) + c16;
+            float acc = 0.f;
 #pragma unroll
-        for (int u = 0; u < DR_FO; u++) {
-            const int o = f + 64 * DR_FW * u, tq = o >> 8, jj = (o >> 4) & 15, rr = o & 15;
-            const int ln = 16 * (jj >> 2) + rr, v = jj & 3;
-            if (fi.tp + jj < fi.np) {
-                float acc = 0.f;
-#pragma unroll
-                for (int c = 0; c < DR_HB; c++) acc += red[j & 1][c][tq][v][ln];
-                const int r = DR_ROWS * fi.s + 16 * tq + rr;
-                a.part[(size_t)(fi.p0 + fi.tp + jj) * a.D + r] = pl[jj] * (acc + 0.f);
-            }
+            for (int c = 0; c < DR_HB; c++) acc += red[j & 1][t][c][tq][v][ln];
+            if (16 * t + jj < f.nv) a.part[(size_t)(f.pf + 16 * t + jj) * a.D + f.r + 16 * tq + c16] = f.pw[u] * (acc + 0.f);
         }
     };
     auto run_end = [&](int s0) { return min(ldc(a.rb_rend, (size_t)(i0 + s0)), i0 + n) - i0; };
 
     /* as in the gate/up ring: between the barriers of items i and i + 1 the
-     * compute waves compute item i (slot i % DR_SLOTS, red[i % 2]) while the
-     * copy waves copy item i + DR_SLOTS - 1 into item i - 1's slot and the
-     * finishing waves finish item i - 1 (red[(i - 1) % 2]) */
+     * compute waves finish item i - 1 (red[(i - 1) % 2]) and compute item i
+     * (slot i % DR_SLOTS, red[i % 2]) while the copy waves copy item
+     * i + DR_SLOTS - 1 into item i - 1's slot */
     if (copier) {
         for (int j = 0; j < DR_SLOTS - 1 && j < n; j++) issue_copies(j, info_code(item(j)));
         Info fc = info_code(item(min(DR_SLOTS - 1, n - 1)));   /* item i + DR_SLOTS - 1 */
@@ -956,56 +1027,45 @@ __global__ __launch_bounds__(DR_NT) void k_moe_qb_ring(MoeArgs a) {
         wait_copies();   /* no copy outlives the workgroup */
         return;
     }
-    if (loader) {
-        Fin ff = fin_head(item(0));                /* item i - 1, weights too */
-        fin_pw(ff);
-        Fin fh = fin_head(item(min(1, n - 1)));    /* item i */
-        int code = item(min(2, n - 1));            /* item i + 1 */
-        for (int i = 0; i < n; i++) {
-            bar_lds();   /* its own weight words are written and read in order */
-            if (i > 0) {
-                finish(i - 1, ff);
-                ff = fh;
-                fin_pw(ff);
-                fh = fin_head(code);
-                code = item(min(i + 2, n - 1));
-            }
-        }
-        bar_lds();   /* item n - 1's terms are in LDS */
-        finish(n - 1, ff);
-        return;
-    }
     auto settle = [&](DrX &x) __attribute__((always_inline)) {
-        asm volatile(""
-                     : "+v"(x.x0[0]), "+v"(x.x0[1]), "+v"(x.x0[2]), "+v"(x.x0[3]), "+v"(x.x1[0]), "+v"(x.x1[1]),
-                       "+v"(x.x1[2]), "+v"(x.x1[3]), "+v"(x.s16a), "+v"(x.s16b), "+v"(x.xd));
-    };
-    auto prep = [&](DrX &x) __attribute__((always_inline)) {
 #pragma unroll
-        for (int v = 0; v < 4; v++) x.xdv[v] = __shfl(x.xd, 4 * g + v, 64);
+        for (int t = 0; t < RING_T; t++) {
+            if (t >= x.nt) break;
+            long(&xb)[4] = x.xb[t];
+            asm volatile(""
+                         : "+v"(xb[0]), "+v"(xb[1]), "+v"(xb[2]), "+v"(xb[3]), "+v"(x.s16a[t]), "+v"(x.s16b[t]),
+                           "+v"(x.xd[t]));
+            xdl[w][t][c16] = x.xd[t];   /* the wave's own words, in order */
+        }
     };
-    DrX cur, stage;
-    int run = ldc(a.rb_run0, blockIdx.x);   /* the run of item 0; the runs follow in order */
-    load_x(run, cur);
-    settle(cur);
-    prep(cur);
-    int re = run_end(0);
-    for (int i = 0; i < n;) {
-        const int pf = max(i, re - (DR_SLOTS - 1));
-        for (; i < re; i++) {
-            if (i == pf && re < n) load_x(run + 1, stage);
-            bar_lds();   /* item i's slab has landed, item i - 1's terms are read */
-            compute(i, cur);
-        }
-        if (i < n) {
-            re = run_end(i);
-            settle(stage);
-            cur = stage;
-            prep(cur);
-            run++;
-        }
+    DrX cur;
+    Done done = {0, 0, 0, {0.f, 0.f}};
+    int run = ldc(a.rb_run0, wg);   /* the run of item 0; the runs follow in order */
+    int slab = (item(0) >> 8) & 255;
+    for (int i = 0; i < n; run++, slab = 0) {
+        load_x(run, cur);
+        const int re = run_end(i);
+        const int *rc = a.rb_runs + (size_t)RING_REC * run;
+        const int pf = ldc(rc, 0), nv = ldc(rc, 1);
+        float pw[2];
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+            pw[u] = __uint_as_float(ld4(pw_b, out_pair(u) < nv ? (uint32_t)(pf + out_pair(u)) * 4u : OOB));
+        settle(cur);
+        asm volatile("" : "+v"(pw[0]), "+v"(pw[1]));
+        auto step = [&](auto tiles) __attribute__((always_inline)) {
+            for (; i < re; i++, slab++) {
+                bar_lds();   /* item i's slab has landed, item i - 1's terms are in LDS */
+                finish(i - 1, done);   /* nothing before the first item: no pairs */
+                done = Done{pf, nv, DR_ROWS * slab, {pw[0], pw[1]}};
+                compute(i, cur, tiles);
+            }
+        };
+        if (cur.nt == 1) step(std::integral_constant<int, 1>());
+        else step(std::integral_constant<int, 2>());
     }
     bar_lds();   /* item n - 1's terms are in LDS */
+    finish(n - 1, done);
 }
 
 bool qb_ring_shape(int I, int D) { return I == DR_NB * 256 && D % DR_ROWS == 0 && D / DR_ROWS <= 256; }
@@ -1041,28 +1101,63 @@ bool qa_ring_shape(int gate_fmt, int D, int I) { return gate_fmt == TG_FMT_Q4K &
  * pair, pair count, the input rows of its first 16 pairs) in list order and
  * run0[w] the run of workgroup w's first item, so a compute wave reaches a
  * run's operands with one round trip of scalar loads. */
-void ring_items(const ExpDesc *ed, int n_act, int slabs, int G, const int *p_row, int P, RingLists &r) {
+void ring_items(const ExpDesc *ed, int n_act, int slabs, int G, const int *p_row, int P, const RingCost &c,
+                RingLists &r) {
     r.items.clear();
     r.rend.clear();
     r.runs.clear();
-    std::vector<int> run_of;
     for (int ei = 0; ei < n_act; ei++)
-        for (int t = 0; t < std::max(1, (ed[ei].np + 15) / 16); t++) {
-            const int run = (int)(r.runs.size() / RING_REC), pf = ed[ei].p0 + 16 * t;
+        for (int t = 0; t < std::max(1, (ed[ei].np + RING_P - 1) / RING_P); t++) {
+            const int run = (int)(r.runs.size() / RING_REC), pf = ed[ei].p0 + RING_P * t;
             r.runs.push_back(pf);
-            r.runs.push_back(ed[ei].np - 16 * t);
-            for (int j = 0; j < 16; j++) r.runs.push_back(p_row[std::min(pf + j, P - 1)]);
+            r.runs.push_back(ed[ei].np - RING_P * t);
+            for (int j = 0; j < RING_P; j++) r.runs.push_back(p_row[std::min(pf + j, P - 1)]);
+            r.runs.push_back(ed[ei].e);
             r.runs.resize((size_t)(run + 1) * RING_REC, 0);
             for (int s = 0; s < slabs; s++) r.items.push_back(ei << 16 | s << 8 | t);
             r.rend.resize(r.items.size(), (int)r.items.size());
-            run_of.resize(r.items.size(), run);
         }
-    r.off.resize(G + 1);
-    r.run0.resize(G + 1);
-    for (int w = 0; w <= G; w++) {
-        r.off[w] = (int)((int64_t)r.items.size() * w / G);
-        r.run0[w] = r.off[w] < (int)run_of.size() ? run_of[r.off[w]] : 0;
+    /* The cut: the smallest time T (found to 1 %) in which G workgroups get
+     * through the list in order, each taking items while they fit.  A run
+     * costs its start (its operands) in every workgroup that touches it. */
+    const int runs = (int)(r.runs.size() / RING_REC);
+    auto two = [&](int run) { return r.runs[(size_t)RING_REC * run + 1] > 16; };
+    auto cut = [&](int64_t T, bool write) {
+        int w = -1;
+        int64_t room = 0;
+        for (int run = 0; run < runs; run++) {
+            const int64_t start = two(run) ? c.start2 : c.start1, each = two(run) ? c.item2 : c.item1;
+            for (int left = slabs; left > 0;) {
+                if (room < start + each) {
+                    if (++w == G) return false;
+                    room = T;
+                    if (write) {
+                        r.off[w] = run * slabs + slabs - left;
+                        r.run0[w] = run;
+                    }
+                }
+                const int take = (int)std::min<int64_t>(left, (room - start) / each);
+                room -= start + take * each;
+                left -= take;
+            }
+        }
+        return true;
+    };
+    int64_t lo = std::max(c.start1 + c.item1, c.start2 + c.item2), all = 0;
+    for (int run = 0; run < runs; run++) all += two(run) ? c.start2 + slabs * c.item2 : c.start1 + slabs * c.item1;
+    lo = std::max(lo, all / G);   /* cut(lo - 1) fails */
+    int64_t hi = lo;
+    while (!cut(hi, false)) {
+        lo = hi;
+        hi += hi / 4;
     }
+    while (hi - lo > hi / 100 + 1) {
+        const int64_t mid = (lo + hi) / 2;
+        (cut(mid, false) ? hi : lo) = mid;
+    }
+    r.off.assign(G + 1, (int)r.items.size());
+    r.run0.assign(G + 1, 0);
+    cut(hi, true);
 }
 
 void launch_moe_a_qk(const MoeArgs &a, hipStream_t st) {

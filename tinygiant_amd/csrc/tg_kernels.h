@@ -131,7 +131,7 @@ int grouped_min_rows();
  * shape, 17 where both persistent rings run, 40 elsewhere) */
 bool qk_grouped_fits(const MoeArgs &a);
 /* The persistent int8 MFMA gate/up phase (Q4_K, D = 2048): its items, (index
- * ei into the busiest-first active experts, 16-row slab s, pass t of 16
+ * ei into the busiest-first active experts, 16-row slab s, pass t of RING_P
  * pairs) as ei << 16 | s << 8 | t, and off[0 .. G] the range of each of G
  * workgroups.  False when the shape is not the phase's. */
 bool qa_ring_shape(int gate_fmt, int D, int I);
@@ -139,14 +139,26 @@ bool qb_ring_shape(int I, int D);
 /* The persistent phases' items (expert, pass, slab of `slabs`) cut into G
  * workgroup ranges (off), the end of each item's run (rend: the items of one
  * expert and pass), the runs' records (RING_REC ints each: the run's first
- * pair p0 + 16 t, the pairs from there on, np - 16 t, possibly more than 16,
- * and the input rows of its first 16 pairs, the last pair's row past the
- * end) and the run of each workgroup's first item (run0). */
-constexpr int RING_REC = 20;
+ * pair p0 + RING_P t, the pairs from there on, possibly more than RING_P,
+ * the input rows of its first RING_P pairs, the last pair's row past the
+ * end, and the expert) and the run of each workgroup's first item (run0). */
+constexpr int RING_T = 2, RING_P = 16 * RING_T;   /* tiles of 16 pairs a pass, pairs a pass */
+constexpr int RING_REC = 2 + RING_P + 2;   /* padded */
 struct RingLists {
     std::vector<int> items, off, rend, runs, run0;
 };
-void ring_items(const ExpDesc *ed, int n_act, int slabs, int G, const int *p_row, int P, RingLists &r);
+/* nanoseconds of a workgroup's run start and item, for runs of one tile of
+ * pairs and of two: device timestamps at 128 and 509 tokens (gate/up: starts
+ * of 1.9 to 5 us, items of 1.6 and 2.3), the starts of two tiles and the down
+ * phase's figures then fitted to the layer's time.  An equal number of items
+ * a workgroup took 101 against 72 us at 33 tokens, 150 against 110 at 128. */
+struct RingCost {
+    int start1, item1, start2, item2;
+};
+constexpr RingCost QA_RING_COST = {2500, 1600, 6500, 2300}, QB_RING_COST = {2000, 1450, 5500, 2200};
+constexpr int RING_MAX_ROWS = 256 * RING_P;   /* an item holds its pass in 8 bits */
+void ring_items(const ExpDesc *ed, int n_act, int slabs, int G, const int *p_row, int P, const RingCost &c,
+                RingLists &r);
 constexpr int QA_RING_MAX_G = 1024;
 void launch_moe_a_qk(const MoeArgs &a, hipStream_t st);
 void launch_moe_b_qk(const MoeArgs &a, hipStream_t st);
