@@ -149,3 +149,27 @@ def test_grouped_run_to_run_identical(tg):
         b = tg.moe_forward_rows_v2(g, u, d, O.FMT_MXFP4, [O.FMT_MXFP4] * n, None, None, None, O.ACT_SILU, rw, x,
                                    np.zeros((48, D), np.float32), I)
     assert a.tobytes() == b.tobytes()
+
+
+@pytest.mark.parametrize("D,I,k,n", [
+    (32, 96, 17, 2),       # one block a row: three of the four waves of a half idle; a pass of 16 and one of 1
+    (2880, 160, 16, 3),    # the longest row of the persistent phases; the down phase's last group partly past its row
+    (160, 2880, 33, 2),    # three passes
+    (2912, 2944, 5, 2),    # one block past the longest row: k_moe_mx in both phases
+    (64, 4128, 6, 2),      # more item rows than an item's code holds in the gate/up phase, not in the down phase
+    (1184, 1344, 40, 5),   # 37 and 42 blocks: partial groups in a wave's range
+])
+def test_grouped_ring_edges(tg, orc, D, I, k, n):
+    """The persistent phases at the edges of their rows, groups and passes:
+    each expert takes its own share of the rows, so the passes hold 1 to 16
+    pairs.  Bars as above: the same exact block sums, f32 additions in another
+    order."""
+    rng = np.random.default_rng(D + I + k)
+    rw = rng.uniform(0.1, 1.0, (n, k)).astype(np.float32) / n
+    for e in range(1, n):
+        rw[e, rng.permutation(k)[:k * e // n]] = 0
+    x = rng.standard_normal((k, D)).astype(np.float32)
+    base = rng.standard_normal((k, D)).astype(np.float32)
+    say(f"ring edges: D={D} I={I} k={k}")
+    with _grouped_rows(tg, 1):
+        _check_moe(tg, orc, n, k, D, I, O.FMT_MXFP4, [O.FMT_MXFP4] * n, O.ACT_GPTOSS, True, rw, x, base)

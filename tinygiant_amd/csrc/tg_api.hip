@@ -429,6 +429,13 @@ static int cu_count() {
 /* row-tile tickets of the fused combine: at most one per 4 rows of D */
 static int moe_ctr_words(int D) { return D / 4 + 16; }
 
+static int ceil_div(int a, int b) { return (a + b - 1) / b; }
+
+/* every active expert's down matrix is MXFP4, in the persistent phase's shape */
+static bool mx_down_ring(const HostPlan &h) {
+    return h.fmts_present.size() == 1 && h.fmts_present[0] == TG_FMT_MXFP4 && mx_ring_shape(h.D, h.I, MX_RING_DOWN);
+}
+
 Layout plan_layout(const HostPlan &h) {
     Layout L;
     Bump b;
@@ -443,7 +450,13 @@ Layout plan_layout(const HostPlan &h) {
     if (qa_ring_shape(h.gate_fmt, h.D, h.I))  /* the persistent gate/up phase's items and ranges */
         t += 2 * (size_t)(h.I / 16) * (P / 16 + n + 1) * 4 + (size_t)RING_REC * (P / 16 + n + 1) * 4 +
              2 * (QA_RING_MAX_G + 1) * 4 + 64;
-    if (qb_ring_shape(h.I, h.D))  /* the persistent down phase's */
+    if (h.gate_fmt == TG_FMT_MXFP4 && mx_ring_shape(h.I, h.D, MX_RING_UP))
+        t += 2 * (size_t)ceil_div(h.I, MX_RING_UP) * (P / MX_RING_P + n + 1) * 4 +
+             (size_t)RING_REC * (P / MX_RING_P + n + 1) * 4 + 2 * (QA_RING_MAX_G + 1) * 4 + 64;
+    if (mx_down_ring(h))
+        t += 2 * (size_t)ceil_div(h.D, MX_RING_DOWN) * (P / MX_RING_P + n + 1) * 4 +
+             (size_t)RING_REC * (P / MX_RING_P + n + 1) * 4 + 2 * (QA_RING_MAX_G + 1) * 4 + 64;
+    else if (qb_ring_shape(h.I, h.D))  /* the persistent down phase's */
         t += 2 * (size_t)(h.D / 32) * (P / 16 + n + 1) * 4 + (size_t)RING_REC * (P / 16 + n + 1) * 4 +
              2 * (QA_RING_MAX_G + 1) * 4 + 64;
     L.tables_len = t + 64;
@@ -558,25 +571,32 @@ MoeArgs plan_args(const HostPlan &h, const Layout &L, uint8_t *dev, uint8_t *img
      * first instead of trailing the launch */
     std::stable_sort(ed.begin(), ed.end(), [](const ExpDesc &x, const ExpDesc &y) { return x.np > y.np; });
     a.ed = (const ExpDesc *)put(ed.data(), ed.size() * sizeof(ExpDesc));
-    if (qa_ring_shape(h.gate_fmt, h.D, h.I) && a.n_act_a > 0 && a.max_rows <= RING_MAX_ROWS) {
+    /* the persistent phases' lists */
+    auto ring = [&](int slabs, int pass_pairs, const RingCost &c, const int *&items, const int *&rend, const int *&runs,
+                    const int *&run0, const int *&off, int &n_wg) {
         RingLists r;
-        ring_items(ed.data(), a.n_act_a, h.I / 16, cu_count(), h.p_row.data(), P, QA_RING_COST, r);
-        a.rg_items = (const int *)put(r.items.data(), r.items.size() * 4);
-        a.rg_rend = (const int *)put(r.rend.data(), r.rend.size() * 4);
-        a.rg_runs = (const int *)put(r.runs.data(), r.runs.size() * 4);
-        a.rg_run0 = (const int *)put(r.run0.data(), r.run0.size() * 4);
-        a.rg_off = (const int *)put(r.off.data(), r.off.size() * 4);
-        a.rg_n = (int)r.off.size() - 1;
-    }
-    if (qb_ring_shape(h.I, h.D) && a.n_act_a > 0 && a.max_rows <= RING_MAX_ROWS) {
-        RingLists r;
-        ring_items(ed.data(), a.n_act_a, h.D / 32, cu_count(), h.p_row.data(), P, QB_RING_COST, r);
-        a.rb_items = (const int *)put(r.items.data(), r.items.size() * 4);
-        a.rb_rend = (const int *)put(r.rend.data(), r.rend.size() * 4);
-        a.rb_runs = (const int *)put(r.runs.data(), r.runs.size() * 4);
-        a.rb_run0 = (const int *)put(r.run0.data(), r.run0.size() * 4);
-        a.rb_off = (const int *)put(r.off.data(), r.off.size() * 4);
-        a.rb_n = (int)r.off.size() - 1;
+        ring_items(ed.data(), a.n_act_a, slabs, cu_count(), h.p_row.data(), P, pass_pairs, c, r);
+        items = (const int *)put(r.items.data(), r.items.size() * 4);
+        rend = (const int *)put(r.rend.data(), r.rend.size() * 4);
+        runs = (const int *)put(r.runs.data(), r.runs.size() * 4);
+        run0 = (const int *)put(r.run0.data(), r.run0.size() * 4);
+        off = (const int *)put(r.off.data(), r.off.size() * 4);
+        n_wg = (int)r.off.size() - 1;
+    };
+    const bool mx_up = h.gate_fmt == TG_FMT_MXFP4 && mx_ring_shape(h.I, h.D, MX_RING_UP), mx_down = mx_down_ring(h);
+    a.rg_mx = mx_up && a.max_rows <= MX_RING_MAX_ROWS;
+    a.rb_mx = mx_down && a.max_rows <= MX_RING_MAX_ROWS;
+    if (a.n_act_a > 0) {
+        if (a.rg_mx)
+            ring(ceil_div(h.I, MX_RING_UP), MX_RING_P, MX_COST, a.rg_items, a.rg_rend, a.rg_runs, a.rg_run0, a.rg_off,
+                 a.rg_n);
+        else if (qa_ring_shape(h.gate_fmt, h.D, h.I) && a.max_rows <= RING_MAX_ROWS)
+            ring(h.I / 16, RING_P, QA_RING_COST, a.rg_items, a.rg_rend, a.rg_runs, a.rg_run0, a.rg_off, a.rg_n);
+        if (a.rb_mx)
+            ring(ceil_div(h.D, MX_RING_DOWN), MX_RING_P, MX_COST, a.rb_items, a.rb_rend, a.rb_runs, a.rb_run0,
+                 a.rb_off, a.rb_n);
+        else if (!mx_down && qb_ring_shape(h.I, h.D) && a.max_rows <= RING_MAX_ROWS)
+            ring(h.D / 32, RING_P, QB_RING_COST, a.rb_items, a.rb_rend, a.rb_runs, a.rb_run0, a.rb_off, a.rb_n);
     }
     act_a.insert(act_a.end(), act_b.begin(), act_b.end());
     a.mx_act = (const int *)put(act_a.data(), act_a.size() * 4);

@@ -33,7 +33,9 @@
  * result each.
  * HBM sees each weight byte once however many pairs the expert holds; the
  * fp8 halves of a pass stay in registers from one item to the next of the
- * same expert.
+ * same expert.  Rows of up to 90 blocks take k_moe_mx_ring (slabs copied into
+ * an LDS ring), longer ones and layers whose experts' down formats differ
+ * k_moe_mx (slabs through registers).
  */
 #include <hip/hip_runtime.h>
 #include <math.h>
@@ -574,11 +576,271 @@ static void launch_mx(const MoeArgs &a, int cols, int nitems, hipStream_t st) {
     }
 }
 
+namespace {
+
+/* ---- persistent phases over rows of up to 90 blocks ----
+ *
+ * One workgroup a compute unit walks its list of items (ring_items: active
+ * expert, pass of up to 16 pairs, item rows), the slabs streaming through a
+ * ring of three LDS slots two items ahead of the item computed.  An item is
+ * 48 KiB, two halves of 16 rows: the gate and the up rows (phase A), or 32
+ * down rows (phase B).  Eight compute waves: wave c takes half c / 4 and a
+ * quarter of its rows' blocks, with the fp8 halves of the run's pairs for
+ * those blocks in registers (six groups of four blocks, 96 registers, loaded
+ * once a run); they also finish the previous item, one barrier an item.  Two
+ * copy waves issue the direct-to-LDS copies, one half each, and nothing else,
+ * so they wait for their own with exact counts.
+ *
+ * Against k_moe_mx above (slabs through registers, two barriers and the
+ * reduction between an item and the next loads) the compute unit always has
+ * one to two whole items in flight, phase B moves 48 KiB a step instead of
+ * 24, and a further pass of an expert re-reads its slab from the caches
+ * instead of waiting for that pass's operands on every item.  gpt-oss layer
+ * (top-4 of 128), whole call, 5 / 9 / 16 / 64 / 256 rows: 77.7 / 93.0 / 131 /
+ * 282 / 636 us there, 74.4 / 71.9 / 103 / 184 / 376 here.
+ *
+ * Bound: a compute unit's share of HBM (an item's 48 KiB: 2 us); 71 experts'
+ * 939 MB move at 5.6 TB/s in the two phases' ~167 us of the 64-row call. */
+constexpr int MR_SLAB = 24 * 1024;               /* LDS bytes of a half: 16 rows of up to 90 blocks */
+constexpr int MR_BLOCKS = MR_SLAB / (16 * MXB);  /* 90 */
+constexpr int MR_LC = MR_SLAB / 1024;            /* copies of 1 KiB a half */
+constexpr int MR_SLOTS = 3;
+constexpr int MR_CW = 8, MR_YW = 2;              /* compute and copy waves */
+constexpr int MR_NT = 64 * (MR_CW + MR_YW);
+constexpr int MR_G = 6;                          /* groups of GB blocks a compute wave holds */
+constexpr int MR_B = 2;                          /* groups whose codes are read together */
+static_assert((MR_SLOTS - 2) * MR_LC <= 63, "a vmcnt count");
+static_assert(4 * MR_G * GB >= MR_BLOCKS, "four waves cover a row");
+static_assert(16 * MXB * MR_BLOCKS + (GB - 1) * MXB + 4 <= MR_SLAB, "the last group's reads stay in the half");
+
+/* a compute lane's operands of one run: pair c16's fp8 halves of its wave's groups */
+struct MrX {
+    v8i hi[MR_G], lo[MR_G];
+    float d[MR_G];   /* q8 scale of each group */
+};
+
+template <bool DOWN>
+__global__ __launch_bounds__(MR_NT) void k_moe_mx_ring(MoeArgs a) {
+    __shared__ __attribute__((aligned(16))) uint8_t ring[MR_SLOTS][2][MR_SLAB];
+    __shared__ __attribute__((aligned(16))) v4f red[2][MR_CW][64];   /* by item parity */
+    constexpr int IR = DOWN ? MX_RING_DOWN : MX_RING_UP;
+    const int rows = DOWN ? a.D : a.I, nblk = (DOWN ? a.I : a.D) / 32;
+    const uint32_t rb = (uint32_t)nblk * MXB, mbytes = (uint32_t)rows * rb;
+    const int *items = DOWN ? a.rb_items : a.rg_items, *offs = DOWN ? a.rb_off : a.rg_off;
+    const int *rend = DOWN ? a.rb_rend : a.rg_rend, *runs = DOWN ? a.rb_runs : a.rg_runs;
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4,
+              c16 = lane & 15;
+    const int wg = ring_wg();
+    const int i0 = ldc(offs, wg), n = ldc(offs, wg + 1) - i0;
+    if (n <= 0) return;   /* uniform */
+    /* item j of the list (j < n): expert index, item rows, pass */
+    auto item = [&](int j) { return ldc(items, (size_t)(i0 + j)); };
+
+    /* The two roles run loops of their own, meeting at one barrier an item.
+     * Between the barriers of items i and i + 1 the compute waves finish item
+     * i - 1 (reading red[(i - 1) % 2]) and compute item i (reading slot
+     * i % MR_SLOTS, writing red[i % 2]) while the copy waves copy item i + 2
+     * into item i - 1's slot. */
+    if (w >= MR_CW) {
+        const int m = w - MR_CW;
+        struct Info {   /* an item's matrix and first byte; its scalar loads go out an item ahead */
+            uint64_t base;
+            int s;
+        };
+        auto info = [&](int it) __attribute__((always_inline)) {
+            const ExpDesc *e = &a.ed[it >> 16];
+            Info f;
+            f.base = DOWN ? ldc(&e->down, 0) : m ? ldc(&e->up, 0) : ldc(&e->gate, 0);
+            f.s = (it >> 8) & 255;
+            return f;
+        };
+        const uint32_t slab = 16u * rb;
+        auto copies = [&](int j, const Info &f) __attribute__((always_inline)) {
+            const u32x4 desc = buf_desc((const void *)(uintptr_t)f.base, mbytes);
+            const uint32_t first = (uint32_t)(DOWN ? 2 * f.s + m : f.s) * slab;
+            uint8_t *dst = &ring[j % MR_SLOTS][m][0];
+#pragma unroll
+            for (int k = 0; k < MR_LC; k++) {
+                const uint32_t i = 1024u * k + 16u * (uint32_t)lane;
+                copy_lanes_nt(desc, i < slab ? first + i : OOB, lds_addr(dst + 1024 * k));
+            }
+        };
+        for (int j = 0; j < MR_SLOTS - 1 && j < n; j++) copies(j, info(item(j)));
+        Info fc = info(item(min(MR_SLOTS - 1, n - 1)));   /* item i + MR_SLOTS - 1 */
+        int code = item(min(MR_SLOTS, n - 1));             /* item i + MR_SLOTS */
+        for (int i = 0; i < n; i++) {
+            /* item i's copies have landed, item i + 1's may be in flight */
+            if (i + 1 < n) wait_copies_but<(MR_SLOTS - 2) * MR_LC>();
+            else wait_copies_but<0>();
+            asm volatile("s_barrier" ::: "memory");
+            if (i + MR_SLOTS - 1 < n) copies(i + MR_SLOTS - 1, fc);
+            fc = info(code);
+            code = item(min(i + MR_SLOTS + 1, n - 1));
+        }
+        asm volatile("s_barrier" ::: "memory");
+        wait_copies();   /* no copy outlives the workgroup */
+        return;
+    }
+
+    /* the wave's half and its blocks [b0, b0 + GB ng), whole groups of a row */
+    const int m = w >> 2, cw = ((nblk + 3) / 4 + GB - 1) / GB * GB, b0 = cw * (w & 3);
+    const int ng = max(0, min(cw, nblk - b0) + GB - 1) / GB;
+    const Q8Rows &q = DOWN ? a.hq : a.xq;
+    const int qrows = DOWN ? a.P : a.k;
+    const Buf sp = make_buf(DOWN ? a.hp : a.xp, (uint32_t)((size_t)qrows * nblk * 64));
+    const Buf qd = make_buf(q.d, (uint32_t)((size_t)qrows * q.nb * 4));
+    const Buf pw = make_buf(a.p_w, (uint32_t)a.P * 4u);
+    auto load_x = [&](const int *rc, MrX &x) __attribute__((always_inline)) {
+        const bool pv = c16 < ldc(rc, 1);
+        uint32_t prow = 0u;
+        if (DOWN) {
+            prow = (uint32_t)(ldc(rc, 0) + c16);
+        } else {
+            uint32_t rj[16];
+#pragma unroll
+            for (int j = 0; j < 16; j++) rj[j] = (uint32_t)ldc(rc, 2 + j);
+#pragma unroll
+            for (int j = 0; j < 16; j++) prow = c16 == j ? rj[j] : prow;
+        }
+        const uint32_t base = prow * (uint32_t)nblk * 64u + 16u * (g & 1), dbase = prow * (uint32_t)q.nb;
+#pragma unroll
+        for (int k = 0; k < MR_G; k++) {
+            const int bq = b0 + GB * k, ba = bq + (g >> 1), bb = ba + 2;   /* blocks of bytes 0..15 and 16..31 */
+            const bool in = pv && k < ng;
+            const uint32_t oa = in && ba < nblk ? base + (uint32_t)ba * 64u : OOB;
+            const uint32_t ob = in && bb < nblk ? base + (uint32_t)bb * 64u : OOB;
+            const u32x4 h0 = ld16(sp, oa), h1 = ld16(sp, ob);
+            const u32x4 l0 = ld16(sp, oa + 32u), l1 = ld16(sp, ob + 32u);   /* OOB + 32 is past the buffer too */
+            x.hi[k] = v8i{(int)h0.x, (int)h0.y, (int)h0.z, (int)h0.w, (int)h1.x, (int)h1.y, (int)h1.z, (int)h1.w};
+            x.lo[k] = v8i{(int)l0.x, (int)l0.y, (int)l0.z, (int)l0.w, (int)l1.x, (int)l1.y, (int)l1.z, (int)l1.w};
+            x.d[k] = __uint_as_float(ld4(qd, in ? (dbase + (uint32_t)(bq >> 3)) * 4u : OOB));
+        }
+        /* taken as the values of an empty asm statement: the compiler waits
+         * for the loads there and not at their uses */
+#pragma unroll
+        for (int k = 0; k < MR_G; k++) asm volatile("" : "+v"(x.hi[k]), "+v"(x.lo[k]), "+v"(x.d[k]));
+    };
+    /* item j's slab against x: the wave's quarter of the rows' sums to red.
+     * A group's blocks lie 17 dwords after the one's before, so a lane's codes
+     * start at one byte of a dword in all of them. */
+    const uint32_t e0 = (uint32_t)c16 * rb + (uint32_t)(b0 + g) * MXB;   /* the first group's e byte */
+    const uint32_t sh = (e0 + 1u) & 3u;
+    auto compute = [&](int j, const MrX &x) __attribute__((always_inline)) {
+        const uint8_t *sb = &ring[j % MR_SLOTS][m][0];
+        const uint32_t *dw = (const uint32_t *)(sb + ((e0 + 1u) & ~3u));
+        float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k0 = 0; k0 < MR_G; k0 += MR_B) {
+            uint32_t c[MR_B][5], e[MR_B];
+#pragma unroll
+            for (int i = 0; i < MR_B; i++) {
+                if (k0 + i >= ng) break;   /* uniform */
+#pragma unroll
+                for (int t = 0; t < 5; t++) c[i][t] = dw[17 * (k0 + i) + t];
+                e[i] = sb[e0 + 68u * (k0 + i)];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < MR_B; i++) {
+                const int k = k0 + i;
+                if (k >= ng) break;   /* uniform */
+                v8i av;
+#pragma unroll
+                for (int t = 0; t < 4; t++) av[t] = (int)__builtin_amdgcn_alignbyte(c[i][t + 1], c[i][t], sh);
+                av[4] = av[5] = av[6] = av[7] = 0;
+                /* past the row: the next row's block, or the slab's end, under a finite scale and zero operands */
+                const int es = b0 + GB * k + g < nblk ? (int)e[i] : 0;
+                const v4f z = {0.f, 0.f, 0.f, 0.f};
+                v4f r = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, x.hi[k], z, FMT_FP4, FMT_FP8, 0, es, 0,
+                                                                        SCALE_16);
+                r = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, x.lo[k], r, FMT_FP4, FMT_FP8, 0, es, 0, SCALE_1);
+#pragma unroll
+                for (int v = 0; v < 4; v++) acc[v] += x.d[k] * r[v];
+            }
+        }
+        red[j & 1][w][lane] = v4f{acc[0], acc[1], acc[2], acc[3]};
+    };
+    /* finishing item j, a lane one (pair, row) result: pair 4 (w % 4) + g and
+     * row c16 (of half w / 4 in phase B; waves 0 to 3 in phase A), whose sums
+     * sit in lane 16 (c16 / 4) + pair, register c16 % 4 */
+    struct Done {   /* the item to finish: its first pair, pairs from there, first row of the wave's half, biases, pair weight */
+        int pf, nv, r;
+        float b0, b1, wt;
+    };
+    auto finish = [&](int j, const Done &f) __attribute__((always_inline)) {
+        if (!DOWN && w >= 4) return;           /* uniform */
+        if (4 * (w & 3) >= f.nv) return;       /* uniform */
+        int ln = lane;
+        asm volatile("" : "+v"(ln));   /* what follows of it is computed here, not kept in registers */
+        const int jj = 4 * (w & 3) + (ln >> 4), c = ln & 15;
+        const float *p = (const float *)&red[j & 1][DOWN ? 4 * m : 0][16 * (c >> 2) + jj] + (c & 3);
+        float s0 = 0.f, s1 = 0.f;
+#pragma unroll
+        for (int ww = 0; ww < 4; ww++) {
+            s0 += p[256 * ww];
+            if (!DOWN) s1 += p[256 * (4 + ww)];
+        }
+        const int r = f.r + c;
+        if (jj >= f.nv || r >= rows) return;
+        if (DOWN) a.part[(size_t)(f.pf + jj) * a.D + r] = f.wt * (s0 + f.b0);
+        else a.hidden[(size_t)(f.pf + jj) * a.I + r] = act_fn(a.act, s0 + f.b0, s1 + f.b1);
+    };
+
+    MrX cur;
+    Done done = {0, 0, 0, 0.f, 0.f, 0.f};
+    int run = ldc(DOWN ? a.rb_run0 : a.rg_run0, wg);   /* the run of item 0; the runs follow in order */
+    int s = (item(0) >> 8) & 255;
+    const uint64_t *bp0 = DOWN ? a.dbias : a.gbias, *bp1 = DOWN ? nullptr : a.ubias;
+    for (int i = 0; i < n; run++, s = 0) {
+        const int *rc = runs + (size_t)RING_REC * run;
+        load_x(rc, cur);
+        const int re = min(ldc(rend, (size_t)(i0 + i)), i0 + n) - i0;   /* the run's end */
+        const int pf = ldc(rc, 0), nv = ldc(rc, 1), e = ldc(rc, 2 + RING_P);
+        const uint64_t q0 = bp0 ? ldc(bp0, e) : 0, q1 = bp1 ? ldc(bp1, e) : 0;
+        const Buf bb0 = make_buf((const void *)(uintptr_t)q0, q0 ? (uint32_t)rows * 4u : 0u);   /* empty buffers read zero */
+        const Buf bb1 = make_buf((const void *)(uintptr_t)q1, q1 ? (uint32_t)rows * 4u : 0u);
+        const int jj = 4 * (w & 3) + g;
+        const float wt = DOWN ? __uint_as_float(ld4(pw, jj < nv ? (uint32_t)(pf + jj) * 4u : OOB)) : 0.f;
+        for (; i < re; i++, s++) {
+            bar_lds();   /* item i's slab has landed, item i - 1's sums are in LDS */
+            finish(i - 1, done);   /* nothing before the first item: no pairs */
+            done.pf = pf;
+            done.nv = nv;
+            done.r = IR * s + (DOWN ? 16 * m : 0);
+            if (bp0) done.b0 = __uint_as_float(ld4(bb0, (uint32_t)(done.r + c16) * 4u));
+            if (bp1) done.b1 = __uint_as_float(ld4(bb1, (uint32_t)(done.r + c16) * 4u));
+            done.wt = wt;
+            compute(i, cur);
+        }
+    }
+    bar_lds();   /* item n - 1's sums are in LDS */
+    finish(n - 1, done);
+}
+
+/* the operands' offsets and OOB must not meet */
+bool mx_ring_fits(const Q8Rows &q, int qrows, int nblk) {
+    return (uint64_t)qrows * nblk * 64 < OOB && (uint64_t)qrows * q.nb * 4 < OOB;
+}
+
+}  // namespace
+
+bool mx_ring_shape(int rows, int cols, int item_rows) {
+    return cols / 32 <= MR_BLOCKS && (rows + item_rows - 1) / item_rows <= 256;   /* an item holds its rows in 8 bits */
+}
+
 void launch_moe_a_mx(const MoeArgs &a, hipStream_t st) {
+    if (a.rg_items && a.rg_mx && mx_ring_fits(a.xq, a.k, a.D / 32)) {
+        hipLaunchKernelGGL(k_moe_mx_ring<false>, dim3(a.rg_n), dim3(MR_NT), 0, st, a);
+        return;
+    }
     launch_mx<2, false>(a, a.D, a.n_act_a * ((a.I + 15) / 16), st);
 }
 
 void launch_moe_b_mx(const MoeArgs &a, hipStream_t st) {
+    if (a.rb_items && a.rb_mx && mx_ring_fits(a.hq, a.P, a.I / 32)) {
+        hipLaunchKernelGGL(k_moe_mx_ring<true>, dim3(a.rb_n), dim3(MR_NT), 0, st, a);
+        return;
+    }
     launch_mx<1, true>(a, a.I, a.n_act_b * ((a.D + 15) / 16), st);
 }
 

@@ -122,16 +122,6 @@ __device__ inline int mul_bytes(uint32_t q, uint32_t f) {
 
 __device__ inline int byte_of(uint32_t w, int i) { return (int)((w >> (8 * i)) & 0xFFu); }
 
-/* copy_lanes with the nontemporal hint: each slab byte is read once per
- * call (64- and 128-token Qwen3 prefills measured 5% faster with it); the
- * same 5 wait states before the load */
-__device__ inline void copy_lanes_nt(const u32x4 &desc, uint32_t voff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds"
-                 :
-                 : "s"(lds), "v"(voff), "s"(desc)
-                 : "memory");
-}
-
 }  // namespace
 
 /* Phase A: hidden[p][r] = act(gate_r . xq_p + bg[r], up_r . xq_p + bu[r])
@@ -337,13 +327,6 @@ constexpr int RG_NT = 64 * (RG_CW + RG_YW);
 static_assert((RG_SLOTS - 2) * RG_LC <= 63, "a vmcnt count");
 static_assert(RG_SLAB % 1024 == 0, "whole copies");
 static_assert(RG_UNITS % 8 == 0, "the swizzle stays inside a row");
-
-/* Workgroup g runs on XCD g % 8: neighbouring stretches of the item list go
- * to one XCD, so the passes of an expert read its slabs from that XCD's L2 */
-__device__ inline int ring_wg() {
-    const int g = (int)blockIdx.x, G = (int)gridDim.x;
-    return G % 8 ? g : (g % 8) * (G / 8) + g / 8;
-}
 
 __device__ inline uint32_t rg_unit(int r, int u) { return (uint32_t)(RG_UNITS * r + (u ^ ((r >> 1) & 7))); }
 
@@ -1101,16 +1084,16 @@ bool qa_ring_shape(int gate_fmt, int D, int I) { return gate_fmt == TG_FMT_Q4K &
  * pair, pair count, the input rows of its first 16 pairs) in list order and
  * run0[w] the run of workgroup w's first item, so a compute wave reaches a
  * run's operands with one round trip of scalar loads. */
-void ring_items(const ExpDesc *ed, int n_act, int slabs, int G, const int *p_row, int P, const RingCost &c,
-                RingLists &r) {
+void ring_items(const ExpDesc *ed, int n_act, int slabs, int G, const int *p_row, int P, int pass_pairs,
+                const RingCost &c, RingLists &r) {
     r.items.clear();
     r.rend.clear();
     r.runs.clear();
     for (int ei = 0; ei < n_act; ei++)
-        for (int t = 0; t < std::max(1, (ed[ei].np + RING_P - 1) / RING_P); t++) {
-            const int run = (int)(r.runs.size() / RING_REC), pf = ed[ei].p0 + RING_P * t;
+        for (int t = 0; t < std::max(1, (ed[ei].np + pass_pairs - 1) / pass_pairs); t++) {
+            const int run = (int)(r.runs.size() / RING_REC), pf = ed[ei].p0 + pass_pairs * t;
             r.runs.push_back(pf);
-            r.runs.push_back(ed[ei].np - RING_P * t);
+            r.runs.push_back(ed[ei].np - pass_pairs * t);
             for (int j = 0; j < RING_P; j++) r.runs.push_back(p_row[std::min(pf + j, P - 1)]);
             r.runs.push_back(ed[ei].e);
             r.runs.resize((size_t)(run + 1) * RING_REC, 0);

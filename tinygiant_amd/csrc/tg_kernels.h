@@ -64,6 +64,7 @@ struct MoeArgs {
     const int *rb_items, *rb_off, *rb_rend; /* the persistent down phase's, or null */
     const int *rb_runs, *rb_run0;
     int rb_n;
+    int rg_mx, rb_mx;                       /* those lists are the MXFP4 phases' (passes of MX_RING_P pairs) */
 };
 
 int items_per_row(int fmt, int ncols);
@@ -139,9 +140,9 @@ bool qb_ring_shape(int I, int D);
 /* The persistent phases' items (expert, pass, slab of `slabs`) cut into G
  * workgroup ranges (off), the end of each item's run (rend: the items of one
  * expert and pass), the runs' records (RING_REC ints each: the run's first
- * pair p0 + RING_P t, the pairs from there on, possibly more than RING_P,
- * the input rows of its first RING_P pairs, the last pair's row past the
- * end, and the expert) and the run of each workgroup's first item (run0). */
+ * pair p0 + pass_pairs t, the pairs from there on, possibly more than a pass
+ * holds, the input rows of its first RING_P pairs, the last pair's row past
+ * the end, and the expert) and the run of each workgroup's first item (run0). */
 constexpr int RING_T = 2, RING_P = 16 * RING_T;   /* tiles of 16 pairs a pass, pairs a pass */
 constexpr int RING_REC = 2 + RING_P + 2;   /* padded */
 struct RingLists {
@@ -157,8 +158,16 @@ struct RingCost {
 };
 constexpr RingCost QA_RING_COST = {2500, 1600, 6500, 2300}, QB_RING_COST = {2000, 1450, 5500, 2200};
 constexpr int RING_MAX_ROWS = 256 * RING_P;   /* an item holds its pass in 8 bits */
-void ring_items(const ExpDesc *ed, int n_act, int slabs, int G, const int *p_row, int P, const RingCost &c,
-                RingLists &r);
+void ring_items(const ExpDesc *ed, int n_act, int slabs, int G, const int *p_row, int P, int pass_pairs,
+                const RingCost &c, RingLists &r);
+/* The persistent MXFP4 phases (tg_grouped.hip): rows of up to 90 blocks, passes
+ * of MX_RING_P pairs, gate/up items of 16 rows of both matrices and down items
+ * of 32 rows. */
+constexpr int MX_RING_P = 16, MX_RING_UP = 16, MX_RING_DOWN = 32;
+constexpr int MX_RING_MAX_ROWS = 256 * MX_RING_P;
+/* an item is 48 KiB, 2 us of a compute unit's share of HBM; a run's operands come behind 1.5 items */
+constexpr RingCost MX_COST = {3000, 2000, 3000, 2000};
+bool mx_ring_shape(int rows, int cols, int item_rows);
 constexpr int QA_RING_MAX_G = 1024;
 void launch_moe_a_qk(const MoeArgs &a, hipStream_t st);
 void launch_moe_b_qk(const MoeArgs &a, hipStream_t st);
