@@ -194,6 +194,8 @@ struct Q8Rows {
     const float *f;   /* the unquantized f32 rows (used by F16 weights) */
     int nb;
     int fstride;      /* floats per f32 row */
+    uint8_t *split;   /* where the rows' fp8 halves go as they are quantized (q8_split_store), or null */
+    int split_nblk;   /* 32-value blocks of a row there */
 };
 
 struct Q8Row {
@@ -282,6 +284,40 @@ __device__ inline float wave_sum_x(float v) {
     return seg_sum_x<32>(v);
 }
 
+/* fp8 e4m3 code of an integer in [-15, 15] (exact) */
+__device__ inline uint32_t e4m3_int(int n) {
+    if (n == 0) return 0;
+    const uint32_t m = (uint32_t)(n < 0 ? -n : n);
+    const uint32_t e = 31u - (uint32_t)__builtin_clz(m);   /* 0..3 */
+    return (n < 0 ? 0x80u : 0u) | ((e + 7u) << 3) | ((m << (3u - e)) & 7u);
+}
+
+/* The fp8 halves of the wave's q8 block (lane l: its values 4l .. 4l + 3), for
+ * the block-scaled MFMA phases: dst[row][block of 32][part][32], the codes of
+ * hi = x >> 4 (part 0) and lo = x & 15 (part 1), position 2t value t and
+ * 2t + 1 value 16 + t of the block.  Lanes l and l ^ 4 of a block hold values
+ * 16 apart: they trade a half, so each writes eight bytes of one part.  (In a
+ * launch of its own, one byte of q8 a load, this took 4.9 us after every q8
+ * launch of 4.1.) */
+__device__ inline void q8_split_store(uint32_t packed, int lane, uint8_t *dst, int nblk, int r, int b) {
+    uint32_t h = 0, l = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int v = (int)(int8_t)(packed >> (8 * j));
+        h |= e4m3_int(v >> 4) << (8 * j);
+        l |= e4m3_int(v & 15) << (8 * j);
+    }
+    const bool up = lane & 4;   /* values 16 .. 31 of the block; writes the lo part */
+    const uint32_t got = (uint32_t)__shfl_xor((int)(up ? h : l), 4, 64);
+    const uint32_t a = up ? got : h, c = up ? l : got;   /* values t and 16 + t */
+    const int blk = b * 8 + (lane >> 3);
+    if (blk >= nblk) return;
+    u32x2 o;
+    o.x = __builtin_amdgcn_perm(c, a, 0x05010400u);
+    o.y = __builtin_amdgcn_perm(c, a, 0x07030602u);
+    *reinterpret_cast<u32x2 *>(dst + ((size_t)r * nblk + blk) * 64 + (up ? 32 : 0) + 8 * (lane & 3)) = o;
+}
+
 /* q8_block_quant of the wave's block, written to block b of row r */
 __device__ inline void q8_block_store(float v0, float v1, float v2, float v3, int lane, const Q8Rows &out, int r,
                                       int b) {
@@ -296,6 +332,7 @@ __device__ inline void q8_block_store(float v0, float v1, float v2, float v3, in
         out.d[rb] = q.sc;
         out.sum[rb] = q.tot;
     }
+    if (out.split) q8_split_store(q.packed, lane, out.split, out.split_nblk, r, b);   /* uniform */
 }
 
 __device__ inline Q8Row q8_row(const Q8Rows &a, int r) {

@@ -87,35 +87,15 @@ __device__ inline T ldg(const T *p, size_t i) {
     return ((const __attribute__((address_space(1))) T *)(uintptr_t)p)[i];
 }
 
-/* fp8 e4m3 code of an integer in [-15, 15] (exact) */
-__device__ inline uint32_t e4m3_int(int n) {
-    if (n == 0) return 0;
-    const uint32_t m = (uint32_t)(n < 0 ? -n : n);
-    const uint32_t e = 31u - (uint32_t)__builtin_clz(m);   /* 0..3 */
-    return (n < 0 ? 0x80u : 0u) | ((e + 7u) << 3) | ((m << (3u - e)) & 7u);
-}
-
 }  // namespace
 
-/* dst[r][b][part][32]: for q8 row r and block b of 32 values, the fp8 codes of
- * hi = x >> 4 (part 0) and lo = x & 15 (part 1) in MFMA K order (position 2t
- * holds value t, 2t + 1 value 16 + t).  One thread per 4 output bytes. */
+/* q8_split_store of rows that were quantized elsewhere.  One wave per 256
+ * values. */
 __global__ __launch_bounds__(256) void k_mx_split(Q8Rows q, int nrows, int nblk, uint8_t *dst) {
-    const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;   /* 4-byte group */
-    const size_t per_row = (size_t)nblk * 16;
-    if (i >= (size_t)nrows * per_row) return;
-    const int r = (int)(i / per_row), rem = (int)(i % per_row);
-    const int b = rem / 16, part = (rem / 8) & 1, p0 = (rem % 8) * 4;
-    const int8_t *x = q.qs + (size_t)r * q.nb * 256 + (size_t)b * 32;
-    uint32_t w = 0;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int p = p0 + j;
-        const int v = x[(p & 1) ? 16 + (p >> 1) : (p >> 1)];
-        const int half = part == 0 ? (v >> 4) : (v & 15);
-        w |= e4m3_int(half) << (8 * j);
-    }
-    *(uint32_t *)(dst + (size_t)r * nblk * 64 + (size_t)b * 64 + part * 32 + p0) = w;
+    const int wave = (int)((blockIdx.x * (size_t)blockDim.x + threadIdx.x) >> 6), lane = threadIdx.x & 63;
+    if (wave >= nrows * q.nb) return;   /* uniform per wave */
+    const uint32_t packed = reinterpret_cast<const uint32_t *>(q.qs + (size_t)wave * 256)[lane];
+    q8_split_store(packed, lane, dst, nblk, wave / q.nb, wave % q.nb);
 }
 
 /* The e8m0 scale byte 255 means 2^127 to the reference (e8m0_to_fp32_half,
@@ -137,9 +117,9 @@ void launch_mx_scan_e255(const uint8_t *p, uint64_t nbytes, unsigned *flag_dev, 
 }
 
 void launch_mx_split(const Q8Rows &q, int nrows, int ncols, uint8_t *dst, hipStream_t st) {
-    const size_t n = (size_t)nrows * (ncols / 32) * 16;
-    if (n == 0) return;
-    hipLaunchKernelGGL(k_mx_split, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, q, nrows, ncols / 32, dst);
+    const int waves = nrows * q.nb;
+    if (waves <= 0) return;
+    hipLaunchKernelGGL(k_mx_split, dim3((waves + 3) / 4), dim3(256), 0, st, q, nrows, ncols / 32, dst);
 }
 
 namespace {

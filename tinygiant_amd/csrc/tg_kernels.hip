@@ -1137,13 +1137,18 @@ void launch_moe(const MoeArgs &a, const int *down_fmts_present, int n_down_fmts,
                      (uint64_t)a.P * a.D * 4 < (1ull << 31);
     /* 1. quantize the k input rows */
     if (quantize_x && !qx_fused) {
-        launch_quantize(a.xin, a.D, a.k, a.D, a.xq, st);
+        Q8Rows xq = a.xq;
+        if (mx_a) {   /* the MFMA phases read the rows' fp8 halves */
+            xq.split = a.xp;
+            xq.split_nblk = a.D / 32;
+        }
+        launch_quantize(a.xin, a.D, a.k, a.D, xq, st);
         if (mark) (*mark)(1);
     }
     /* 2. phase A: MXFP4 experts with many pairs take the MFMA kernel, which
      * reads each weight block once for up to 64 pairs */
     if (mx_a) {
-        launch_mx_split(a.xq, a.k, a.D, a.xp, st);
+        if (!quantize_x) launch_mx_split(a.xq, a.k, a.D, a.xp, st);
         launch_moe_a_mx(a, st);
     } else {
         int T;
@@ -1176,14 +1181,18 @@ void launch_moe(const MoeArgs &a, const int *down_fmts_present, int n_down_fmts,
     if (mark) (*mark)(2);
     /* 3. quantize the hidden rows */
     if (!qh_fused) {
-        launch_quantize(a.hidden, a.I, a.P, a.I, a.hq, st);
+        Q8Rows hq = a.hq;
+        if (mx_grouped && a.hp) {
+            hq.split = a.hp;
+            hq.split_nblk = a.I / 32;
+        }
+        launch_quantize(a.hidden, a.I, a.P, a.I, hq, st);
         if (mark) (*mark)(3);
     }
     /* 4. phase B, once per down format present */
     for (int i = 0; i < n_down_fmts; i++) {
         const int fmt = down_fmts_present[i];
         if (mx_grouped && fmt == TG_FMT_MXFP4 && a.hp) {
-            launch_mx_split(a.hq, a.P, a.I, a.hp, st);
             launch_moe_b_mx(a, st);
             continue;
         }
