@@ -287,3 +287,15 @@ def test_attention_span_edges(tg, orc, hd, nkv, ratio, kv_len, window):
     c = _case(500 + kv_len + hd, 256, nkv * ratio, nkv, hd, (Q80, Q80, Q80, Q80), kv_len + 3, kv_len, norms=ratio != 4,
               sinks=ratio == 8, x_scale=0.02 if ratio == 4 else 1.0)
     _check(orc, c, window, _gpu(tg, c, window), _oracle(orc, c, window))
+
+
+@pytest.mark.parametrize("hd,nkv,ratio,kv_len", [
+    (128, 2, 2, 2112),     # 33 spans, the first count that is not combined in the span kernel
+    (64, 2, 2, 8200),      # 65: one chunk past those requested up front, four heads a block
+    (128, 1, 2, 16400)])   # 256, the most: one KV head, a workgroup a CU
+def test_attention_combine_edges(tg, orc, hd, nkv, ratio, kv_len):
+    """k_attn_combine_q8 at the edges of what it requests up front."""
+    say("attention combine", hd, nkv, ratio, kv_len)
+    c = _case(700 + kv_len + hd, 256, nkv * ratio, nkv, hd, (Q80, Q80, Q80, Q80), kv_len + 3, kv_len, norms=True,
+              sinks=hd != 128)
+    _check(orc, c, 0, _gpu(tg, c, 0), _oracle(orc, c, 0))

@@ -646,72 +646,102 @@ __global__ __launch_bounds__(256) void k_attn_combine(const float *__restrict__ 
  * of k_quantize_q8) into aq.  Wave g takes the chunks c = g (mod 8); lane p
  * takes values 4p .. 4p + 3 of the block (head p / (head_dim / 4)), so the
  * chunk loads of a thread are independent and go out together.  The eight
- * wave partials are added in wave order. */
-constexpr int CQ_WAVES = 8;
+ * wave partials are added in wave order.
+ * Bound: one memory round trip and the launch; the maxima, sums and first
+ * CQ_PRE chunks a wave are one batch of loads (in three, one behind the
+ * other, a call over 4,000 positions of 4 KV heads took 25.7 us, not 24.4). */
+constexpr int CQ_WAVES = 8, CQ_PRE = 8;
+static_assert(SPAN_WGS <= CQ_WAVES * 64, "a thread a chunk: head_dim 64 and 128 run k_attn_span");
 __global__ __launch_bounds__(CQ_WAVES * 64) void k_attn_combine_q8(const float *__restrict__ part,
                                                                    const float *__restrict__ sinks, float *att,
                                                                    int n_heads, int head_dim, int nchunks,
                                                                    Q8Rows aq) {
-    __shared__ float scale[4 * ATTN_MAX_CHUNKS];   /* [head][chunk]: hpb <= 4 (head_dim >= 64) */
+    __shared__ float scale[4 * SPAN_WGS];   /* [head][chunk]: hpb <= 4 (head_dim >= 64) */
     __shared__ float redm[CQ_WAVES][4], redl[CQ_WAVES][4];
-    __shared__ float hm[4], hl[4];
+    __shared__ float hl[4];
     __shared__ __attribute__((aligned(16))) float osum[CQ_WAVES][256];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int hpb = 256 / head_dim, h0 = blockIdx.x * hpb;
     const size_t stride = (size_t)head_dim + 2;
     float *sc = scale;   /* sc[j * nchunks + c] */
+    /* the thread's maxima and sums of each head, and the V sums of its first
+     * CQ_PRE chunks, all requested before any is used */
+    float2 ml[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+        ml[j] = j < hpb && tid < nchunks ? *reinterpret_cast<const float2 *>(part + ((size_t)(h0 + j) * nchunks + tid) * stride)
+                                         : make_float2(-INFINITY, 0.f);
+    float sk[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) sk[j] = sinks && j < hpb ? sinks[h0 + j] : 0.f;
+    const int tph = head_dim / 4;
+    const int j = lane / tph, d = 4 * (lane - j * tph);
+    const float *ph = part + (size_t)(h0 + j) * nchunks * stride + 2 + d;
+    float2 va[CQ_PRE], vb[CQ_PRE];
+#pragma unroll
+    for (int i = 0; i < CQ_PRE; i++) {
+        const int c = wave + CQ_WAVES * i;
+        va[i] = vb[i] = make_float2(0.f, 0.f);
+        if (c < nchunks) {   /* uniform */
+            va[i] = *reinterpret_cast<const float2 *>(ph + c * stride);
+            vb[i] = *reinterpret_cast<const float2 *>(ph + c * stride + 2);
+        }
+    }
     /* maxima, per head over all chunks */
-    for (int j = 0; j < hpb; j++) {
-        const float *ph = part + (size_t)(h0 + j) * nchunks * stride;
-        float m = -INFINITY;
-        for (int c = tid; c < nchunks; c += CQ_WAVES * 64) m = fmaxf(m, ph[c * stride]);
-        m = wave_max(m);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        if (j >= hpb) break;
+        const float m = wave_max(ml[j].x);
         if (lane == 0) redm[wave][j] = m;
     }
     __syncthreads();
-    if (tid < hpb) {
-        float M = redm[0][tid];
-        for (int w = 1; w < CQ_WAVES; w++) M = fmaxf(M, redm[w][tid]);
-        if (sinks) M = fmaxf(M, sinks[h0 + tid]);
-        hm[tid] = M;
-    }
-    __syncthreads();
     /* chunk scales and the sums of exponentials */
-    for (int j = 0; j < hpb; j++) {
-        const float *ph = part + (size_t)(h0 + j) * nchunks * stride;
-        const float M = hm[j];
+    float hm[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        if (j >= hpb) break;
+        float M = redm[0][j];
+#pragma unroll
+        for (int w = 1; w < CQ_WAVES; w++) M = fmaxf(M, redm[w][j]);
+        if (sinks) M = fmaxf(M, sk[j]);
+        hm[j] = M;
         float l = 0.f;
-        for (int c = tid; c < nchunks; c += CQ_WAVES * 64) {
-            const float e = expf(ph[c * stride] - M);
-            sc[j * nchunks + c] = e;
-            l = fmaf(ph[c * stride + 1], e, l);
+        if (tid < nchunks) {
+            const float e = expf(ml[j].x - M);
+            sc[j * nchunks + tid] = e;
+            l = fmaf(ml[j].y, e, l);
         }
         l = wave_sum(l);
         if (lane == 0) redl[wave][j] = l;
     }
     __syncthreads();
-    if (tid < hpb) {
-        float L = redl[0][tid];
-        for (int w = 1; w < CQ_WAVES; w++) L += redl[w][tid];
-        if (sinks) L += expf(sinks[h0 + tid] - hm[tid]);
-        hl[tid] = 1.f / L;
+    if (wave == 0) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (j >= hpb) break;
+            float L = redl[0][j];
+            for (int w = 1; w < CQ_WAVES; w++) L += redl[w][j];
+            if (sinks) L += expf(sk[j] - hm[j]);
+            if (lane == 0) hl[j] = 1.f / L;   /* read by this wave alone */
+        }
     }
     /* V sums: lane p, chunks c = wave (mod 8) */
-    const int tph = head_dim / 4;
-    const int j = lane / tph, d = 4 * (lane - j * tph);
-    const float *ph = part + (size_t)(h0 + j) * nchunks * stride + 2 + d;
     const float *sj = sc + j * nchunks;
     float o0 = 0.f, o1 = 0.f, o2 = 0.f, o3 = 0.f;
-#pragma unroll 8
-    for (int c = wave; c < nchunks; c += CQ_WAVES) {
-        const float2 a = *reinterpret_cast<const float2 *>(ph + c * stride);
-        const float2 b = *reinterpret_cast<const float2 *>(ph + c * stride + 2);
-        const float e = sj[c];
+    auto add = [&](const float2 &a, const float2 &b, float e) {
         o0 = fmaf(a.x, e, o0);
         o1 = fmaf(a.y, e, o1);
         o2 = fmaf(b.x, e, o2);
         o3 = fmaf(b.y, e, o3);
+    };
+#pragma unroll
+    for (int i = 0; i < CQ_PRE; i++) {
+        const int c = wave + CQ_WAVES * i;
+        if (c < nchunks) add(va[i], vb[i], sj[c]);
     }
+#pragma unroll 8
+    for (int c = wave + CQ_WAVES * CQ_PRE; c < nchunks; c += CQ_WAVES)
+        add(*reinterpret_cast<const float2 *>(ph + c * stride), *reinterpret_cast<const float2 *>(ph + c * stride + 2), sj[c]);
     reinterpret_cast<float4 *>(osum[wave])[lane] = make_float4(o0, o1, o2, o3);
     __syncthreads();
     if (wave == 0) {
