@@ -91,8 +91,6 @@ struct Ctx {
     /* grow-only device arena for per-call scratch, pinned host staging */
     uint8_t *arena = nullptr;
     size_t arena_cap = 0;
-    uint8_t *pin = nullptr;
-    size_t pin_cap = 0;
     /* coherent (uncached on the device) pinned rows that kernels read and
      * write in place: the input and output rows of the host-pointer MoE call */
     uint8_t *io = nullptr;
@@ -124,19 +122,6 @@ uint8_t *arena(size_t n) {
         g.arena_cap = cap;
     }
     return g.arena;
-}
-
-uint8_t *pinned(size_t n) {
-    if (n > g.pin_cap) {
-        if (g.pin) {
-            HIPCHECK(hipStreamSynchronize(g.st));
-            HIPCHECK(hipHostFree(g.pin));
-        }
-        size_t cap = std::max(n, (size_t)4 << 20);
-        HIPCHECK(hipHostMalloc(&g.pin, cap, hipHostMallocDefault));
-        g.pin_cap = cap;
-    }
-    return g.pin;
 }
 
 uint8_t *io_rows(size_t n) {
@@ -278,6 +263,8 @@ struct HostPlan {
     std::vector<float> p_w;
     bool has_gb = false, has_ub = false, has_db = false;
     std::vector<int> fmts_present;
+    int max_rows = 0;      /* most pairs of any one expert */
+    bool rings = true;     /* lay out the persistent phases' lists */
 };
 
 /* ---- MXFP4 scale byte 255 ----
@@ -402,6 +389,8 @@ void build_pairs(HostPlan &h, const float *row_weights) {
     }
     h.r_off[h.k] = (int)h.r_pair.size();
     h.fmts_present.clear();
+    h.max_rows = 0;
+    for (int e = 0; e < h.n; e++) h.max_rows = std::max(h.max_rows, h.p_off[e + 1] - h.p_off[e]);
     for (int e = 0; e < h.n; e++)
         if (h.p_off[e + 1] > h.p_off[e] &&
             std::find(h.fmts_present.begin(), h.fmts_present.end(), h.down_fmt[e]) == h.fmts_present.end())
@@ -435,7 +424,7 @@ static int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
 /* every active expert's down matrix is MXFP4, in the persistent phase's shape */
 static bool mx_down_ring(const HostPlan &h) {
-    return h.fmts_present.size() == 1 && h.fmts_present[0] == TG_FMT_MXFP4 && mx_ring_shape(h.D, h.I, MX_RING_DOWN);
+    return h.rings && h.fmts_present.size() == 1 && h.fmts_present[0] == TG_FMT_MXFP4 && mx_ring_shape(h.D, h.I, MX_RING_DOWN);
 }
 
 Layout plan_layout(const HostPlan &h) {
@@ -449,16 +438,16 @@ Layout plan_layout(const HostPlan &h) {
     t += (size_t)(n + 1) * 4 + (size_t)P * 4 * 4 + (size_t)(k + 1) * 4 + 8;   /* p_off, p_row, p_exp, p_w, r_off, r_pair */
     t += (size_t)4 * (n + 1) * 4 + 16;      /* active expert lists and their cost prefixes */
     t += (size_t)n * sizeof(ExpDesc) + 16;  /* active expert descriptors */
-    if (qa_ring_shape(h.gate_fmt, h.D, h.I))  /* the persistent gate/up phase's items and ranges */
+    if (h.rings && qa_ring_shape(h.gate_fmt, h.D, h.I))  /* the persistent gate/up phase's items and ranges */
         t += 2 * (size_t)(h.I / 16) * (P / 16 + n + 1) * 4 + (size_t)RING_REC * (P / 16 + n + 1) * 4 +
              2 * (QA_RING_MAX_G + 1) * 4 + 64;
-    if (h.gate_fmt == TG_FMT_MXFP4 && mx_ring_shape(h.I, h.D, MX_RING_UP))
+    if (h.rings && h.gate_fmt == TG_FMT_MXFP4 && mx_ring_shape(h.I, h.D, MX_RING_UP))
         t += 2 * (size_t)ceil_div(h.I, MX_RING_UP) * (P / MX_RING_P + n + 1) * 4 +
              (size_t)RING_REC * (P / MX_RING_P + n + 1) * 4 + 2 * (QA_RING_MAX_G + 1) * 4 + 64;
     if (mx_down_ring(h))
         t += 2 * (size_t)ceil_div(h.D, MX_RING_DOWN) * (P / MX_RING_P + n + 1) * 4 +
              (size_t)RING_REC * (P / MX_RING_P + n + 1) * 4 + 2 * (QA_RING_MAX_G + 1) * 4 + 64;
-    else if (qb_ring_shape(h.I, h.D))  /* the persistent down phase's */
+    else if (h.rings && qb_ring_shape(h.I, h.D))  /* the persistent down phase's */
         t += 2 * (size_t)(h.D / 32) * (P / 16 + n + 1) * 4 + (size_t)RING_REC * (P / 16 + n + 1) * 4 +
              2 * (QA_RING_MAX_G + 1) * 4 + 64;
     L.tables_len = t + 64;
@@ -585,10 +574,10 @@ MoeArgs plan_args(const HostPlan &h, const Layout &L, uint8_t *dev, uint8_t *img
         off = (const int *)put(r.off.data(), r.off.size() * 4);
         n_wg = (int)r.off.size() - 1;
     };
-    const bool mx_up = h.gate_fmt == TG_FMT_MXFP4 && mx_ring_shape(h.I, h.D, MX_RING_UP), mx_down = mx_down_ring(h);
+    const bool mx_up = h.rings && h.gate_fmt == TG_FMT_MXFP4 && mx_ring_shape(h.I, h.D, MX_RING_UP), mx_down = mx_down_ring(h);
     a.rg_mx = mx_up && a.max_rows <= MX_RING_MAX_ROWS;
     a.rb_mx = mx_down && a.max_rows <= MX_RING_MAX_ROWS;
-    if (a.n_act_a > 0) {
+    if (h.rings && a.n_act_a > 0) {
         if (a.rg_mx)
             ring(ceil_div(h.I, MX_RING_UP), MX_RING_P, MX_COST, a.rg_items, a.rg_rend, a.rg_runs, a.rg_run0, a.rg_off,
                  a.rg_n);
@@ -646,6 +635,10 @@ void moe_host(const uint8_t *const *gate_ptrs, const uint8_t *const *up_ptrs, co
     build_pairs(h, row_weights);
     if (h.P == 0) return;   /* every weight is zero: output unchanged */
 
+    /* the lists only where launch_moe can take the persistent phases (for one
+     * row of 8 experts they would be ten times the other tables) */
+    const int qk = qk_min_rows() >= 0 ? qk_min_rows() : QK_RING_MIN_ROWS, mx = grouped_min_rows();
+    h.rings = (qk > 0 && h.max_rows >= qk) || (mx > 0 && h.max_rows >= mx);
     Layout L = plan_layout(h);
     Bump bump;
     bump.off = L.total;
@@ -696,13 +689,13 @@ void moe_host(const uint8_t *const *gate_ptrs, const uint8_t *const *up_ptrs, co
     uint8_t *dev = arena(bump.off);
     for (auto &f : fixes) (*f.vec)[f.idx] += (uint64_t)(uintptr_t)dev;
 
-    /* the tables go over in one copy; the input rows are read and the output
-     * rows accumulated in place in coherent pinned memory (the q8 kernel and
-     * the combine reach them over the host link), which saves three copy
-     * launches per call */
-    const size_t io_len = (size_t)k * D * 4;
-    uint8_t *img = pinned(L.tables_len);
-    uint8_t *io = io_rows(2 * io_len);
+    /* Nothing is copied in a launch of its own: the input rows are read and
+     * the output rows accumulated in place in coherent pinned memory (the q8
+     * kernel and the combine reach them over the host link), and the q8
+     * kernel, the first of the call, moves the tables. */
+    const size_t io_len = (size_t)k * D * 4, tab_len = (L.tables_len + 15) & ~(size_t)15;
+    uint8_t *io = io_rows(2 * io_len + tab_len);
+    uint8_t *img = io + 2 * io_len;   /* io_len is a multiple of 128 */
     MoeArgs a = plan_args(h, L, dev, img);
     memcpy(io, inputs, io_len);
     memcpy(io + io_len, output, io_len);
@@ -714,7 +707,7 @@ void moe_host(const uint8_t *const *gate_ptrs, const uint8_t *const *up_ptrs, co
      * of their own that every fused combine leaves zeroed */
     a.ctr = host_call_tickets(moe_ctr_words(D));
     a.ctr_n = a.ctr ? moe_ctr_words(D) : 0;
-    HIPCHECK(hipMemcpyAsync(dev + L.tables, img, L.tables_len, hipMemcpyHostToDevice, g.st));
+    a.tables = {img, dev + L.tables, (uint32_t)tab_len};
     for (auto &it : sg.items) HIPCHECK(hipMemcpyAsync(dev + it.off, it.host, it.n, hipMemcpyHostToDevice, g.st));
     if (grouped_min_rows() > 0 && a.max_rows >= grouped_min_rows()) {
         /* the MFMA phases are a candidate: no e8m0 byte of 255 may reach
@@ -1190,7 +1183,6 @@ TG_API void tg_hip_shutdown(void) {
     release_marks();
     if (g.arena) HIPCHECK(hipFree(g.arena));
     if (g.tickets) HIPCHECK(hipFree(g.tickets));
-    if (g.pin) HIPCHECK(hipHostFree(g.pin));
     if (g.io) HIPCHECK(hipHostFree(g.io));
     HIPCHECK(hipStreamDestroy(g.st));
     g = Ctx();

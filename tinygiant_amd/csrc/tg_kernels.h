@@ -25,6 +25,14 @@ struct ExpDesc {
     int row[EXP_ROWS];
 };
 
+/* n bytes (a multiple of 16, both ends 16-byte aligned) that a q8 launch moves
+ * on the way, for the kernels behind it */
+struct TableCopy {
+    const uint8_t *src;
+    uint8_t *dst;
+    uint32_t n;
+};
+
 /* Everything one MoE layer call needs, all pointers on the device.
  * Pairs p = (expert e, active input row) are numbered expert-major, in the
  * order the reference gathers them (csrc/libtinygiant.c:1411-1423). */
@@ -64,6 +72,7 @@ struct MoeArgs {
     const int *rb_items, *rb_off, *rb_rend; /* the persistent down phase's, or null */
     const int *rb_runs, *rb_run0;
     int rb_n;
+    TableCopy tables;                       /* with xin_remote: the call's tables, in host memory until the q8 launch moves them */
     int rg_mx, rb_mx;                       /* those lists are the MXFP4 phases' (passes of MX_RING_P pairs) */
 };
 
@@ -73,7 +82,7 @@ uint32_t row_bytes(int fmt, int ncols);
 /* q8 of nrows rows; clear[0 .. nclear) (nclear <= 64) are zeroed on the way,
  * for a consumer launched next (the fused head's argmax keys) */
 void launch_quantize(const float *x, int ncols, int nrows, long xstride, const Q8Rows &out, hipStream_t st,
-                     unsigned long long *clear = nullptr, int nclear = 0);
+                     unsigned long long *clear = nullptr, int nclear = 0, const TableCopy &cp = {});
 /* up to three matrices of one width (ncols) against the same k rows:
  * y_j[i * ystride + r] = dot(W_j row r, x_i) + bias_j[r] */
 struct GemvJob {
@@ -172,6 +181,7 @@ constexpr int QA_RING_MAX_G = 1024;
 void launch_moe_a_qk(const MoeArgs &a, hipStream_t st);
 void launch_moe_b_qk(const MoeArgs &a, hipStream_t st);
 void set_qk_min_rows(int rows);
+constexpr int QK_RING_MIN_ROWS = 17;
 int qk_min_rows();
 /* Q4_K / Q6_K experts: one workgroup column per active expert, each weight
  * row read once for all its pairs (EM_ON), or one per pair (0).  For layers

@@ -31,16 +31,22 @@ namespace tg {
 
 /* ======================= q8 quantization ======================= */
 
-/* One wave per 256-value block: lane l owns values 4l..4l+3. */
+/* One wave per 256-value block: lane l owns values 4l..4l+3; the waves after
+ * them move cp, 1 KiB each. */
 __global__ __launch_bounds__(256) void k_quantize_q8(const float *__restrict__ x, int ncols, int nrows,
-                                                     long xstride, Q8Rows out, unsigned long long *clear, int nclear) {
+                                                     long xstride, Q8Rows out, unsigned long long *clear, int nclear,
+                                                     TableCopy cp) {
     const int lane = threadIdx.x & 63;
     if (blockIdx.x == 0 && (int)threadIdx.x < nclear) clear[threadIdx.x] = 0;
     /* readfirstlane: the block's descriptor stays in scalar registers (in
      * vector ones every load would be wrapped in a loop over its values) */
     const int wave = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * (size_t)blockDim.x + threadIdx.x) >> 6));
     const int nb = out.nb;
-    if (wave >= nrows * nb) return;   /* uniform per wave */
+    if (wave >= nrows * nb) {   /* uniform per wave */
+        const uint32_t o = (uint32_t)(wave - nrows * nb) * 1024u + 16u * (uint32_t)lane;
+        if (o < cp.n) *reinterpret_cast<u32x4 *>(cp.dst + o) = *reinterpret_cast<const u32x4 *>(cp.src + o);
+        return;
+    }
     const int r = wave / nb, b = wave % nb;
     const int n = min(256, ncols - b * 256);
     Buf xb = make_buf(x + (size_t)r * xstride + (size_t)b * 256, (uint32_t)n * 4u);
@@ -839,11 +845,11 @@ static int pick_TB(int T) { return T >= 3 ? 4 : T; }
     }
 
 void launch_quantize(const float *x, int ncols, int nrows, long xstride, const Q8Rows &out, hipStream_t st,
-                     unsigned long long *clear, int nclear) {
-    const int waves = nrows * out.nb;
+                     unsigned long long *clear, int nclear, const TableCopy &cp) {
+    const int waves = nrows * out.nb + (int)((cp.n + 1023) / 1024);
     if (waves <= 0) return;
     hipLaunchKernelGGL(k_quantize_q8, dim3((waves + 3) / 4), dim3(256), 0, st, x, ncols, nrows, xstride, out, clear,
-                       clear ? nclear : 0);
+                       clear ? nclear : 0, cp);
 }
 
 static size_t device_max_lds() {
@@ -1013,9 +1019,9 @@ int grouped_min_rows() { return g_grouped_min_rows; }
  * Qwen3 expert shape) they beat the v_dot4 phases from ~20 pairs on the
  * busiest expert (128 experts, Zipf top-8: 22 pairs 66 against 74 us, 29
  * pairs 81 against 95 us, 10-15 pairs even); the grid forms of other shapes
- * from ~40.  17 keeps every batch of up to 16 rows (a verify batch) on the
+ * from ~40.  QK_RING_MIN_ROWS keeps every batch of up to 16 rows (a verify batch) on the
  * v_dot4 phases, whose bits the persistent multi-row step shares. */
-constexpr int QK_RING_MIN_ROWS = 17, QK_GRID_MIN_ROWS = 40;
+constexpr int QK_GRID_MIN_ROWS = 40;
 static int g_qk_min_rows = -1;
 void set_qk_min_rows(int rows) { g_qk_min_rows = rows < 0 ? -1 : rows; }
 int qk_min_rows() { return g_qk_min_rows; }
@@ -1093,7 +1099,7 @@ void launch_moe(const MoeArgs &a, const int *down_fmts_present, int n_down_fmts,
     if (qk_min > 0 && a.max_rows >= qk_min && n_down_fmts == 1 && down_fmts_present[0] == TG_FMT_Q6K &&
         qk_grouped_fits(a)) {
         if (quantize_x) {
-            launch_quantize(a.xin, a.D, a.k, a.D, a.xq, st);
+            launch_quantize(a.xin, a.D, a.k, a.D, a.xq, st, nullptr, 0, a.tables);
             if (mark) (*mark)(1);
         }
         launch_moe_a_qk(a, st);
@@ -1142,7 +1148,7 @@ void launch_moe(const MoeArgs &a, const int *down_fmts_present, int n_down_fmts,
             xq.split = a.xp;
             xq.split_nblk = a.D / 32;
         }
-        launch_quantize(a.xin, a.D, a.k, a.D, xq, st);
+        launch_quantize(a.xin, a.D, a.k, a.D, xq, st, nullptr, 0, a.tables);
         if (mark) (*mark)(1);
     }
     /* 2. phase A: MXFP4 experts with many pairs take the MFMA kernel, which
