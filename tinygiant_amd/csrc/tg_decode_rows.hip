@@ -235,19 +235,31 @@ __device__ inline void a_compute(const Tab &tb, int item, const WA &w, const uin
     const int s = item / A_TILES, p0 = ufl(tb.ex[s].p0), np = ufl(tb.ex[s].np);
     const int r = a_row(item, wave, lane), sl = lane & 31;
     const FQ4K::Wd g = FQ4K::decode(w.g, sl), u = FQ4K::decode(w.u, sl);
+    /* every lane of a segment ends with the sums; lane j keeps pair j's (np
+     * <= ROWS_MAXK), so the activation and the store are issued once an item
+     * and not once a pair for one lane */
+    float kg = 0.f, ku = 0.f;
+    /* lane j also holds pair j's row, and a pair's values are read while the
+     * pair before computes: no LDS round trip in the chain */
+    const int rows = tb.prow[p0 + (lane < np ? lane : 0)];
+    auto load = [&](int j) {
+        return FQ4K::load_x(q8_lds_slot(xl, NBX, __builtin_amdgcn_readlane(rows, j < np ? j : 0)), sl);
+    };
+    FQ4K::X nx = load(0);
     for (int j = 0; j < np; j++) {
-        const int p = p0 + j;
-        const Q8Lds xr = q8_lds_slot(xl, NBX, ufl(tb.prow[p]));
-        const FQ4K::X x = FQ4K::load_x(xr, sl);
+        const FQ4K::X x = nx;
+        nx = load(j + 1);
         float ag = 0.f, au = 0.f;
         ag += FQ4K::value_d(g, x);
         au += FQ4K::value_d(u, x);
-        const float vg = seg_sum_x<32>(ag), vu = seg_sum_x<32>(au);
-        if (sl == 0) {
-            const float hv = act_fn(TG_ACT_SILU, vg, vu);
-            st_tag(hid, (uint32_t)(p * I + r), tag, hv);
-            if (dbg_hid) dbg_hid[p * I + r] = hv;
-        }
+        const float vg = seg_sum<32>(ag), vu = seg_sum<32>(au);
+        kg = sl == j ? vg : kg;
+        ku = sl == j ? vu : ku;
+    }
+    if (sl < np) {
+        const float hv = act_fn(TG_ACT_SILU, kg, ku);
+        st_tag(hid, (uint32_t)((p0 + sl) * I + r), tag, hv);
+        if (dbg_hid) dbg_hid[(p0 + sl) * I + r] = hv;
     }
 }
 
@@ -318,18 +330,25 @@ __device__ inline void b_compute(const Tab &tb, int item, const WB &w, const uin
     FQ6K::Wd wd[B_PASS];
 #pragma unroll
     for (int q = 0; q < B_PASS; q++) wd[q] = FQ6K::decode(w.w[q], sl);
+    float kv[B_PASS] = {};   /* lane j keeps pair j's sums, as in a_compute */
+    auto load = [&](int j) { return FQ6K::load_x(q8_lds_slot(hl, NBH, j < np ? j : 0), sl < B_ITEMS ? sl : 0); };
+    FQ6K::X nx = load(0);
     for (int j = 0; j < np; j++) {
-        const int p = p0 + j;
-        const Q8Lds xr = q8_lds_slot(hl, NBH, j);
-        const float pw = __int_as_float(ufl(__float_as_int(tb.pw[p])));
-        const FQ6K::X x = FQ6K::load_x(xr, sl < B_ITEMS ? sl : 0);
+        const FQ6K::X x = nx;
+        nx = load(j + 1);
 #pragma unroll
         for (int q = 0; q < B_PASS; q++) {
             float acc = 0.f;
             if (sl < B_ITEMS) acc += FQ6K::value_d(wd[q], x);
-            const float v = seg_sum_x<16>(acc);
-            if (sl == 0) st_tag(part, (uint32_t)(p * D + b_row(item, q, wave, lane)), tag, pw * (v + 0.f));
+            const float v = seg_sum<16>(acc);
+            kv[q] = sl == j ? v : kv[q];
         }
+    }
+    if (sl < np) {
+        const float pw = tb.pw[p0 + sl];
+#pragma unroll
+        for (int q = 0; q < B_PASS; q++)
+            st_tag(part, (uint32_t)((p0 + sl) * D + b_row(item, q, wave, lane)), tag, pw * (kv[q] + 0.f));
     }
 }
 
@@ -445,7 +464,7 @@ __device__ inline bool phase_c(const RowsLayer *ly, const Tab *tb, const RowsLay
     float ss = 0.f;
 #pragma unroll
     for (int c = 0; c < 4; c++) ss += o[c] * o[c];
-    ss = wave_sum_x(ss);
+    ss = seg_sum<64>(ss);
     if (lane == 0) red[wave] = ss;
     bar_lds();
     if (ts) ts[7] = wall_clock64();   /* every wave's squares are in */

@@ -538,6 +538,11 @@ __global__ __launch_bounds__(256) void k_moe_ax(MoeArgs a, int nitems, int T) {
             q.finish(a.xq, srow, nc, xl);
         }
         __syncthreads();
+        /* every lane of a segment ends with the sums; lane s keeps pair s's,
+         * so the activation is issued once for the chunk's pairs and not once
+         * a pair for one lane */
+        static_assert(S >= MOE_X_MAXP, "a lane a pair");
+        float kg[NP] = {}, ku[NP] = {};
         for (int s = 0; s < nc; s++) {
             const Q8Lds xr = q8_lds_slot(xl, a.xq.nb, s);
 #pragma unroll
@@ -554,13 +559,19 @@ __global__ __launch_bounds__(256) void k_moe_ax(MoeArgs a, int nitems, int T) {
                         au += F::value(wu[i][u], x, item);
                     }
                 }
-                float vg = seg_sum<S>(ag);
-                float vu = seg_sum<S>(au);
-                if (rv && sl == 0) {
-                    if (a.gbias) vg += gb[i];
-                    if (a.ubias) vu += ub[i];
-                    a.hidden[(size_t)(p0 + c0 + s) * a.I + r] = act_fn(a.act, vg, vu);
-                }
+                const float vg = seg_sum<S>(ag), vu = seg_sum<S>(au);
+                kg[i] = sl == s ? vg : kg[i];
+                ku[i] = sl == s ? vu : ku[i];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < NP; i++) {
+            const int r = rw + i * G;
+            if (sl < nc && r < a.I) {
+                float vg = kg[i], vu = ku[i];
+                if (a.gbias) vg += gb[i];
+                if (a.ubias) vu += ub[i];
+                a.hidden[(size_t)(p0 + c0 + sl) * a.I + r] = act_fn(a.act, vg, vu);
             }
         }
     }
@@ -618,9 +629,10 @@ __global__ __launch_bounds__(256) void k_moe_bx(MoeArgs a, int fmt, uint32_t rb,
             q.finish(a.hq, srow, nc, xl);
         }
         __syncthreads();
+        static_assert(S >= MOE_X_MAXP, "a lane a pair");
+        float kd[NP] = {};   /* lane s keeps pair s's sums, as in k_moe_ax */
         for (int s = 0; s < nc; s++) {
             const Q8Lds xr = q8_lds_slot(xl, a.hq.nb, s);
-            const int p = p0 + c0 + s;
 #pragma unroll
             for (int i = 0; i < NP; i++) {
                 const int r = rw + i * G;
@@ -632,15 +644,20 @@ __global__ __launch_bounds__(256) void k_moe_bx(MoeArgs a, int fmt, uint32_t rb,
                     if (rv && u < T && item < nitems) acc += F::value(wd[i][u], F::load_x(xr, item), item);
                 }
                 const float v = seg_sum<S>(acc);
-                if (rv && sl == 0) {
-                    const float o = a.p_w[p] * (v + (a.dbias ? db[i] : 0.f));
-                    if (CMB)
-                        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o), make_buf(a.part, 0x7FFFFFFFu).r,
-                                                              (int)(((uint32_t)p * (uint32_t)a.D + (uint32_t)r) * 4u),
-                                                              0, 16 /* sc1 */);
-                    else
-                        a.part[(size_t)p * a.D + r] = o;
-                }
+                kd[i] = sl == s ? v : kd[i];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < NP; i++) {
+            const int r = rw + i * G, p = p0 + c0 + sl;
+            if (sl < nc && r < a.D) {
+                const float o = a.p_w[p] * (kd[i] + (a.dbias ? db[i] : 0.f));
+                if (CMB)
+                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o), make_buf(a.part, 0x7FFFFFFFu).r,
+                                                          (int)(((uint32_t)p * (uint32_t)a.D + (uint32_t)r) * 4u),
+                                                          0, 16 /* sc1 */);
+                else
+                    a.part[(size_t)p * a.D + r] = o;
             }
         }
     }
