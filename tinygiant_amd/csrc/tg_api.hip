@@ -250,8 +250,6 @@ Q8Rows q8_view(uint8_t *base, int nrows, int ncols, const float *f) {
     q.sum = (int32_t *)((uint8_t *)q.s16 + (size_t)nrows * nb * 64);
     q.f = f;
     q.fstride = ncols;
-    q.split = nullptr;
-    q.split_nblk = 0;
     return q;
 }
 

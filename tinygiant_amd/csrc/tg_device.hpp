@@ -194,8 +194,6 @@ struct Q8Rows {
     const float *f;   /* the unquantized f32 rows (used by F16 weights) */
     int nb;
     int fstride;      /* floats per f32 row */
-    uint8_t *split;   /* where the rows' fp8 halves go as they are quantized (q8_split_store), or null */
-    int split_nblk;   /* 32-value blocks of a row there */
 };
 
 struct Q8Row {
@@ -311,9 +309,10 @@ __device__ inline void q8_split_store(uint32_t packed, int lane, uint8_t *dst, i
     *reinterpret_cast<u32x2 *>(dst + ((size_t)r * nblk + blk) * 64 + (up ? 32 : 0) + 8 * (lane & 3)) = o;
 }
 
-/* q8_block_quant of the wave's block, written to block b of row r */
-__device__ inline void q8_block_store(float v0, float v1, float v2, float v3, int lane, const Q8Rows &out, int r,
-                                      int b) {
+/* q8_block_quant of the wave's block, written to block b of row r; the lane's
+ * four codes */
+__device__ inline uint32_t q8_block_store(float v0, float v1, float v2, float v3, int lane, const Q8Rows &out, int r,
+                                          int b) {
     const Q8Quant q = q8_block_quant(v0, v1, v2, v3);
     const int nb = out.nb;
     int8_t *qrow = out.qs + ((size_t)r * nb + b) * 256;
@@ -325,7 +324,7 @@ __device__ inline void q8_block_store(float v0, float v1, float v2, float v3, in
         out.d[rb] = q.sc;
         out.sum[rb] = q.tot;
     }
-    if (out.split) q8_split_store(q.packed, lane, out.split, out.split_nblk, r, b);   /* uniform */
+    return q.packed;
 }
 
 __device__ inline Q8Row q8_row(const Q8Rows &a, int r) {

@@ -79,10 +79,12 @@ struct MoeArgs {
 int items_per_row(int fmt, int ncols);
 uint32_t row_bytes(int fmt, int ncols);
 
-/* q8 of nrows rows; clear[0 .. nclear) (nclear <= 64) are zeroed on the way,
- * for a consumer launched next (the fused head's argmax keys) */
+/* q8 of nrows rows, and their fp8 halves (launch_mx_split) where split is
+ * given; clear[0 .. nclear) (nclear <= 64) are zeroed on the way, for a
+ * consumer launched next (the fused head's argmax keys) */
 void launch_quantize(const float *x, int ncols, int nrows, long xstride, const Q8Rows &out, hipStream_t st,
-                     unsigned long long *clear = nullptr, int nclear = 0, const TableCopy &cp = {});
+                     unsigned long long *clear = nullptr, int nclear = 0, const TableCopy &cp = {},
+                     uint8_t *split = nullptr);
 /* up to three matrices of one width (ncols) against the same k rows:
  * y_j[i * ystride + r] = dot(W_j row r, x_i) + bias_j[r] */
 struct GemvJob {

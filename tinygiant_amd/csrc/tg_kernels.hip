@@ -31,11 +31,12 @@ namespace tg {
 
 /* ======================= q8 quantization ======================= */
 
-/* One wave per 256-value block: lane l owns values 4l..4l+3; the waves after
- * them move cp, 1 KiB each. */
+/* One wave per 256-value block: lane l owns values 4l..4l+3, and writes their
+ * fp8 halves too where `split` is given (q8_split_store, split_nblk blocks of
+ * 32 a row); the waves after them move cp, 1 KiB each. */
 __global__ __launch_bounds__(256) void k_quantize_q8(const float *__restrict__ x, int ncols, int nrows,
                                                      long xstride, Q8Rows out, unsigned long long *clear, int nclear,
-                                                     TableCopy cp) {
+                                                     TableCopy cp, uint8_t *split, int split_nblk) {
     const int lane = threadIdx.x & 63;
     if (blockIdx.x == 0 && (int)threadIdx.x < nclear) clear[threadIdx.x] = 0;
     /* readfirstlane: the block's descriptor stays in scalar registers (in
@@ -51,8 +52,9 @@ __global__ __launch_bounds__(256) void k_quantize_q8(const float *__restrict__ x
     const int n = min(256, ncols - b * 256);
     Buf xb = make_buf(x + (size_t)r * xstride + (size_t)b * 256, (uint32_t)n * 4u);
     u32x4 raw = ld16(xb, (uint32_t)lane * 16u);   /* zeros past n */
-    q8_block_store(__uint_as_float(raw.x), __uint_as_float(raw.y), __uint_as_float(raw.z), __uint_as_float(raw.w),
-                   lane, out, r, b);
+    const uint32_t codes = q8_block_store(__uint_as_float(raw.x), __uint_as_float(raw.y), __uint_as_float(raw.z),
+                                          __uint_as_float(raw.w), lane, out, r, b);
+    if (split) q8_split_store(codes, lane, split, split_nblk, r, b);   /* uniform */
 }
 
 /* RMSNorm of one row per workgroup, wave w owning the 256-value blocks
@@ -862,11 +864,11 @@ static int pick_TB(int T) { return T >= 3 ? 4 : T; }
     }
 
 void launch_quantize(const float *x, int ncols, int nrows, long xstride, const Q8Rows &out, hipStream_t st,
-                     unsigned long long *clear, int nclear, const TableCopy &cp) {
+                     unsigned long long *clear, int nclear, const TableCopy &cp, uint8_t *split) {
     const int waves = nrows * out.nb + (int)((cp.n + 1023) / 1024);
     if (waves <= 0) return;
     hipLaunchKernelGGL(k_quantize_q8, dim3((waves + 3) / 4), dim3(256), 0, st, x, ncols, nrows, xstride, out, clear,
-                       clear ? nclear : 0, cp);
+                       clear ? nclear : 0, cp, split, ncols / 32);
 }
 
 static size_t device_max_lds() {
@@ -1160,12 +1162,8 @@ void launch_moe(const MoeArgs &a, const int *down_fmts_present, int n_down_fmts,
                      (uint64_t)a.P * a.D * 4 < (1ull << 31);
     /* 1. quantize the k input rows */
     if (quantize_x && !qx_fused) {
-        Q8Rows xq = a.xq;
-        if (mx_a) {   /* the MFMA phases read the rows' fp8 halves */
-            xq.split = a.xp;
-            xq.split_nblk = a.D / 32;
-        }
-        launch_quantize(a.xin, a.D, a.k, a.D, xq, st, nullptr, 0, a.tables);
+        /* the MFMA phases read the rows' fp8 halves */
+        launch_quantize(a.xin, a.D, a.k, a.D, a.xq, st, nullptr, 0, a.tables, mx_a ? a.xp : nullptr);
         if (mark) (*mark)(1);
     }
     /* 2. phase A: MXFP4 experts with many pairs take the MFMA kernel, which
@@ -1204,12 +1202,7 @@ void launch_moe(const MoeArgs &a, const int *down_fmts_present, int n_down_fmts,
     if (mark) (*mark)(2);
     /* 3. quantize the hidden rows */
     if (!qh_fused) {
-        Q8Rows hq = a.hq;
-        if (mx_grouped && a.hp) {
-            hq.split = a.hp;
-            hq.split_nblk = a.I / 32;
-        }
-        launch_quantize(a.hidden, a.I, a.P, a.I, hq, st);
+        launch_quantize(a.hidden, a.I, a.P, a.I, a.hq, st, nullptr, 0, {}, mx_grouped ? a.hp : nullptr);
         if (mark) (*mark)(3);
     }
     /* 4. phase B, once per down format present */
