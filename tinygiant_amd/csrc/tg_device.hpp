@@ -98,11 +98,12 @@ __device__ inline int dot4(uint32_t a, uint32_t b, int c) {
  * every lane of a group holds the same (commutatively identical) sum. */
 template <int CTRL, int ROW_MASK = 0xF>
 __device__ inline int dpp_i(int old, int v) {
-    return __builtin_amdgcn_update_dpp(old, v, CTRL, ROW_MASK, 0xF, false);
+    if constexpr (ROW_MASK == 0xF) return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true);
+    else return __builtin_amdgcn_update_dpp(old, v, CTRL, ROW_MASK, 0xF, false);
 }
 template <int CTRL, int ROW_MASK = 0xF>
 __device__ inline float dpp_f(float old, float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(v), CTRL, ROW_MASK, 0xF, false));
+    return __int_as_float(dpp_i<CTRL, ROW_MASK>(__float_as_int(old), __float_as_int(v)));
 }
 
 /* sum over aligned groups of S lanes (S = 2..64); the result is exact in
@@ -432,8 +433,9 @@ struct FQ4K {
             lo = dot4(w.lo[i], a[i], lo);
             hi = dot4(w.hi[i], b[i], hi);
         }
-        int A = w.sc_lo * lo + w.sc_hi * hi;
-        int B = w.m_lo * x.s_lo + w.m_hi * x.s_hi;
+        /* 24-bit products (the sums are below 2^17): a 32-bit one issues at a quarter of the rate */
+        int A = __mul24(w.sc_lo, lo) + __mul24(w.sc_hi, hi);
+        int B = __mul24(w.m_lo, x.s_lo) + __mul24(w.m_hi, x.s_hi);
         return x.d * (w.d * (float)A - w.dmin * (float)B);
     }
     __device__ static inline float value(const W &w, const X &x, int item) { return value_d(decode(w, item), x); }
@@ -536,13 +538,13 @@ struct FQ6K {
                                    {x.x1.x, x.x1.y, x.x1.z, x.x1.w},
                                    {x.x2.x, x.x2.y, x.x2.z, x.x2.w},
                                    {x.x3.x, x.x3.y, x.x3.z, x.x3.w}};
-        int a[4] = {0, 0, 0, 0};
+        int a[4] = {-32 * x.s0, -32 * x.s1, -32 * x.s2, -32 * x.s3};   /* the codes' offset */
 #pragma unroll
         for (int c = 0; c < 4; c++)
 #pragma unroll
             for (int g = 0; g < 4; g++) a[g] = dot4(w.q[g][c], xs[g][c], a[g]);
-        const int s0 = a[0] - 32 * x.s0, s1 = a[1] - 32 * x.s1, s2 = a[2] - 32 * x.s2, s3 = a[3] - 32 * x.s3;
-        int A = w.sc[0] * s0 + w.sc[1] * s1 + w.sc[2] * s2 + w.sc[3] * s3;
+        /* 24-bit products (a sum of 16 is below 2^18): a 32-bit one issues at a quarter of the rate */
+        int A = __mul24(w.sc[0], a[0]) + __mul24(w.sc[1], a[1]) + __mul24(w.sc[2], a[2]) + __mul24(w.sc[3], a[3]);
         return w.d * x.d * (float)A;
     }
     __device__ static inline float value(const W &w, const X &x, int item) { return value_d(decode(w, item), x); }
