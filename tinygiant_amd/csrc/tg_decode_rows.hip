@@ -706,9 +706,10 @@ int decode_rows_threads() { return NT; }
  * items are split evenly over them, so a workgroup works on one expert per
  * phase: a down item that starts another expert would first wait a memory
  * round trip for that expert's hidden rows.  A workgroup's time in a phase is
- * about its items x an item's cost, fitted on per-workgroup phase times of
- * 48-layer steps: an A item 0.91 us + 0.34 us a pair of its expert, a B item
- * 0.90 us + 0.38 us a pair after the expert's hidden rows are in.  The split
+ * about its items x an item's cost: with a pair of the expert at 0.27 of an A
+ * item without pairs and 0.30 of a B item, fitted to whole passes (9 rows: 0.37
+ * and 0.42 1679 us, 0.32 and 0.36 1654, these 1628, 0.22 and 0.25 1625; 16
+ * rows: 2399, 2377, 2355, 2369).  The split
  * takes the smallest such time every expert can meet within the workgroups
  * (items a workgroup = floor(T / cost), at least one), then hands the
  * workgroups left over, one at a time, to the expert whose workgroups take
@@ -720,6 +721,7 @@ int decode_rows_threads() { return NT; }
  * slower (1,342-1,357 and 1,908-1,916).  The down items
  * skip workgroups 0 .. c - 1, which combine the rows: they start a row's
  * combine as soon as its last partial lands. */
+constexpr double A_PAIR = 0.27, B_PAIR = 0.30;
 static void split_phase(const int *np, int n_act, int tiles, int w0, double c1, int *s) {
     const int G = ROWS_GRID - w0;
     std::vector<int> wgs(n_act, 1);
@@ -777,8 +779,8 @@ static void split_phase(const int *np, int n_act, int tiles, int w0, double c1, 
 }
 
 void decode_rows_split(const int *np, int n_act, int c, int *split) {
-    split_phase(np, n_act, A_TILES, 0, 0.34 / 0.91, split);
-    split_phase(np, n_act, B_TILES, c, 0.38 / 0.90, split + ROWS_GRID + 1);
+    split_phase(np, n_act, A_TILES, 0, A_PAIR, split);
+    split_phase(np, n_act, B_TILES, c, B_PAIR, split + ROWS_GRID + 1);
 }
 
 }  // namespace tg
