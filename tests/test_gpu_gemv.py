@@ -59,3 +59,39 @@ def test_matmul_dev_forms(tg, orc, fmt, nrows, ncols, k, bias):
     for j in range(k):
         ref = orc.matmul(fmt, w, b, x[j], nrows, ncols)
         assert np.abs(got[j] - ref).max() <= 1e-5 * np.abs(ref).max(), j
+
+
+@pytest.mark.parametrize("fmt,size", [(Q4K, 144), (Q6K, 210)])
+@pytest.mark.parametrize("byte", [0x00, 0x7F, 0x80, 0xFF])
+def test_scale_products_at_their_largest(tg, orc, fmt, size, byte):
+    """Blocks whose codes and scales are all one byte against rows of one
+    sign (every q8 code 127) and of alternating signs: the integer sums and
+    their products with the scales at the ends of their ranges (below 2^18
+    and 2^26).  They are exact, so only the f32 terms' order differs: two
+    blocks a row, 1e-6."""
+    lib = tg.lib()
+    nrows, ncols = 3, 512
+    w = np.full((nrows * ncols // 256, size), byte, np.uint8)
+    half = np.array([0.0371], np.float16).view(np.uint8)
+    if fmt == Q4K:
+        w[:, 0:2] = half
+        w[:, 2:4] = half
+    else:
+        w[:, 208:210] = half
+    w = w.reshape(-1)
+    x = np.full((2, ncols), 1.7, np.float32)
+    x[1, ::2] = -1.7
+    print("scale products", fmt, byte, flush=True)
+    bufs = [tg.DeviceArray(n) for n in (w.nbytes, x.nbytes, 2 * nrows * 4, lib.tg_hip_matmul_scratch_bytes(2, ncols))]
+    bufs[0].upload(w)
+    bufs[1].upload(x)
+    lib.tg_hip_clear_error()
+    lib.tg_hip_matmul_dev(fmt, bufs[0].ptr, None, bufs[1].ptr, bufs[2].ptr, nrows, ncols, 2, bufs[3].ptr, None)
+    lib.tg_hip_synchronize()
+    assert tg.last_error() == ""
+    got = bufs[2].download(np.float32, 2 * nrows).reshape(2, nrows)
+    for b in bufs:
+        b.free()
+    for j in range(2):
+        ref = orc.matmul(fmt, w, None, x[j], nrows, ncols)
+        assert np.abs(got[j] - ref).max() <= 1e-6 * max(np.abs(ref).max(), 1e-3), (j, got[j], ref)
