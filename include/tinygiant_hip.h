@@ -174,7 +174,9 @@ int tg_hip_moe_plan_pairs(const tg_hip_moe_plan *plan);
 void tg_hip_moe_plan_destroy(tg_hip_moe_plan *plan);
 
 /* k-row device GEMV: y[j][r] = dot(mat row r, q8(x_j)) + bias[r];
- * scratch_dev holds tg_hip_matmul_scratch_bytes(k, ncols) bytes. */
+ * scratch_dev holds tg_hip_matmul_scratch_bytes(k, ncols) bytes.  outputs_dev
+ * may overlap inputs_dev (a quantized format's rows are in q8 before any
+ * output is written), except for F16, which reads the f32 rows themselves. */
 void tg_hip_matmul_dev(int fmt, const void *mat_dev, const float *bias_dev, const float *inputs_dev,
                        float *outputs_dev, int nrows, int ncols, int k, void *scratch_dev, void *stream);
 size_t tg_hip_matmul_scratch_bytes(int k, int ncols);

@@ -95,3 +95,43 @@ def test_scale_products_at_their_largest(tg, orc, fmt, size, byte):
     for j in range(2):
         ref = orc.matmul(fmt, w, None, x[j], nrows, ncols)
         assert np.abs(got[j] - ref).max() <= 1e-6 * max(np.abs(ref).max(), 1e-3), (j, got[j], ref)
+
+
+@pytest.mark.parametrize("fmt,nrows,ncols,k,shift", [
+    (Q4K, 2048, 2048, 1, 0), (Q6K, 8192, 8192, 1, 0), (Q80, 2880, 2880, 1, 0), (MXFP4, 4096, 512, 8, 0),
+    (Q4K, 768, 2048, 1, 1500), (Q4K, 768, 2048, 1, -700), (Q80, 100, 288, 3, 860), (Q6K, 512, 512, 9, 0)])
+@pytest.mark.parametrize("alloc", [True, False])
+def test_matmul_dev_over_its_inputs(tg, fmt, nrows, ncols, k, shift, alloc):
+    """Outputs that lie over the inputs (in place, and shifted by `shift`
+    values either way) are the bits of a call with buffers apart: one row and
+    few blocks, whose launch would quantize the rows while others write, and
+    more, which are in q8 before."""
+    print(f"matmul over its inputs: fmt {fmt} {nrows} x {ncols}, {k} rows, shift {shift}", flush=True)
+    lib = tg.lib()
+    rng = np.random.default_rng(fmt + nrows + ncols + k)
+    x = rng.standard_normal((k, ncols)).astype(np.float32)
+    nx, ny, pad = k * ncols, k * nrows, max(0, -shift)
+    wd = tg.DeviceArray(nrows * lib.tg_row_bytes(fmt, ncols))
+    wd.upload(_matrix(tg, rng, fmt, nrows, ncols))
+    room = tg.DeviceArray(4 * (pad + max(nx, max(shift, 0) + ny)))
+    apart = tg.DeviceArray(4 * ny)
+    sc = tg.DeviceArray(lib.tg_hip_matmul_scratch_bytes(k, ncols))
+
+    def call(y):
+        room.upload(np.concatenate([np.zeros(pad, np.float32), x.reshape(-1)]))
+        if alloc:
+            lib.tg_hip_matmul_dev(fmt, wd.ptr, None, room.ptr + 4 * pad, y, nrows, ncols, k, sc.ptr, None)
+        else:
+            lib.tg_hip_matmul_dev_noalloc(fmt, wd.ptr, None, room.ptr + 4 * pad, y, nrows, ncols, k, None)
+        lib.tg_hip_synchronize()
+        assert tg.last_error() == ""
+
+    lib.tg_hip_clear_error()
+    lib.tg_hip_init()
+    call(apart.ptr)
+    call(room.ptr + 4 * (pad + shift))
+    ref = apart.download(np.float32, ny)
+    got = room.download(np.float32, room.nbytes // 4)[pad + shift:][:ny]
+    for d in (wd, room, apart, sc):
+        d.free()
+    assert got.tobytes() == ref.tobytes()

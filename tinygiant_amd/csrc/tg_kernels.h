@@ -107,7 +107,8 @@ void launch_gemv(int fmt, const uint8_t *W, int nrows, int ncols, const float *b
                  float *y, long ystride, hipStream_t st);
 void launch_gemv_multi(int fmt, const GemvJobs &jobs, int njobs, int ncols, const Q8Rows &x, int k, hipStream_t st);
 /* one matrix against k f32 rows of ncols values; x is the room for their q8,
- * used where the matrix's launch does not quantize the rows itself */
+ * used where the matrix's launch does not quantize the rows itself.  y may
+ * overlap xf, except for F16, whose launch reads the f32 rows. */
 void launch_matmul(int fmt, const uint8_t *W, int nrows, int ncols, const float *bias, const float *xf,
                    const Q8Rows &x, int k, float *y, long ystride, hipStream_t st);
 /* q8 of one f32 row and up to three matrices of one format family (Q4_K and

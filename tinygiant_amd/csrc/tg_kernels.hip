@@ -1005,9 +1005,18 @@ void launch_gemv(int fmt, const uint8_t *W, int nrows, int ncols, const float *b
     launch_gemv_multi(fmt, jobs, 1, ncols, x, k, st);
 }
 
+/* the rows' q8 in a launch of its own where the outputs lie over the inputs: a
+ * workgroup that quantizes them would read what others have written */
+static bool matmul_over_inputs(const float *xf, int ncols, const float *y, long ystride, int nrows, int k) {
+    const uintptr_t x0 = (uintptr_t)xf, x1 = x0 + (size_t)k * ncols * 4;
+    const uintptr_t y0 = (uintptr_t)y, y1 = y0 + ((size_t)(k - 1) * ystride + nrows) * 4;
+    return x0 < y1 && y0 < x1;
+}
+
 void launch_matmul(int fmt, const uint8_t *W, int nrows, int ncols, const float *bias, const float *xf,
                    const Q8Rows &x, int k, float *y, long ystride, hipStream_t st) {
-    if (gemv_staged_ok(&fmt, 1, ncols) && (k == 1 || k * ((ncols + 255) / 256) <= GEMV_QX_BLOCKS)) {
+    if (gemv_staged_ok(&fmt, 1, ncols) && (k == 1 || k * ((ncols + 255) / 256) <= GEMV_QX_BLOCKS) &&
+        (fmt == TG_FMT_F16 || !matmul_over_inputs(xf, ncols, y, ystride, nrows, k))) {
         const GemvJobs jobs = {{{W, bias, y, ystride, nrows}}};
         launch_gemv_staged(&fmt, jobs, 1, ncols, xf, x, k, nullptr, 0, st);
         return;
