@@ -147,3 +147,33 @@ def test_qk_ring_pair_counts(tg, orc, counts, bias):
     with _qk_rows(tg, 1):
         _check_moe(tg, orc, len(counts), k, 2048, 768, O.FMT_Q4K, [O.FMT_Q6K] * len(counts),
                    O.ACT_GPTOSS if bias else O.ACT_SILU, bias, rw, x)
+
+
+def test_qk_ring_null_biases(tg, orc):
+    """Experts without gate and up biases beside experts with them, on the
+    persistent rings' shape: null entries count as no bias, as in the oracle
+    and the grid form.  Bars: _check_moe's."""
+    say("qk ring null biases")
+    counts, D, I = (33, 20, 17, 5), 2048, 768
+    n, k = len(counts), max(counts)
+    rng = np.random.default_rng(7)
+    rw = np.zeros((n, k), np.float32)
+    for e, c in enumerate(counts):
+        rw[e, rng.choice(k, c, replace=False)] = rng.uniform(0.1, 1.0, c)
+    x = rng.standard_normal((k, D)).astype(np.float32)
+    b = [rng.uniform(-0.5, 0.5, I).astype(np.float32) for _ in range(n)]
+    gb, ub = [None, b[0], None, b[1]], [None, b[2], None, b[3]]
+    g, u, d = _experts(n, D, I, O.FMT_Q4K, [O.FMT_Q6K] * n, 98)
+    P = sum(counts)
+    h_ref, h_gpu = np.zeros((P, I), np.float32), np.zeros((P, I), np.float32)
+    args = (g, u, d, O.FMT_Q4K, [O.FMT_Q6K] * n, gb, ub, None, O.ACT_GPTOSS, rw, x)
+    orc.moe_v2(*args, np.zeros((k, D), np.float32), I, hidden_out=h_ref)
+    with _qk_rows(tg, 1):
+        got = tg.moe_forward_rows_v2(*args, np.zeros((k, D), np.float32), I, hidden_out=h_gpu)
+    assert tg.last_error() == ""
+    for p in range(P):
+        ok, rel = close(h_gpu[p], h_ref[p], tol=1e-4)
+        assert ok, ("hidden", p, rel)
+    ref = orc.moe_v2(*args, np.zeros((k, D), np.float32), I, hidden_in=h_gpu)
+    ok, rel = close(got, ref)
+    assert ok, rel

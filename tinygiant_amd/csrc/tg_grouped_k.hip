@@ -587,8 +587,10 @@ __global__ __launch_bounds__(RG_NT) void k_moe_qa_ring(MoeArgs a) {
         const int re = run_end(i);
         const int *rc = a.rg_runs + (size_t)RING_REC * run;
         const int pf = ldc(rc, 0), nv = ldc(rc, 1), e = ldc(rc, 2 + RING_P);
-        const Buf gb = make_buf(a.gbias ? (const void *)(uintptr_t)ldc(a.gbias, e) : nullptr, a.gbias ? (uint32_t)a.I * 4u : 0u);
-        const Buf ub = make_buf(a.ubias ? (const void *)(uintptr_t)ldc(a.ubias, e) : nullptr, a.ubias ? (uint32_t)a.I * 4u : 0u);
+        /* a null entry: an empty buffer, which reads zero */
+        const uint64_t qg = a.gbias ? ldc(a.gbias, e) : 0, qu = a.ubias ? ldc(a.ubias, e) : 0;
+        const Buf gb = make_buf((const void *)(uintptr_t)qg, qg ? (uint32_t)a.I * 4u : 0u);
+        const Buf ub = make_buf((const void *)(uintptr_t)qu, qu ? (uint32_t)a.I * 4u : 0u);
         auto step = [&](auto tiles) __attribute__((always_inline)) {
             for (; i < re; i++, slab++) {
                 bar_lds();   /* item i's slab has landed, item i - 1's sums are in LDS */
