@@ -522,8 +522,9 @@ __global__ __launch_bounds__(256) void k_moe_ax(MoeArgs a, int nitems, int T) {
             wg[i][u] = F::load_w(gw, iv ? (uint32_t)r * rb : ROW_OOB, iv ? item : 0);
             wu[i][u] = F::load_w(uw, iv ? (uint32_t)r * rb : ROW_OOB, iv ? item : 0);
         }
-        gb[i] = rv && a.gbias ? ((const float *)a.gbias[e])[r] : 0.f;
-        ub[i] = rv && a.ubias ? ((const float *)a.ubias[e])[r] : 0.f;
+        /* null entries: no bias */
+        gb[i] = rv && a.gbias && a.gbias[e] ? ((const float *)a.gbias[e])[r] : 0.f;
+        ub[i] = rv && a.ubias && a.ubias[e] ? ((const float *)a.ubias[e])[r] : 0.f;
     }
     for (int c0 = 0; c0 < np; c0 += MOE_X_MAXP) {
         const int nc = min(MOE_X_MAXP, np - c0);
@@ -614,7 +615,7 @@ __global__ __launch_bounds__(256) void k_moe_bx(MoeArgs a, int fmt, uint32_t rb,
             const bool iv = rv && u < T && item < nitems;
             wd[i][u] = F::load_w(dw, iv ? (uint32_t)r * rb : ROW_OOB, iv ? item : 0);
         }
-        db[i] = rv && a.dbias ? ((const float *)a.dbias[e])[r] : 0.f;
+        db[i] = rv && a.dbias && a.dbias[e] ? ((const float *)a.dbias[e])[r] : 0.f;
     }
     for (int c0 = 0; c0 < np; c0 += MOE_X_MAXP) {
         const int nc = min(MOE_X_MAXP, np - c0);
