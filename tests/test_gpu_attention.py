@@ -83,9 +83,10 @@ def _dev(tg, a):
     return d
 
 
-def _gpu(tg, c, window):
+def _gpu(tg, c, window, att_at=None):
     """tg_hip_attention_dev on device copies; returns output, attention output
-    and the device caches read back."""
+    and the device caches read back.  att_at: att_out at this byte of one
+    buffer with the output at 4096."""
     lib = tg.lib()
     keep = []
 
@@ -100,18 +101,21 @@ def _gpu(tg, c, window):
     kk, vv = _dev(tg, c["kv_k"]), _dev(tg, c["kv_v"])
     keep += [kk, vv]
     rc, rs, x = dev(c["rc"]), dev(c["rs"]), dev(c["x"])
-    out = tg.DeviceArray(c["D"] * 4)
-    att = tg.DeviceArray(c["nh"] * c["hd"] * 4)
+    nq = c["nh"] * c["hd"]
+    out = tg.DeviceArray(c["D"] * 4 if att_at is None else 8192 + 4 * (c["D"] + nq))
+    att = tg.DeviceArray(nq * 4)
+    out_at = 0 if att_at is None else 4096
+    att_buf = att if att_at is None else out
     sb = lib.tg_hip_attention_scratch_bytes(c["D"], c["nh"], c["nkv"], c["hd"], c["kv_max"])
     scr = tg.DeviceArray(sb)
     keep += [out, att, scr]
     lib.tg_hip_clear_error()
     lib.tg_hip_attention_dev(*c["fmts"], *w, *b, qn, kn, sk, kk.ptr, vv.ptr, c["kv_len"], c["kv_max"], window, rc, rs,
-                             x, out.ptr, c["D"], c["nh"], c["nkv"], c["hd"], c["kv_len"], ctypes.c_float(1e-6),
-                             att.ptr, scr.ptr, None)
+                             x, out.ptr + out_at, c["D"], c["nh"], c["nkv"], c["hd"], c["kv_len"],
+                             ctypes.c_float(1e-6), att_buf.ptr + (att_at or 0), scr.ptr, None)
     lib.tg_hip_synchronize()
     assert tg.last_error() == "", tg.last_error()
-    r = (out.download(np.float32, c["D"]), att.download(np.float32, c["nh"] * c["hd"]),
+    r = (out.download(np.float32, c["D"], out_at), att_buf.download(np.float32, nq, att_at or 0),
          kk.download(np.float32, c["kv_k"].size).reshape(c["kv_k"].shape),
          vv.download(np.float32, c["kv_v"].size).reshape(c["kv_v"].shape))
     for a in keep:
@@ -299,3 +303,19 @@ def test_attention_combine_edges(tg, orc, hd, nkv, ratio, kv_len):
     c = _case(700 + kv_len + hd, 256, nkv * ratio, nkv, hd, (Q80, Q80, Q80, Q80), kv_len + 3, kv_len, norms=True,
               sinks=hd != 128)
     _check(orc, c, 0, _gpu(tg, c, 0), _oracle(orc, c, 0))
+
+
+@pytest.mark.parametrize("fmt_o", [Q80, F16])
+@pytest.mark.parametrize("hd", [64, 32])
+@pytest.mark.parametrize("att_at", [4096, 4096 + 512, 4096 - 512, 4096 - 1024])
+def test_attention_att_out_over_output(tg, orc, fmt_o, hd, att_at):
+    """att_out over the output: what overlaps is the attention output, the
+    rest of the output the projection (256 values each; the last offset only
+    touches).  The bits are those of buffers apart."""
+    say("attention att_out over output", fmt_o, hd, att_at)
+    c = _case(900 + hd, 256, 256 // hd, 2, hd, (Q80, Q80, Q80, fmt_o), 40, 33)
+    apart, over = _gpu(tg, c, 0), _gpu(tg, c, 0, att_at)
+    assert over[1].tobytes() == apart[1].tobytes()
+    free = np.ones(256, bool)
+    free[max(0, (att_at - 4096) // 4):max(0, (att_at - 4096) // 4 + 256)] = False
+    assert over[0][free].tobytes() == apart[0][free].tobytes()

@@ -1303,8 +1303,11 @@ static void attn_run(int fmt_q, int fmt_k, int fmt_v, int fmt_o, const void *wq,
         }
     }
     /* the attention output goes straight to the caller's buffer where the
-     * combine's 16-byte stores can */
-    float *att = att_out && ((uintptr_t)att_out & 15) == 0 ? att_out : (float *)(scratch + L.att);
+     * combine's 16-byte stores can and the output projection does not write
+     * over it (att_out is what remains where the two overlap) */
+    const bool apart = att_out && ((uintptr_t)att_out + (size_t)q_dim * 4 <= (uintptr_t)output ||
+                                   (uintptr_t)output + (size_t)embed_dim * 4 <= (uintptr_t)att_out);
+    float *att = apart && ((uintptr_t)att_out & 15) == 0 ? att_out : (float *)(scratch + L.att);
     Q8Rows aq = q8_view(scratch + L.aq, 1, q_dim, att);
     /* attention; q8 of its output fused into the combine where the block
      * layout allows, and the combine into the partial kernel for short spans
