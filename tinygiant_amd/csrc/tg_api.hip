@@ -262,7 +262,9 @@ struct HostPlan {
     bool has_gb = false, has_ub = false, has_db = false;
     std::vector<int> fmts_present;
     int max_rows = 0;      /* most pairs of any one expert */
-    bool rings = true;     /* lay out the persistent phases' lists */
+    /* whether launch_moe may take the int8 and the MXFP4 persistent phases, by
+     * the thresholds in force (a plan outlives a change of them) */
+    bool qk_rings = true, mx_rings = true;
 };
 
 /* ---- MXFP4 scale byte 255 ----
@@ -420,9 +422,18 @@ static int moe_ctr_words(int D) { return D / 4 + 16; }
 
 static int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
-/* every active expert's down matrix is MXFP4, in the persistent phase's shape */
-static bool mx_down_ring(const HostPlan &h) {
-    return h.rings && h.fmts_present.size() == 1 && h.fmts_present[0] == TG_FMT_MXFP4 && mx_ring_shape(h.D, h.I, MX_RING_DOWN);
+/* The persistent phases whose lists a call's tables hold: those that
+ * launch_moe can take for its formats, shape and pair counts. */
+struct RingUse {
+    bool qa, qb, mx_up, mx_down;
+};
+static RingUse ring_use(const HostPlan &h) {
+    auto down = [&](int fmt) { return h.fmts_present.size() == 1 && h.fmts_present[0] == fmt; };
+    const bool qk = h.qk_rings && h.gate_fmt == TG_FMT_Q4K && down(TG_FMT_Q6K) && h.max_rows <= RING_MAX_ROWS;
+    const bool mx = h.mx_rings && h.max_rows <= MX_RING_MAX_ROWS;
+    return {qk && qa_ring_shape(h.gate_fmt, h.D, h.I), qk && !h.has_db && qb_ring_shape(h.I, h.D),
+            mx && h.gate_fmt == TG_FMT_MXFP4 && mx_ring_shape(h.I, h.D, MX_RING_UP),
+            mx && down(TG_FMT_MXFP4) && mx_ring_shape(h.D, h.I, MX_RING_DOWN)};
 }
 
 Layout plan_layout(const HostPlan &h) {
@@ -436,18 +447,16 @@ Layout plan_layout(const HostPlan &h) {
     t += (size_t)(n + 1) * 4 + (size_t)P * 4 * 4 + (size_t)(k + 1) * 4 + 8;   /* p_off, p_row, p_exp, p_w, r_off, r_pair */
     t += (size_t)4 * (n + 1) * 4 + 16;      /* active expert lists and their cost prefixes */
     t += (size_t)n * sizeof(ExpDesc) + 16;  /* active expert descriptors */
-    if (h.rings && qa_ring_shape(h.gate_fmt, h.D, h.I))  /* the persistent gate/up phase's items and ranges */
-        t += 2 * (size_t)(h.I / 16) * (P / 16 + n + 1) * 4 + (size_t)RING_REC * (P / 16 + n + 1) * 4 +
-             2 * (QA_RING_MAX_G + 1) * 4 + 64;
-    if (h.rings && h.gate_fmt == TG_FMT_MXFP4 && mx_ring_shape(h.I, h.D, MX_RING_UP))
-        t += 2 * (size_t)ceil_div(h.I, MX_RING_UP) * (P / MX_RING_P + n + 1) * 4 +
-             (size_t)RING_REC * (P / MX_RING_P + n + 1) * 4 + 2 * (QA_RING_MAX_G + 1) * 4 + 64;
-    if (mx_down_ring(h))
-        t += 2 * (size_t)ceil_div(h.D, MX_RING_DOWN) * (P / MX_RING_P + n + 1) * 4 +
-             (size_t)RING_REC * (P / MX_RING_P + n + 1) * 4 + 2 * (QA_RING_MAX_G + 1) * 4 + 64;
-    else if (h.rings && qb_ring_shape(h.I, h.D))  /* the persistent down phase's */
-        t += 2 * (size_t)(h.D / 32) * (P / 16 + n + 1) * 4 + (size_t)RING_REC * (P / 16 + n + 1) * 4 +
-             2 * (QA_RING_MAX_G + 1) * 4 + 64;
+    /* the persistent phases' items, run ends, run records and ranges */
+    auto lists = [&](int slabs, int pass_pairs) {
+        const size_t runs = P / pass_pairs + n + 1;
+        t += (2 * (size_t)slabs + RING_REC) * runs * 4 + 2 * (QA_RING_MAX_G + 1) * 4 + 64;
+    };
+    const RingUse use = ring_use(h);
+    if (use.qa) lists(h.I / 16, RING_P);
+    if (use.qb) lists(h.D / 32, RING_P);
+    if (use.mx_up) lists(ceil_div(h.I, MX_RING_UP), MX_RING_P);
+    if (use.mx_down) lists(ceil_div(h.D, MX_RING_DOWN), MX_RING_P);
     L.tables_len = t + 64;
     b.take(L.tables_len);
     L.xin = b.take((size_t)k * h.D * 4);
@@ -572,20 +581,18 @@ MoeArgs plan_args(const HostPlan &h, const Layout &L, uint8_t *dev, uint8_t *img
         off = (const int *)put(r.off.data(), r.off.size() * 4);
         n_wg = (int)r.off.size() - 1;
     };
-    const bool mx_up = h.rings && h.gate_fmt == TG_FMT_MXFP4 && mx_ring_shape(h.I, h.D, MX_RING_UP), mx_down = mx_down_ring(h);
-    a.rg_mx = mx_up && a.max_rows <= MX_RING_MAX_ROWS;
-    a.rb_mx = mx_down && a.max_rows <= MX_RING_MAX_ROWS;
-    if (h.rings && a.n_act_a > 0) {
-        if (a.rg_mx)
+    const RingUse use = ring_use(h);
+    a.rg_mx = use.mx_up;
+    a.rb_mx = use.mx_down;
+    if (a.n_act_a > 0) {
+        if (use.mx_up)
             ring(ceil_div(h.I, MX_RING_UP), MX_RING_P, MX_COST, a.rg_items, a.rg_rend, a.rg_runs, a.rg_run0, a.rg_off,
                  a.rg_n);
-        else if (qa_ring_shape(h.gate_fmt, h.D, h.I) && a.max_rows <= RING_MAX_ROWS)
-            ring(h.I / 16, RING_P, QA_RING_COST, a.rg_items, a.rg_rend, a.rg_runs, a.rg_run0, a.rg_off, a.rg_n);
-        if (a.rb_mx)
+        if (use.qa) ring(h.I / 16, RING_P, QA_RING_COST, a.rg_items, a.rg_rend, a.rg_runs, a.rg_run0, a.rg_off, a.rg_n);
+        if (use.mx_down)
             ring(ceil_div(h.D, MX_RING_DOWN), MX_RING_P, MX_COST, a.rb_items, a.rb_rend, a.rb_runs, a.rb_run0,
                  a.rb_off, a.rb_n);
-        else if (!mx_down && qb_ring_shape(h.I, h.D) && a.max_rows <= RING_MAX_ROWS)
-            ring(h.D / 32, RING_P, QB_RING_COST, a.rb_items, a.rb_rend, a.rb_runs, a.rb_run0, a.rb_off, a.rb_n);
+        if (use.qb) ring(h.D / 32, RING_P, QB_RING_COST, a.rb_items, a.rb_rend, a.rb_runs, a.rb_run0, a.rb_off, a.rb_n);
     }
     act_a.insert(act_a.end(), act_b.begin(), act_b.end());
     a.mx_act = (const int *)put(act_a.data(), act_a.size() * 4);
@@ -633,10 +640,19 @@ void moe_host(const uint8_t *const *gate_ptrs, const uint8_t *const *up_ptrs, co
     build_pairs(h, row_weights);
     if (h.P == 0) return;   /* every weight is zero: output unchanged */
 
-    /* the lists only where launch_moe can take the persistent phases (for one
+    h.has_gb = gate_bias != nullptr;
+    h.has_ub = up_bias != nullptr;
+    h.has_db = down_bias != nullptr;
+    if (h.has_gb != h.has_ub) {
+        set_err("moe: gate and up biases must both be given or both be NULL");
+        return;
+    }
+    /* the lists only where launch_moe takes the persistent phases (for one
      * row of 8 experts they would be ten times the other tables) */
-    const int qk = qk_min_rows() >= 0 ? qk_min_rows() : QK_RING_MIN_ROWS, mx = grouped_min_rows();
-    h.rings = (qk > 0 && h.max_rows >= qk) || (mx > 0 && h.max_rows >= mx);
+    const RingUse shape = ring_use(h);
+    const int qk = qk_threshold(shape.qa && shape.qb), mx = grouped_min_rows();
+    h.qk_rings = qk > 0 && h.max_rows >= qk;
+    h.mx_rings = mx > 0 && h.max_rows >= mx;
     Layout L = plan_layout(h);
     Bump bump;
     bump.off = L.total;
@@ -650,13 +666,6 @@ void moe_host(const uint8_t *const *gate_ptrs, const uint8_t *const *up_ptrs, co
     h.gbias.assign(n, 0);
     h.ubias.assign(n, 0);
     h.dbias.assign(n, 0);
-    h.has_gb = gate_bias != nullptr;
-    h.has_ub = up_bias != nullptr;
-    h.has_db = down_bias != nullptr;
-    if (h.has_gb != h.has_ub) {
-        set_err("moe: gate and up biases must both be given or both be NULL");
-        return;
-    }
     std::vector<char> staged_flags;
     struct Fix {
         std::vector<uint64_t> *vec;

@@ -184,8 +184,8 @@ constexpr int QA_RING_MAX_G = 1024;
 void launch_moe_a_qk(const MoeArgs &a, hipStream_t st);
 void launch_moe_b_qk(const MoeArgs &a, hipStream_t st);
 void set_qk_min_rows(int rows);
-constexpr int QK_RING_MIN_ROWS = 17;
 int qk_min_rows();
+int qk_threshold(bool rings);   /* the pair count in force, where both persistent rings run or not */
 /* Q4_K / Q6_K experts: one workgroup column per active expert, each weight
  * row read once for all its pairs (EM_ON), or one per pair (0).  For layers
  * with at most two pairs per expert: EM_FUSE_Q8, the phases quantize their
