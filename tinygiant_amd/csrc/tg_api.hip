@@ -474,9 +474,9 @@ Layout plan_layout(const HostPlan &h) {
     return L;
 }
 
-/* serialises the tables into img (host, tables_len bytes) and returns the
- * MoeArgs for a device base address */
-MoeArgs plan_args(const HostPlan &h, const Layout &L, uint8_t *dev, uint8_t *img) {
+/* serialises the tables into img (host, tables_len bytes, of which `used` are
+ * written) and returns the MoeArgs for a device base address */
+MoeArgs plan_args(const HostPlan &h, const Layout &L, uint8_t *dev, uint8_t *img, size_t *used = nullptr) {
     const int n = h.n, k = h.k, P = std::max(h.P, 1);
     size_t o = 0;
     auto put = [&](const void *src, size_t bytes) {
@@ -597,6 +597,7 @@ MoeArgs plan_args(const HostPlan &h, const Layout &L, uint8_t *dev, uint8_t *img
     act_a.insert(act_a.end(), act_b.begin(), act_b.end());
     a.mx_act = (const int *)put(act_a.data(), act_a.size() * 4);
     a.mx_cum = (const int *)put(cum.data(), cum.size() * 4);
+    if (used) *used = o;
     return a;
 }
 
@@ -703,7 +704,8 @@ void moe_host(const uint8_t *const *gate_ptrs, const uint8_t *const *up_ptrs, co
     const size_t io_len = (size_t)k * D * 4, tab_len = (L.tables_len + 15) & ~(size_t)15;
     uint8_t *io = io_rows(2 * io_len + tab_len);
     uint8_t *img = io + 2 * io_len;   /* io_len is a multiple of 128 */
-    MoeArgs a = plan_args(h, L, dev, img);
+    size_t tab_used = 0;
+    MoeArgs a = plan_args(h, L, dev, img, &tab_used);
     memcpy(io, inputs, io_len);
     memcpy(io + io_len, output, io_len);
     a.xin = (const float *)io;
@@ -714,7 +716,7 @@ void moe_host(const uint8_t *const *gate_ptrs, const uint8_t *const *up_ptrs, co
      * of their own that every fused combine leaves zeroed */
     a.ctr = host_call_tickets(moe_ctr_words(D));
     a.ctr_n = a.ctr ? moe_ctr_words(D) : 0;
-    a.tables = {img, dev + L.tables, (uint32_t)tab_len};
+    a.tables = {img, dev + L.tables, (uint32_t)((tab_used + 15) & ~(size_t)15)};
     for (auto &it : sg.items) HIPCHECK(hipMemcpyAsync(dev + it.off, it.host, it.n, hipMemcpyHostToDevice, g.st));
     if (grouped_min_rows() > 0 && a.max_rows >= grouped_min_rows()) {
         /* the MFMA phases are a candidate: no e8m0 byte of 255 may reach
