@@ -293,9 +293,9 @@ __device__ inline uint32_t q8_block_wave(float v0, float v1, float v2, float v3,
     int q0 = (int)__builtin_rintf(v0 * inv), q1 = (int)__builtin_rintf(v1 * inv);
     int q2 = (int)__builtin_rintf(v2 * inv), q3 = (int)__builtin_rintf(v3 * inv);
     int s = q0 + q1 + q2 + q3;
-    s += dpp_i<0xB1>(s, s);
-    s += dpp_i<0x4E>(s, s);                  /* 16-element sum in every lane of the quad */
-    const int t32 = s + dpp_i<0x141>(s, s);  /* 32-element sum (half-row mirror pairs quads) */
+    s += dpp_i<0xB1>(s);
+    s += dpp_i<0x4E>(s);                  /* 16-element sum in every lane of the quad */
+    const int t32 = s + dpp_i<0x141>(s);  /* 32-element sum (half-row mirror pairs quads) */
     if (s16 && (lane & 3) == 0) s16[lane >> 2] = s;
     if (s32 && (lane & 7) == 0) s32[lane >> 3] = t32;
     if (lane == 0) *d = amax / 127.f;

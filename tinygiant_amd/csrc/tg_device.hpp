@@ -93,17 +93,33 @@ __device__ inline int dot4(uint32_t a, uint32_t b, int c) {
 
 /* ---- DPP cross-lane reductions ----
  * GFX9 DPP controls: quad_perm [1,0,3,2] = 0xB1, [2,3,0,1] = 0x4E,
- * row_half_mirror = 0x141, row_mirror = 0x140, row_bcast:15 = 0x142,
- * row_bcast:31 = 0x143.  Each step adds a lane's value to one partner's, so
- * every lane of a group holds the same (commutatively identical) sum. */
-template <int CTRL, int ROW_MASK = 0xF>
-__device__ inline int dpp_i(int old, int v) {
-    if constexpr (ROW_MASK == 0xF) return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true);
-    else return __builtin_amdgcn_update_dpp(old, v, CTRL, ROW_MASK, 0xF, false);
+ * row_half_mirror = 0x141, row_mirror = 0x140, row_ror:n = 0x120 + n,
+ * row_bcast:15 = 0x142, row_bcast:31 = 0x143.  Each step adds a lane's value
+ * to one partner's, so every lane of a group holds the same (commutatively
+ * identical) sum.
+ *
+ * dpp_i / dpp_f: the controls under which every lane has a source in its own
+ * 16-lane row (a permutation), for whole active waves.  They can fuse into
+ * the addition behind them, which a form that keeps an old value cannot. */
+template <int CTRL>
+__device__ inline int dpp_i(int v) {
+    static_assert((CTRL >= 0 && CTRL <= 0xFF) || (CTRL >= 0x121 && CTRL <= 0x12F) || CTRL == 0x140 || CTRL == 0x141,
+                  "quad_perm, row_ror, row_mirror, row_half_mirror");
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true);
 }
-template <int CTRL, int ROW_MASK = 0xF>
-__device__ inline float dpp_f(float old, float v) {
-    return __int_as_float(dpp_i<CTRL, ROW_MASK>(__float_as_int(old), __float_as_int(v)));
+template <int CTRL>
+__device__ inline float dpp_f(float v) {
+    return __int_as_float(dpp_i<CTRL>(__float_as_int(v)));
+}
+/* the row broadcasts: rows outside ROW_MASK, and lanes without a source, get old */
+template <int CTRL, int ROW_MASK>
+__device__ inline int dpp_bcast_i(int old, int v) {
+    static_assert(CTRL == 0x142 || CTRL == 0x143, "row_bcast:15, row_bcast:31");
+    return __builtin_amdgcn_update_dpp(old, v, CTRL, ROW_MASK, 0xF, false);
+}
+template <int CTRL, int ROW_MASK>
+__device__ inline float dpp_bcast_f(float old, float v) {
+    return __int_as_float(dpp_bcast_i<CTRL, ROW_MASK>(__float_as_int(old), __float_as_int(v)));
 }
 
 /* sum over aligned groups of S lanes (S = 2..64); the result is exact in
@@ -111,22 +127,22 @@ __device__ inline float dpp_f(float old, float v) {
 template <int S>
 __device__ inline float seg_sum_last(float v) {
     static_assert(S >= 2 && S <= 64 && (S & (S - 1)) == 0, "segment");
-    v += dpp_f<0xB1>(v, v);
-    if (S >= 4) v += dpp_f<0x4E>(v, v);
-    if (S >= 8) v += dpp_f<0x141>(v, v);
-    if (S >= 16) v += dpp_f<0x140>(v, v);
-    if (S >= 32) v += dpp_f<0x142, 0xA>(0.f, v);
-    if (S >= 64) v += dpp_f<0x143, 0xC>(0.f, v);
+    v += dpp_f<0xB1>(v);
+    if (S >= 4) v += dpp_f<0x4E>(v);
+    if (S >= 8) v += dpp_f<0x141>(v);
+    if (S >= 16) v += dpp_f<0x140>(v);
+    if (S >= 32) v += dpp_bcast_f<0x142, 0xA>(0.f, v);
+    if (S >= 64) v += dpp_bcast_f<0x143, 0xC>(0.f, v);
     return v;
 }
 template <int S>
 __device__ inline int seg_isum_last(int v) {
-    v += dpp_i<0xB1>(v, v);
-    if (S >= 4) v += dpp_i<0x4E>(v, v);
-    if (S >= 8) v += dpp_i<0x141>(v, v);
-    if (S >= 16) v += dpp_i<0x140>(v, v);
-    if (S >= 32) v += dpp_i<0x142, 0xA>(0, v);
-    if (S >= 64) v += dpp_i<0x143, 0xC>(0, v);
+    v += dpp_i<0xB1>(v);
+    if (S >= 4) v += dpp_i<0x4E>(v);
+    if (S >= 8) v += dpp_i<0x141>(v);
+    if (S >= 16) v += dpp_i<0x140>(v);
+    if (S >= 32) v += dpp_bcast_i<0x142, 0xA>(0, v);
+    if (S >= 64) v += dpp_bcast_i<0x143, 0xC>(0, v);
     return v;
 }
 /* wave-wide sum / max, broadcast to every lane (fixed combination order) */
@@ -139,10 +155,10 @@ __device__ inline float wave_sum(float v) {
     return (a + b) + (c + d);
 }
 __device__ inline float wave_max(float v) {
-    v = fmaxf(v, dpp_f<0xB1>(v, v));
-    v = fmaxf(v, dpp_f<0x4E>(v, v));
-    v = fmaxf(v, dpp_f<0x141>(v, v));
-    v = fmaxf(v, dpp_f<0x140>(v, v));
+    v = fmaxf(v, dpp_f<0xB1>(v));
+    v = fmaxf(v, dpp_f<0x4E>(v));
+    v = fmaxf(v, dpp_f<0x141>(v));
+    v = fmaxf(v, dpp_f<0x140>(v));
     const float a = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 15));
     const float b = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 31));
     const float c = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 47));
@@ -168,13 +184,13 @@ __device__ inline float seg_sum(float v) {
     if (S >= 64) v += __shfl_xor(v, 32, 64);
     if (S >= 32) v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x401F));
     if (S >= 16) {
-        v += dpp_f<0x128>(v, v);   /* row_ror:8 */
-        v += dpp_f<0x124>(v, v);   /* row_ror:4 */
+        v += dpp_f<0x128>(v);   /* row_ror:8 */
+        v += dpp_f<0x124>(v);   /* row_ror:4 */
     } else if (S == 8) {
         v += __shfl_xor(v, 4, 64);
     }
-    if (S >= 4) v += dpp_f<0x4E>(v, v);    /* quad_perm [2,3,0,1] */
-    if (S >= 2) v += dpp_f<0xB1>(v, v);    /* quad_perm [1,0,3,2] */
+    if (S >= 4) v += dpp_f<0x4E>(v);    /* quad_perm [2,3,0,1] */
+    if (S >= 2) v += dpp_f<0xB1>(v);    /* quad_perm [1,0,3,2] */
     return v;
 }
 __device__ inline float seg_sum_rt(float v, int S) {
@@ -268,10 +284,10 @@ __device__ inline Q8Quant q8_block_quant_dpp(float v0, float v1, float v2, float
     r.packed = (uint32_t)(q0 & 0xFF) | ((uint32_t)(q1 & 0xFF) << 8) | ((uint32_t)(q2 & 0xFF) << 16) |
                ((uint32_t)(q3 & 0xFF) << 24);
     int s = q0 + q1 + q2 + q3;
-    s += dpp_i<0xB1>(s, s);
-    s += dpp_i<0x4E>(s, s);               /* 16-element sum */
+    s += dpp_i<0xB1>(s);
+    s += dpp_i<0x4E>(s);               /* 16-element sum */
     r.s16 = s;
-    r.s32 = s + dpp_i<0x141>(s, s);       /* 32-element sum */
+    r.s32 = s + dpp_i<0x141>(s);       /* 32-element sum */
     r.tot = 0;
     return r;
 }

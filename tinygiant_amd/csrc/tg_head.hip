@@ -159,10 +159,10 @@ __device__ inline void rs_step(float *v, bool hi) {
         for (int i = 0; i < M / 2; i++) {
             const float send = hi ? v[i] : v[i + M / 2];
             const float keep = hi ? v[i + M / 2] : v[i];
-            v[i] = keep + dpp_f<CTRL>(0.f, send);
+            v[i] = keep + dpp_f<CTRL>(send);
         }
     } else {
-        v[0] += dpp_f<CTRL>(0.f, v[0]);
+        v[0] += dpp_f<CTRL>(v[0]);
     }
 }
 /* Sums N slots (N a power of two <= 16) over the 16 lanes of each row of a
