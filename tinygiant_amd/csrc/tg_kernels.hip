@@ -772,7 +772,7 @@ __global__ __launch_bounds__(256) void k_copy(const u32x4 *__restrict__ src, u32
 
 /* ======================= launchers ======================= */
 
-static int pick_S(int nitems, int *T) {
+static constexpr int pick_S(int nitems, int *T) {
     /* fewest lane slots S*T (S power of two <= 64); ties go to larger S */
     int bestS = 64, bestT = (nitems + 63) / 64, best = bestS * bestT;
     for (int S = 32; S >= 8; S >>= 1) {
@@ -830,30 +830,52 @@ uint32_t row_bytes(int fmt, int ncols) {
         default: TG_DISPATCH_TB(TB_, 64, CALL) break;  \
     }
 static int pick_TB(int T) { return T >= 3 ? 4 : T; }
-/* the same for k_gemv_staged, which also has a form of three items */
-#define TG_DISPATCH_T4(TB_, S_, CALL)   \
-    switch (TB_) {                      \
-        case 1: CALL(S_, 1); break;     \
-        case 2: CALL(S_, 2); break;     \
-        case 3: CALL(S_, 3); break;     \
-        default: CALL(S_, 4); break;    \
+/* The forms (S, TB) of k_gemv_staged: a row's items on S lanes, at most max_t a
+ * lane, TB the next of 1, 2, 3, 4, 8 and 16. */
+struct GemvForm {
+    int S, T, TB;
+};
+static constexpr GemvForm gemv_form(int nitems, int max_t) {
+    int T = 0, S = pick_S(nitems, &T);
+    while (T > max_t) {
+        S *= 2;
+        T = (nitems + S - 1) / S;
     }
-#define TG_DISPATCH_S4(S_, TB_, CALL)                  \
-    switch (S_) {                                      \
-        case 8: TG_DISPATCH_T4(TB_, 8, CALL) break;    \
-        case 16: TG_DISPATCH_T4(TB_, 16, CALL) break;  \
-        case 32: TG_DISPATCH_T4(TB_, 32, CALL) break;  \
-        default: TG_DISPATCH_T4(TB_, 64, CALL) break;  \
+    return {S, T, T <= 4 ? T : T <= 8 ? 8 : 16};
+}
+constexpr int GEMV_MAX_T = 4, GEMV_MAX_T_F16 = 16;
+/* the forms that some row length takes (any number of items; whole units of 32
+ * values, four items, for F16), and no other */
+#define GEMV_FORMS(X)                     \
+    X(8, 1) X(8, 3)                       \
+    X(16, 1) X(16, 3) X(16, 4)            \
+    X(32, 1) X(32, 3) X(32, 4)            \
+    X(64, 1) X(64, 2) X(64, 3) X(64, 4)
+#define GEMV_FORMS_F16(X)                 \
+    X(8, 1) X(8, 3) X(8, 8) X(8, 16)      \
+    X(16, 1) X(16, 3) X(16, 8) X(16, 16)  \
+    X(32, 1) X(32, 3) X(32, 8) X(32, 16)  \
+    X(64, 1) X(64, 2) X(64, 3) X(64, 4) X(64, 8) X(64, 16)
+template <int N>
+static constexpr bool gemv_forms_are(const int (&forms)[N][2], int step, int max_t) {
+    bool taken[N] = {};
+    for (int n = step; n <= 64 * max_t; n += step) {
+        const GemvForm f = gemv_form(n, max_t);
+        int at = 0;
+        while (at < N && (forms[at][0] != f.S || forms[at][1] != f.TB)) at++;
+        if (at == N) return false;
+        taken[at] = true;
     }
-
-/* k_gemv_staged's F16 forms of 8 and 16 items a lane */
-#define TG_DISPATCH_S16(S_, TB_)          \
-    switch (S_) {                         \
-        case 8: CALL16(8, TB_); break;    \
-        case 16: CALL16(16, TB_); break;  \
-        case 32: CALL16(32, TB_); break;  \
-        default: CALL16(64, TB_); break;  \
-    }
+    for (int i = 0; i < N; i++)
+        if (!taken[i]) return false;
+    return true;
+}
+#define FORM(S_, TB_) {S_, TB_},
+static constexpr int gemv_forms[][2] = {GEMV_FORMS(FORM)}, gemv_forms_f16[][2] = {GEMV_FORMS_F16(FORM)};
+#undef FORM
+static_assert(gemv_forms_are(gemv_forms, 1, GEMV_MAX_T), "Q8_0 and MXFP4 rows");
+static_assert(gemv_forms_are(gemv_forms, 4, GEMV_MAX_T), "Q4_K and Q6_K rows, four items a block");
+static_assert(gemv_forms_are(gemv_forms_f16, 4, GEMV_MAX_T_F16), "F16 rows");
 
 #define TG_DISPATCH_F(fmt, BODY)                    \
     switch (fmt) {                                  \
@@ -915,7 +937,7 @@ static void launch_gemv_general(int fmt, const GemvJobs &jobs, int njobs, int nc
 /* formats that cut a row into as many items: one launch takes any of them */
 static int gemv_family(int fmt) { return fmt == TG_FMT_Q4K || fmt == TG_FMT_Q6K ? 0 : fmt == TG_FMT_F16 ? 2 : 1; }
 /* items a lane holds of a row, at most */
-static int gemv_max_t(int fmt) { return fmt == TG_FMT_F16 ? 16 : 4; }
+static int gemv_max_t(int fmt) { return fmt == TG_FMT_F16 ? GEMV_MAX_T_F16 : GEMV_MAX_T; }
 static uint32_t gemv_stride(int fmt, int ncols) {
     return fmt == TG_FMT_F16 ? (uint32_t)ncols * 4u : q8_lds_stride((ncols + 255) / 256);
 }
@@ -931,16 +953,14 @@ bool gemv_staged_ok(const int *fmts, int njobs, int ncols) {
 static void launch_gemv_staged(const int *fmts, const GemvJobs &jobs, int njobs, int ncols, const float *xf,
                                const Q8Rows &xq, int k, unsigned *zero, int n_zero, hipStream_t st) {
     const int nitems = items_per_row(fmts[0], ncols);
-    int T, S = pick_S(nitems, &T);
-    while (T > gemv_max_t(fmts[0])) {
-        S *= 2;
-        T = (nitems + S - 1) / S;
-    }
+    const GemvForm form = gemv_form(nitems, gemv_max_t(fmts[0]));
+    const int S = form.S, T = form.T, TB = form.TB;
     const int G = 64 / S;
     const uint32_t stride = gemv_stride(fmts[0], ncols);
     const int kc = std::min(k, std::max(1, (int)(GEMV_LDS / stride)));
     /* a workgroup's row groups: one a wave while the grid stays within
-     * GEMV_WGS workgroups, more above, so the staging is paid once */
+     * GEMV_ALL workgroups; above, GEMV_WGS workgroups walk several, so the
+     * staging is paid once */
     int wgs[3] = {0, 0, 0}, total = 0;
     for (int i = 0; i < njobs; i++) total += wgs[i] = (jobs.j[i].nrows + 4 * G - 1) / (4 * G);
     const int iters = total <= GEMV_ALL ? 1 : (total + GEMV_WGS - 1) / GEMV_WGS;
@@ -966,25 +986,27 @@ static void launch_gemv_staged(const int *fmts, const GemvJobs &jobs, int njobs,
             hipLaunchKernelGGL((k_gemv_staged<A, B, S_, TB_, GEMV_Q8>), dim3(wg), dim3(256), lds, st, jobs, m, xf,    \
                                xq, ncols, k, kc, nitems, T, zero, n_zero);                                            \
     } while (0)
+#define FORM(S_, TB_) if (S == S_ && TB == TB_) CALL(S_, TB_); else
     if (gemv_family(fmts[0]) == 0) {
         typedef FQ4K A;
         typedef FQ6K B;
-        TG_DISPATCH_S4(S, T, CALL)
+        GEMV_FORMS(FORM) {}
     } else if (gemv_family(fmts[0]) == 1) {
         typedef FQ80 A;
         typedef FMXFP4 B;
-        TG_DISPATCH_S4(S, T, CALL)
+        GEMV_FORMS(FORM) {}
     } else {
         typedef FF16 A;
         typedef FF16 B;
 #define CALL16(S_, TB_)                                                                                               \
     hipLaunchKernelGGL((k_gemv_staged<A, B, S_, TB_, GEMV_QX>), dim3(wg), dim3(256), lds, st, jobs, m, xf, xq, ncols, k, \
                        kc, nitems, T, zero, n_zero)
-        if (T > 8) TG_DISPATCH_S16(S, 16)
-        else if (T > 4) TG_DISPATCH_S16(S, 8)
-        else TG_DISPATCH_S4(S, T, CALL16)
+#undef FORM
+#define FORM(S_, TB_) if (S == S_ && TB == TB_) CALL16(S_, TB_); else
+        GEMV_FORMS_F16(FORM) {}
 #undef CALL16
     }
+#undef FORM
 #undef CALL
 }
 
