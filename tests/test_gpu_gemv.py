@@ -1,5 +1,5 @@
-"""tg_hip_matmul_dev over its dispatch: every format at row lengths that give a
-lane one to four items (16 for F16), partial q8 blocks and rows past what the
+"""tg_hip_matmul_dev over its dispatch: every format at row lengths of each form
+in which the launch cuts a row, partial q8 blocks and rows past what the
 staged kernel holds, row counts around a wave's groups and past one grid, and
 input row counts that quantize in the kernel, in a launch of their own, and in
 several staged chunks.  Bar: max|d| <= 1e-5 max|ref| against the oracle, whose
@@ -30,6 +30,26 @@ def _matrix(tg, rng, fmt, nrows, ncols):
     (F16, 3, 32, 1, True), (F16, 70, 1056, 5, False), (F16, 33, 2880, 4, True), (F16, 21, 8192, 3, True),
     (F16, 9, 8224, 2, False), (F16, 1025, 512, 1, True)])
 def test_matmul_dev_forms(tg, orc, fmt, nrows, ncols, k, bias):
+    _check_matmul(tg, orc, fmt, nrows, ncols, k, bias)
+
+
+# a row's items on 8, 16, 32 and 64 lanes, 1 to 4 a lane (up to 16 for F16), as the launch cuts it: a row length of
+# each form, the longest or one with lanes left over
+K_COLS = [512, 1280, 1536, 768, 2304, 2560, 3328, 3584, 1792, 4352, 7168, 3840, 7936, 8448, 12544]
+BLOCK32_COLS = [96, 544, 288, 1056, 1568, 800, 2080, 3104, 1824, 3872, 4128, 6176]
+F16_COLS = [32, 160, 288, 544, 96, 352, 608, 1056, 224, 736, 1248, 2080, 480, 992, 1504, 2016, 2528, 4128]
+
+
+@pytest.mark.parametrize("fmt,ncols", [(f, c) for f in (Q4K, Q6K) for c in K_COLS] +
+                         [(f, c) for f in (Q80, MXFP4) for c in BLOCK32_COLS] + [(F16, c) for c in F16_COLS])
+def test_matmul_dev_every_row_form(tg, orc, fmt, ncols):
+    """Each form with one row (quantized by the launch), two (quantized by it
+    up to eight blocks a row) and nineteen (in q8 before it)."""
+    for k in (1, 2, 19):
+        _check_matmul(tg, orc, fmt, 37, ncols, k, k == 2)
+
+
+def _check_matmul(tg, orc, fmt, nrows, ncols, k, bias):
     print(f"matmul fmt {fmt} {nrows} x {ncols}, {k} rows, bias {bias}", flush=True)
     lib = tg.lib()
     rng = np.random.default_rng(fmt * 1000 + nrows + ncols + k)
