@@ -139,7 +139,7 @@ void tg_hip_memcpy_d2d(void *dst_dev, const void *src_dev, size_t n, void *strea
 void tg_hip_synchronize(void);
 /* No counterpart in the reference (its CPU library holds no device state).
  * Waits for the device, then releases the library's stream, arena, pinned
- * rows, upload buffers and timing marks; a later call re-initialises.  Plans,
+ * buffer, upload buffers and timing marks; a later call re-initialises.  Plans,
  * decode steps and device arrays are the caller's to destroy first. */
 void tg_hip_shutdown(void);
 

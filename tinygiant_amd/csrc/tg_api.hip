@@ -88,11 +88,12 @@ struct Ctx {
     bool ready = false;
     int dev = 0;
     hipStream_t st = nullptr;
-    /* grow-only device arena for per-call scratch, pinned host staging */
+    /* grow-only device arena for per-call scratch */
     uint8_t *arena = nullptr;
     size_t arena_cap = 0;
-    /* coherent (uncached on the device) pinned rows that kernels read and
-     * write in place: the input and output rows of the host-pointer MoE call */
+    /* coherent (uncached on the device) pinned memory of the host-pointer MoE
+     * call: the input and output rows, which kernels read and write in place,
+     * and the call's tables until its q8 launch moves them */
     uint8_t *io = nullptr;
     size_t io_cap = 0;
     /* row-tile tickets of the host call's fused MoE combine (zero between calls) */
@@ -1179,7 +1180,7 @@ static void release_upload_buffers();
 static void release_marks();
 
 /* Waits for the device and releases everything the library holds: its
- * stream, the device arena, the pinned and coherent host rows, the ticket
+ * stream, the device arena, the host call's coherent buffer, the ticket
  * words, the file-upload buffers and the timing marks.  Objects the caller
  * created (plans, decode steps, device arrays) stay theirs to destroy first.
  * A later call re-initialises the library. */
@@ -1321,8 +1322,8 @@ static void attn_run(int fmt_q, int fmt_k, int fmt_v, int fmt_o, const void *wq,
     float *att = apart && ((uintptr_t)att_out & 15) == 0 ? att_out : (float *)(scratch + L.att);
     Q8Rows aq = q8_view(scratch + L.aq, 1, q_dim, att);
     /* attention; q8 of its output fused into the combine where the block
-     * layout allows, and the combine into the partial kernel for short spans
-     * (its counters are cleared by the fused projection launch) */
+     * layout allows, and the combine into the span or partial kernel where it
+     * writes few records (its counters are cleared by the fused projection launch) */
     const bool fuse_q8 = fmt_o != TG_FMT_F16 && attention_combine_q8_ok(n_heads, head_dim);
     launch_attention_core(qkv, q_norm_w, k_norm_w, sinks, kv_k, kv_v, kv_len, kv_max, window, rope_cos_row,
                           rope_sin_row, n_heads, n_kv, head_dim, eps, (float *)(scratch + L.part), att,

@@ -11,12 +11,13 @@
 #define ATTN_MAX_HEAD_DIM 128  /* head_dim: even, multiple of 4, at most this */
 #define ATTN_MAX_GQA 8         /* query heads per KV head, at most this */
 #define ATTN_MAX_CHUNKS 2048   /* kv_max <= ATTN_CHUNK * ATTN_MAX_CHUNKS */
-#define ATTN_FUSE_MAX_CHUNKS 32  /* chunks up to which the partial kernel also combines */
+#define ATTN_FUSE_MAX_CHUNKS 32  /* spans or chunks up to which the span or partial kernel also combines */
 
 namespace tg {
 
-/* The combine folded into the span or partial kernel: the last workgroup of each KV head, by a ticket from ctr[kh], merges the chunks of
- * its query heads, writes att and q8 of it into row 0 of aq. */
+/* The combine folded into the span or partial kernel: the last workgroup of
+ * each KV head, by a ticket from ctr[kh], merges the spans or chunks of its
+ * query heads, writes att and q8 of it into row 0 of aq. */
 struct AttnFuse {
     unsigned *ctr;        /* n_kv counters, zero when the kernel starts */
     const float *sinks;

@@ -38,6 +38,10 @@
  * read from the q8 rows in global memory; 256 threads add the waves' partial
  * sums in wave order and write one result each.  HBM sees each weight byte
  * once however many pairs the expert holds.
+ *
+ * All this is the form of k_moe_qa and k_moe_qb.  k_moe_qa_ring (scales in the
+ * codes, MFMAs of K = 64) and k_moe_qb_ring (the codes, not the pairs, zeroed
+ * in one half of K) form the same integer sums, in persistent workgroups.
  */
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -355,12 +359,11 @@ __global__ __launch_bounds__(RG_NT) void k_moe_qa_ring(MoeArgs a) {
 
     /* item j of the list (j < n): expert index, slab, pass */
     auto item = [&](int j) { return ldc(a.rg_items, (size_t)(i0 + j)); };
-    /* What the copy and finishing waves need of an item comes through the
-     * scalar path in stages, each from loads issued an item earlier (an item
-     * code, then its expert's entries, then the biases): a chain of dependent
-     * scalar loads in one item's step would stall the wave for each round
-     * trip, and the barrier with it. */
-    struct Info {   /* a copy wave's: its matrix (gate for wave RG_CW, up for the next) and slab */
+    /* What a copy wave needs of an item comes through the scalar path in
+     * stages, each from loads issued an item earlier (an item code, then its
+     * expert's entry): a chain of dependent scalar loads in one item's step
+     * would stall the wave for each round trip, and the barrier with it. */
+    struct Info {   /* its matrix (gate for wave RG_CW, up for the next) and slab */
         uint64_t base;
         int s;
     };
@@ -860,13 +863,12 @@ __global__ __launch_bounds__(DR_NT) void k_moe_qb_ring(MoeArgs a) {
     const int hbw = w % DR_HB, bi = hbw >> 1, h = hbw & 1, tw = w / DR_HB;   /* a compute wave's half-block, tile */
 
     auto item = [&](int j) { return ldc(a.rb_items, (size_t)(i0 + j)); };
-    /* What the copy and finishing waves need of an item comes through the
-     * scalar path in stages, each from loads issued an item earlier: an item
-     * code, then its expert's table entries, then the pair weights.  A chain
-     * of dependent scalar loads in one item's step would stall the wave for
-     * each load's round trip (about a microsecond under the weight stream)
-     * and the barrier with it. */
-    struct Info {   /* a copy wave's: the matrix and slab */
+    /* What a copy wave needs of an item comes through the scalar path in
+     * stages, each from loads issued an item earlier: an item code, then its
+     * expert's table entry.  A chain of dependent scalar loads in one item's
+     * step would stall the wave for each load's round trip (about a
+     * microsecond under the weight stream) and the barrier with it. */
+    struct Info {   /* the matrix and slab */
         uint64_t base;
         int s;
     };
@@ -1076,16 +1078,17 @@ bool qk_grouped_fits(const MoeArgs &a) {
 
 bool qa_ring_shape(int gate_fmt, int D, int I) { return gate_fmt == TG_FMT_Q4K && D == 256 * RG_NB && I % 16 == 0 && I <= 4096; }
 
-/* Items in the order expert (busiest first), pass, slab, cut into G
- * contiguous stretches of equal length: each workgroup's stretch is a few
- * runs of one (expert, pass), and the passes of an expert run at about the
- * same time on neighbouring workgroups, so their slabs' second reads come
- * from the caches.  rend[i] is the end of item i's run (the items of its
- * expert and pass): a workgroup finds where its run ends with one load, not
- * by scanning the items that follow.  runs holds each run's record (first
- * pair, pair count, the input rows of its first 16 pairs) in list order and
- * run0[w] the run of workgroup w's first item, so a compute wave reaches a
- * run's operands with one round trip of scalar loads. */
+/* Items in the order expert (busiest first), pass, slab, cut into at most G
+ * contiguous stretches of about equal cost (RingCost; workgroups past the
+ * last stretch get none): each workgroup's stretch is a few runs of one
+ * (expert, pass), and the passes of an expert run at about the same time on
+ * neighbouring workgroups, so their slabs' second reads come from the caches.
+ * rend[i] is the end of item i's run (the items of its expert and pass): a
+ * workgroup finds where its run ends with one load, not by scanning the items
+ * that follow.  runs holds each run's record (first pair, the pairs from
+ * there on, the input rows of its first RING_P pairs, the expert) in list
+ * order and run0[w] the run of workgroup w's first item, so a compute wave
+ * reaches a run's operands with one round trip of scalar loads. */
 void ring_items(const ExpDesc *ed, int n_act, int slabs, int G, const int *p_row, int P, int pass_pairs,
                 const RingCost &c, RingLists &r) {
     r.items.clear();
