@@ -156,7 +156,9 @@ def test_grouped_run_to_run_identical(tg):
     (2880, 160, 16, 3),    # the longest row of the persistent phases; the down phase's last group partly past its row
     (160, 2880, 33, 2),    # three passes
     (2912, 2944, 5, 2),    # one block past the longest row: k_moe_mx in both phases
-    (64, 4128, 6, 2),      # more item rows than an item's code holds in the gate/up phase, not in the down phase
+    (64, 4128, 6, 2),      # down rows whose slab k_moe_mx has no room for: the v_dot4 phases
+    (2912, 160, 20, 2),    # gate/up rows of 91 blocks in k_moe_mx, down rows of 5 in the persistent phase
+    (160, 2912, 20, 2),    # gate/up in the persistent phase, down rows of 91 blocks in k_moe_mx
     (1184, 1344, 40, 5),   # 37 and 42 blocks: partial groups in a wave's range
 ])
 def test_grouped_ring_edges(tg, orc, D, I, k, n):
