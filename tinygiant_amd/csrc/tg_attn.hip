@@ -7,8 +7,8 @@
  *   k_attn_span     head_dim 64 and 128, split over the sequence: one
  *                   workgroup per (KV head, span of positions) runs the GQA
  *                   query heads that share the K and V rows over them on f32
- *                   MFMA, so each cache byte is read once; per query head it
- *                   writes the span's max score, sum of exponentials and
+ *                   MFMA, so a row is read for all of them together; per query
+ *                   head it writes the span's max score, sum of exponentials and
  *                   unnormalised V sum.  It also does the heads' preparation:
  *                   the optional QK RMS norm (tg_rms_norm, :680-698) and RoPE
  *                   at pos (apply_rope_inplace, :702-719) of its query heads,
@@ -365,14 +365,18 @@ __global__ __launch_bounds__(256) void k_attn_partial(const float *__restrict__ 
  * positions.
  *
  * Measured (whole calls, k_attn_partial before): 30,001 positions, 8 KV
- * heads of 64, 91.3 -> 56.1 us; 4 KV heads of 128: 31,000 positions 70.6 ->
- * 44.8, 4,000 28.5 -> 25.8, 500 23.6 -> 21.4 us.  k_attn_partial read both
+ * heads of 64, 91.3 -> 47.3 us (56.1 before its combine was folded in); 4 KV
+ * heads of 128: 31,000 positions 70.6 -> 44.8, 4,000 28.5 -> 23.6 (25.8
+ * before the combine kernel's one batch of loads), 500 23.6 -> 21.4 us.  k_attn_partial read both
  * factors of every product from LDS and wrote a record per 32 positions
  * (16 MB at 30,001).
  *
  * Bound: the bytes of the cache.  A 16-position tile of a 64-value head is
  * 8 KB for 32 MFMAs of 32 cycles, 32 bytes a cycle and CU, four times the
- * CU's share of HBM, even with half of the 16 columns empty. */
+ * CU's share of HBM, even with half of the 16 columns empty.  A wave asks for
+ * one tile more than it uses, rows of the next span up to kv_len: where a wave
+ * has one tile, as up to about 4,000 positions of 4 KV heads, HBM sees the
+ * cache twice (4,096 positions: 33.6 MB read for 16.8). */
 typedef float v4f __attribute__((ext_vector_type(4)));
 
 template <int HD, bool FUSE>
